@@ -301,9 +301,11 @@ MW3_API int32_t mw3_cheby_spectrum(const double *autoc, int32_t kmax, double emi
                    0: kernel by kernel.  Same kernels, same order of every
                    sum: results are bitwise identical.
    MW3_OPT_RADIAL  1 (default): the radial kinetic correction by the
-                   low-mode kernels (R passes with the sine table in LDS, one
-                   wave per 16-row work item; the two r passes in one kernel)
-                   where the grid allows them; 0: as batched GEMMs.
+                   low-mode kernels where the grid allows them (MW3_FP64: the
+                   r products inside the update, the R products and mode
+                   weights in one kernel between two updates; MW3_MIXED: R
+                   passes with the sine table in LDS around one kernel for
+                   the two r passes); 0: as batched GEMMs.
    MW3_OPT_ANGULAR 0 (default): the angular term by the parity-folded
                    one-pass kernel (with Coriolis-coupled channels, in
                    MW3_MIXED with FP16 products: its forward and back parts
@@ -316,12 +318,8 @@ MW3_API int32_t mw3_cheby_spectrum(const double *autoc, int32_t kmax, double emi
                    (default in MW3_FP64).
    MW3_OPT_ANGULAR_GRID 1 (default) or 2: the folded angular kernel runs
                    its blocks per channel divided by this value.
-   MW3_OPT_RADIAL_GRID  1 (default), 2 or 4: the staged persistent R-pass
-                   kernels run the resident block count divided by this
-                   value (each block loads its waves' sine-table slices
-                   once).  The R passes with the sine table in LDS (FP32,
-                   and FP64 on devices of 16 or more compute units) run a
-                   grid of their own and ignore it; mw3_get_option then
+   MW3_OPT_RADIAL_GRID  accepts 1 (default), 2 or 4 and has no effect: the
+                   radial kernels run grids of their own.  mw3_get_option
                    reports 1.
    MW3_OPT_FP16_PRODUCTS  MW3_MIXED only.  1 (default): the inverse R pass
                    and the folded angular kernel multiply on the FP16 matrix

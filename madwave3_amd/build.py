@@ -13,7 +13,8 @@ CSRC = os.path.join(HERE, "csrc")
 OUT = os.path.join(HERE, "libmw3.so")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 
-SOURCES = ["mw3_setup.cpp", "mw3_kernels.hip", "mw3_api.hip"]
+SOURCES = ["mw3_setup.cpp", "mw3_kernels.hip", "mw3_step_f32.hip", "mw3_step_f64.hip",
+           "mw3_api.hip"]
 FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC",
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",

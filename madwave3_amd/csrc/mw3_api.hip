@@ -59,7 +59,6 @@ void timer_end(Ctx* c, int id, hipStream_t s) {
 static void timer_collect(Ctx* c) {
   if (c->pending.empty()) return;
   (void)hipStreamSynchronize(c->stream);
-  if (c->aux) (void)hipStreamSynchronize(c->aux);
   if (c->side) (void)hipStreamSynchronize(c->side);
   for (auto& p : c->pending) {
     float ms = 0;
@@ -128,9 +127,11 @@ static void free_all(Ctx* c) {
                   c->d_ring_cvj, c->d_zcr, c->d_zcdr, c->d_zs2, c->d_etot, c->d_fdv, c->d_dcvj,
                   c->d_cvj_skip, c->d_norm_part, c->d_ring_norm, c->d_efe, c->d_zfe, c->d_phi,
                   c->d_wmat, c->d_zero_skip, c->d_ch_elec, c->d_ch_omega, c->d_ch_cpl, c->d_potiflux,
-                  c->d_flux_elec, c->d_scratch, c->d_fmap, c->d_ir1flux, c->d_slice,
-                  c->d_psi32, c->d_psim132, c->d_scr32, c->d_uw_row, c->d_uw_word,
-                  c->d_uw_item, c->d_uw_gfirst, c->d_uw_part, c->d_tprod, c->d_ppart,
+                  c->d_flux_elec, c->d_scratch, c->d_fmap, c->d_ir1flux, c->d_ring_slice,
+                  c->d_psi32, c->d_psim132, c->d_scr32, c->d_up_wave, c->d_up_seg,
+                  c->d_up_tile, c->d_up_sfirst, c->d_up_part,
+                  c->d_up_row, c->d_up_tab, c->d_rr_f, c->d_rr_b, c->d_rr_w, c->d_g1,
+                  c->d_g2, c->d_tprod,
                   c->d_dtrans, c->d_ring_prod, c->d_prodwf, c->d_prod_part,
                   c->d_ring_cvjp, c->d_cvjp_last, c->d_zs2prod, c->d_rad_items, c->d_fold_D, c->d_fold_a, c->d_fold_b,
                   c->d_lowT, c->d_mid_items, c->d_mid_sizes, c->d_mid_items2, c->d_mid_wts,
@@ -146,23 +147,16 @@ static void free_all(Ctx* c) {
     (void)hipEventDestroy(t.b);
   }
   c->pool.clear();
-  if (c->aux) {
-    (void)hipStreamSynchronize(c->aux);
-    (void)hipStreamDestroy(c->aux);
-  }
-  if (c->side) {
-    (void)hipStreamSynchronize(c->side);
-    (void)hipStreamDestroy(c->side);
-  }
   for (auto& g : c->graph)
     if (g) {
       (void)hipGraphExecDestroy(g);
       g = nullptr;
     }
   if (c->d_slot) (void)hipFree(c->d_slot);
-  if (c->ev_fork) (void)hipEventDestroy(c->ev_fork);
-  if (c->ev_slice) (void)hipEventDestroy(c->ev_slice);
-  if (c->ev_cvj) (void)hipEventDestroy(c->ev_cvj);
+  if (c->side) {
+    (void)hipStreamSynchronize(c->side);
+    (void)hipStreamDestroy(c->side);
+  }
   if (c->ev_psi) (void)hipEventDestroy(c->ev_psi);
   if (c->ev_ang) (void)hipEventDestroy(c->ev_ang);
   if (c->stream) (void)hipStreamDestroy(c->stream);
@@ -208,8 +202,6 @@ int32_t mw3_create(const mw3_setup* setup, int32_t precision, mw3_ctx** out) {
   }
   c->s = *setup;
   c->precision = precision;
-  // the angular term beside the radial passes on its own stream in mixed
-  // precision (measured faster there; the FP64 pair ran slower side by side)
   c->opt_side = precision == MW3_MIXED ? 1 : 0;
   (void)hipGetDevice(&c->device);
   const HostTables& t = c->t;
@@ -225,20 +217,16 @@ int32_t mw3_create(const mw3_setup* setup, int32_t precision, mw3_ctx** out) {
     }                                                             \
   } while (0)
   CK(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking), "mw3_create: stream");
-  CK(hipStreamCreateWithFlags(&c->aux, hipStreamNonBlocking), "mw3_create: stream");
   // the stream-ordering events only order device work between the library's
   // streams (the host never queries them; host reads follow a stream
   // synchronize and a copy on the main stream), so they carry no system-scope
   // fence: with one, every record and wait wrote back and invalidated the
   // caches, about 10 us of idle GPU at each of the step's two crossings
   const unsigned evf = hipEventDisableTiming | hipEventDisableSystemFence;
-  CK(hipEventCreateWithFlags(&c->ev_slice, evf), "mw3_create: event");
-  CK(hipEventCreateWithFlags(&c->ev_cvj, evf), "mw3_create: event");
   CK(hipStreamCreateWithFlags(&c->side, hipStreamNonBlocking), "mw3_create: stream");
   CK(hipEventCreateWithFlags(&c->ev_psi, evf), "mw3_create: event");
   CK(hipEventCreateWithFlags(&c->ev_ang, evf), "mw3_create: event");
-  CK(hipEventCreateWithFlags(&c->ev_fork, evf), "mw3_create: event");
-  CK(alloc_zero((void**)&c->d_slot, sizeof(int32_t)), "mw3_create: ring slot");
+  CK(alloc_zero((void**)&c->d_slot, 2 * sizeof(int32_t)), "mw3_create: ring slot");
   CK(upload_raw(&c->d_pt_dense, t.pt_dense.data(), t.pt_dense.size()), "mw3_create: index map");
   CK(upload_raw(&c->d_mask, t.mask.data(), t.mask.size()), "mw3_create: mask");
 
@@ -332,53 +320,16 @@ int32_t mw3_create(const mw3_setup* setup, int32_t precision, mw3_ctx** out) {
   CK(upload_raw(&c->d_dcvj, t.dcvj.data(), t.dcvj.size()), "mw3_create: D");
   CK(upload_raw(&c->d_cvj_skip, t.cvj_isref.data(), t.cvj_isref.size()), "mw3_create: flags");
   {
-    // update work items: for each (channel, angle, 64-R chunk), the r rows with
-    // a point of the compressed grid in that chunk (static), cut into items of
-    // at most kUpdRows rows, one per wave of k_update
-    const int nrc = (t.n2 + 63) / 64;
-    std::vector<int32_t> rows, items, gfirst;
-    std::vector<uint64_t> words;
-    std::vector<int32_t> list_off((size_t)t.na * nrc), list_cnt((size_t)t.na * nrc);
-    for (int ia = 0; ia < t.na; ia++)
-      for (int rc = 0; rc < nrc; rc++) {
-        list_off[(size_t)ia * nrc + rc] = (int32_t)rows.size();
-        for (int r = 0; r < t.n1; r++) {
-          uint64_t wd = 0;
-          for (int l = 0; l < 64 && rc * 64 + l < t.n2; l++)
-            if (t.mask[(size_t)ia * t.nplane + (size_t)r * t.n2 + rc * 64 + l]) wd |= 1ull << l;
-          if (wd) {
-            rows.push_back(r);
-            words.push_back(wd);
-          }
-        }
-        list_cnt[(size_t)ia * nrc + rc] = (int32_t)rows.size() - list_off[(size_t)ia * nrc + rc];
+    // per r row: absorption factor and flux derivative (zeros past n1)
+    std::vector<double> row((size_t)4 * ((t.n1 + 15) / 16 * 16), 0.0);
+    for (int r = 0; r < t.n1; r++) {
+      row[(size_t)4 * r] = setup->absfr1[r];
+      if (2 * (size_t)r + 1 < t.zar1flux.size()) {
+        row[(size_t)4 * r + 1] = t.zar1flux[(size_t)2 * r];
+        row[(size_t)4 * r + 2] = t.zar1flux[(size_t)2 * r + 1];
       }
-    for (int ch = 0; ch < t.nc; ch++)
-      for (int ia = 0; ia < t.na; ia++)
-        for (int rc = 0; rc < nrc; rc++) {
-          const int gi = (ch * t.na + ia) * nrc + rc;
-          gfirst.push_back((int32_t)(items.size() / 4));
-          const int lo = list_off[(size_t)ia * nrc + rc], n = list_cnt[(size_t)ia * nrc + rc];
-          for (int k = 0; k < n; k += kUpdRows) {
-            items.push_back(gi);
-            items.push_back(lo + k);
-            items.push_back(std::min(kUpdRows, n - k));
-            items.push_back(0);
-          }
-        }
-    gfirst.push_back((int32_t)(items.size() / 4));
-    if (rows.empty()) {  // keep the arrays non-empty
-      rows.push_back(0);
-      words.push_back(0);
     }
-    c->nnorm_blocks = (int)(items.size() / 4);
-    CK(upload_raw(&c->d_uw_row, rows.data(), rows.size()), "mw3_create: update rows");
-    CK(upload_raw(&c->d_uw_word, words.data(), words.size()), "mw3_create: update rows");
-    if (!items.empty())
-      CK(upload_raw(&c->d_uw_item, items.data(), items.size()), "mw3_create: update items");
-    CK(upload_raw(&c->d_uw_gfirst, gfirst.data(), gfirst.size()), "mw3_create: update items");
-    CK(alloc_zero((void**)&c->d_uw_part, sizeof(double) * 3 * 64 * std::max(1, c->nnorm_blocks)),
-       "mw3_create: update partials");
+    CK(upload_raw(&c->d_up_row, row.data(), row.size()), "mw3_create: update rows");
   }
   {
     std::vector<int32_t> fmap((size_t)t.nc * t.na * t.n2, -1);
@@ -393,11 +344,11 @@ int32_t mw3_create(const mw3_setup* setup, int32_t precision, mw3_ctx** out) {
     std::vector<int32_t> i1f(t.ir1flux.begin(), t.ir1flux.end());
     if (i1f.empty()) i1f.assign(t.na, 1);
     CK(upload_raw(&c->d_ir1flux, i1f.data(), i1f.size()), "mw3_create: flux map");
-    CK(alloc_zero((void**)&c->d_slice, sizeof(double) * (size_t)t.nc * t.n1 * t.na),
-       "mw3_create: slice");
+    if (t.ncvj > 0)
+      CK(alloc_zero((void**)&c->d_ring_slice,
+                    sizeof(double) * kRing * (size_t)t.nc * t.n1 * t.na),
+         "mw3_create: slice");
   }
-  CK(alloc_zero((void**)&c->d_norm_part, sizeof(double) * 2 * std::max(1, c->nnorm_blocks)),
-     "mw3_create: norms");
   CK(alloc_zero((void**)&c->d_ring_norm, sizeof(double) * 2 * kRing), "mw3_create: norms");
   if (setup->nofe > 0) {
     if (!setup->efe) {
@@ -409,6 +360,12 @@ int32_t mw3_create(const mw3_setup* setup, int32_t precision, mw3_ctx** out) {
     CK(alloc_zero((void**)&c->d_zfe, sizeof(double) * 2 * setup->nofe * nd), "mw3_create: zfe");
   }
   CK(build_plans(c), "mw3_create: plans");
+  CK(alloc_zero((void**)&c->d_norm_part,
+                sizeof(double) * 2 * kRing * (size_t)std::max(1, c->up_nwaves)),
+     "mw3_create: norms");
+  CK(alloc_zero((void**)&c->d_up_part,
+                sizeof(double) * kRing * (size_t)std::max(1, c->up_nseg) * 64 * c->up_nt),
+     "mw3_create: segment sums");
   CK(hipStreamSynchronize(c->stream), "mw3_create: sync");
 #undef CK
   *out = reinterpret_cast<mw3_ctx*>(c);
@@ -437,6 +394,7 @@ int32_t mw3_hphi(mw3_ctx* ctx, const double* psi, double* hpsi) {
          "mw3_hphi: upload");
   HIPCHK(c, launch_scatter_a0(c, c->d_a0, c->d_scratch), "mw3_hphi: scatter");
   HIPCHK(c, launch_to_f32(c, c->d_scratch, c->d_scr32), "mw3_hphi: FP32 copy");
+  c->g_fresh = false;
   HIPCHK(c, launch_hpsi(c, c->d_scratch), "mw3_hphi: H psi");
   HIPCHK(c, launch_update(c, 0, c->d_scratch), "mw3_hphi: H psi");
   HIPCHK(c, launch_gather_a0(c, c->d_hout, c->d_a0b), "mw3_hphi: gather");
@@ -475,6 +433,7 @@ int32_t mw3_cheby_begin(mw3_ctx* ctx, const double* psi0, double* stats3) {
   size_t bytes = sizeof(double) * (size_t)c->t.nc * c->t.nslab;
   HIPCHK(c, hipMemcpyAsync(c->d_psi0, c->d_psi, bytes, hipMemcpyDeviceToDevice, c->stream),
          "mw3_cheby_begin: copy");
+  c->g_fresh = false;
   // psi_1 = (H psi_0 - emindlt psi_0)/delta2 is written over psim1; the swap
   // then leaves psi_k = psi_1 and psi_{k-1} = psi_0
   HIPCHK(c, launch_hpsi(c, c->d_psi), "mw3_cheby_begin: H psi0");
@@ -511,8 +470,6 @@ int32_t mw3_cheby_begin(mw3_ctx* ctx, const double* psi0, double* stats3) {
   return MW3_OK;
 }
 
-static int run_deferred(Ctx* c);
-
 // Values of one step's Cvjprod record: the product projection's rows when one
 // is attached and the energy sums run (netot > 0), else none.
 static size_t rec_nprod(const Ctx* c) {
@@ -520,13 +477,8 @@ static size_t rec_nprod(const Ctx* c) {
 }
 
 static int flush_ring(Ctx* c, double* norms_dst, double* auto_dst) {
-  int rd = run_deferred(c);
-  if (rd) return rd;
-  if (c->cvj_pending) {  // the reactant-state sums of the ring are done first
-    HIPCHK(c, hipStreamWaitEvent(c->stream, c->ev_cvj, 0), "ring flush: wait");
-    c->cvj_pending = false;
-  }
   if (c->ring_fill == 0) return MW3_OK;
+  HIPCHK(c, launch_ring_sums(c), "ring sums");
   HIPCHK(c, launch_energy_accum(c), "energy accumulation");
   std::vector<double> nb(2 * (size_t)c->ring_fill);
   HIPCHK(c, hipMemcpyAsync(nb.data(), c->d_ring_norm, nb.size() * sizeof(double),
@@ -567,32 +519,15 @@ static bool graphs_usable(const Ctx* c) {
   return c->graph_mode && !(c->timing && c->timing_step) && c->s.nofe <= 0;
 }
 
-// The captured step body of c on its own streams: on the second stream the
-// projection sums of the step before (ring slot from the device counter,
-// which they advance), beside this step's H psi; then, once both are done,
-// the update (it rewrites the partials those sums read).  Every stream
-// forked from c's main stream joins it again before the update.
+// The captured step body: H psi of psi_k (whose G the step before left), then
+// the update; the ring slot is read on the device.
 static hipError_t capture_body(Ctx* c) {
+  const bool g = c->g_fresh;
   c->graph_slot_dev = true;
-  c->slice_fresh = false;
-  auto body = [&]() -> hipError_t {
-    hipError_t r;
-    if ((r = hipEventRecord(c->ev_fork, c->stream)) != hipSuccess) return r;
-    if ((r = hipStreamWaitEvent(c->aux, c->ev_fork, 0)) != hipSuccess) return r;
-    if ((r = launch_tail_sums(c, 0, c->aux)) != hipSuccess) return r;
-    if ((r = launch_slot_next(c, c->aux)) != hipSuccess) return r;
-    if ((r = hipEventRecord(c->ev_cvj, c->aux)) != hipSuccess) return r;
-    c->cvj_pending = true;
-    if ((r = launch_hpsi(c, c->d_psi)) != hipSuccess) return r;
-    if (!c->cvj_joined && (r = hipStreamWaitEvent(c->stream, c->ev_cvj, 0)) != hipSuccess)
-      return r;
-    return launch_update(c, 2, c->d_psi, true);
-  };
-  hipError_t e = body();
+  hipError_t e = launch_hpsi(c, c->d_psi);
+  if (e == hipSuccess) e = launch_update(c, 2, c->d_psi, true);
   c->graph_slot_dev = false;
-  c->cvj_pending = false;  // the graph's second-stream work ends inside the graph
-  c->cvj_joined = false;
-  c->slice_fresh = false;
+  c->g_fresh = g;
   return e;
 }
 
@@ -620,16 +555,6 @@ void drop_graphs(Ctx* c) {
     }
 }
 
-// the projection sums of the last step, when a captured step left them
-// pending, enqueued the ordinary way
-static int run_deferred(Ctx* c) {
-  if (c->deferred_slot < 0) return MW3_OK;
-  const int slot = c->deferred_slot;
-  c->deferred_slot = -1;
-  HIPCHK(c, launch_projections(c, slot), "mw3_cheby_steps: projections");
-  return MW3_OK;
-}
-
 // Step of c, first part: ring bookkeeping and whether the step may run as a
 // graph.
 static bool step_pre(Ctx* c) {
@@ -638,38 +563,29 @@ static bool step_pre(Ctx* c) {
   return graphs_usable(c);
 }
 
-// Step of c, second part: the kernels, as a graph or one by one.
+// Step of c, second part: the kernels, as a graph or one by one (a step whose
+// psi has no G yet runs one by one: it forms G first).
 static int step_body(Ctx* c, bool graphs) {
-  if (graphs && c->deferred_slot >= 0) {
+  if (graphs && (c->g_fresh || !c->up_nk1 || !c->opt_radial)) {
     const int q = c->d_psi == c->graph_psi0 ? 0 : 1;
+    if (c->dslot_host != c->ring_fill)
+      HIPCHK(c, launch_slot_set(c, q, c->ring_fill), "mw3_cheby_steps: slot");
+    c->dslot_host = c->ring_fill + 1;
     if (!c->graph[q]) HIPCHK(c, capture_step(c, q), "mw3_cheby_steps: step capture");
     HIPCHK(c, hipGraphLaunch(c->graph[q], c->stream), "mw3_cheby_steps: step graph");
     return MW3_OK;
   }
-  int rd = run_deferred(c);  // a graph step before this one left its sums pending
-  if (rd) return rd;
   HIPCHK(c, launch_hpsi(c, c->d_psi), "mw3_cheby_steps: H psi");
-  // the update rewrites the slice the last k_cvj reads (already waited for
-  // through ev_ang when the angular term ran on the third stream)
-  if (c->cvj_pending && !c->cvj_joined)
-    HIPCHK(c, hipStreamWaitEvent(c->stream, c->ev_cvj, 0), "mw3_cheby_steps: wait");
   HIPCHK(c, launch_update(c, 2, c->d_psi, true), "mw3_cheby_steps: update");
-  if (graphs) {  // the next step's graph takes this step's sums (slot counter set here)
-    HIPCHK(c, launch_slot_set(c, c->ring_fill, c->stream), "mw3_cheby_steps: slot");
-  } else {
-    HIPCHK(c, launch_projections(c, c->ring_fill), "mw3_cheby_steps: projections");
-    c->slice_fresh = true;  // nothing below writes psi before the next H psi
-  }
   return MW3_OK;
 }
 
 // Step of c, last part: k, the psi buffers, and the ring flush when the ring
 // is full or when this is step nsteps of the call; *done counts the call's
 // steps (output index).
-static int step_post(Ctx* c, bool graphs, int32_t* done, int32_t nsteps, double* norms,
+static int step_post(Ctx* c, int32_t* done, int32_t nsteps, double* norms,
                      double* autocorr) {
   const int base = *done - c->ring_fill;  // output index of ring slot 0
-  if (graphs) c->deferred_slot = c->ring_fill;
   c->k += 1;
   if (!c->trial) HIPCHK(c, launch_psie(c, c->k), "mw3_cheby_steps: psi(E)");
   std::swap(c->d_psi, c->d_psim1);
@@ -677,19 +593,13 @@ static int step_post(Ctx* c, bool graphs, int32_t* done, int32_t nsteps, double*
   c->ring_fill += 1;
   *done += 1;
   if (c->trial && (c->ring_fill == kRing || *done == nsteps)) {
-    // autotuner trial: the step's sums end, the ring is discarded unread
-    int rc = run_deferred(c);
-    if (rc) return rc;
-    if (c->cvj_pending) HIPCHK(c, hipStreamWaitEvent(c->stream, c->ev_cvj, 0), "trial: wait");
-    c->cvj_pending = false;
+    // autotuner trial: the ring is discarded unread
     c->ring_fill = 0;
     return MW3_OK;
   }
   if (c->ring_fill == kRing || *done == nsteps) {
-    int rc = run_deferred(c);
-    if (rc) return rc;
     c->timing_step = true;  // the energy sums of every ring are timed
-    rc = flush_ring(c, norms ? norms + base : nullptr, autocorr ? autocorr + base : nullptr);
+    int rc = flush_ring(c, norms ? norms + base : nullptr, autocorr ? autocorr + base : nullptr);
     if (rc) return rc;
   }
   c->timing_step = true;
@@ -697,13 +607,12 @@ static int step_post(Ctx* c, bool graphs, int32_t* done, int32_t nsteps, double*
 }
 
 // One Chebyshev step of c (H psi_k, update into psim1 = psi_{k+1},
-// projections, swap).  In graph mode a step's projection sums run inside the
-// next step's graph (or before the flush), on the second stream as before.
+// projections, swap).
 static int step_enqueue(Ctx* c, int32_t* done, int32_t nsteps, double* norms, double* autocorr) {
   const bool graphs = step_pre(c);
   int rc = step_body(c, graphs);
   if (rc) return rc;
-  return step_post(c, graphs, done, nsteps, norms, autocorr);
+  return step_post(c, done, nsteps, norms, autocorr);
 }
 
 int32_t mw3_cheby_steps(mw3_ctx* ctx, int32_t nsteps, double* norms, double* autocorr) {
@@ -714,7 +623,6 @@ int32_t mw3_cheby_steps(mw3_ctx* ctx, int32_t nsteps, double* norms, double* aut
   int32_t done = 0;
   int rc = MW3_OK;
   while (done < nsteps && rc == MW3_OK) rc = step_enqueue(c, &done, nsteps, norms, autocorr);
-  c->slice_fresh = false;  // the caller may write psi before the next H psi
   return rc;
 }
 
@@ -742,8 +650,6 @@ int32_t mw3_cheby_steps_batch(mw3_ctx** ctxs, int32_t n, int32_t nsteps, double*
       rc = step_enqueue(c, &done[i], nsteps, norms ? norms + (size_t)i * nsteps : nullptr,
                         nullptr);
     }
-  for (int i = 0; i < n; i++)  // the caller may write psi before the next H psi
-    reinterpret_cast<Ctx*>(ctxs[i])->slice_fresh = false;
   return rc;
 }
 
@@ -896,7 +802,6 @@ int32_t mw3_psie_get(mw3_ctx* ctx, double* zfe) {
 
 static void free_prod(Ctx* c) {
   void** ptrs[] = {&c->d_tprod,
-                   (void**)&c->d_ppart,
                    (void**)&c->d_dtrans,
                    (void**)&c->d_ring_prod,
                    (void**)&c->d_prodwf,
@@ -1014,8 +919,6 @@ int32_t mw3_prod_attach(mw3_ctx* ctx, const mw3_prod_setup* ps) {
     e = upload_raw(&c->d_dtrans, ps->dtrans, (size_t)t.nc * c->pr_nomb * L);
   if (e == hipSuccess) e = upload_raw(&c->d_prodwf, wf.data(), wf.size());
   if (e == hipSuccess)
-    e = alloc_zero((void**)&c->d_ppart, sizeof(double) * 64 * std::max(1, c->nnorm_blocks));
-  if (e == hipSuccess)
     e = alloc_zero((void**)&c->d_ring_prod, sizeof(double) * kRing * (size_t)c->pr_nomb * K);
   if (e == hipSuccess)
     e = alloc_zero((void**)&c->d_prod_part,
@@ -1101,6 +1004,7 @@ int32_t mw3_state_put(mw3_ctx* ctx, const double* psi_km1, const double* psi_k, 
   HIPCHK(c, hipMemcpyAsync(c->d_a0b, psi_k, n * sizeof(double), hipMemcpyHostToDevice, c->stream),
          "mw3_state_put");
   HIPCHK(c, launch_scatter_a0(c, c->d_a0b, c->d_psi), "mw3_state_put");
+  c->g_fresh = false;
   HIPCHK(c, launch_to_f32(c, c->d_psi, c->d_psi32), "mw3_state_put: FP32 copy");
   HIPCHK(c, launch_to_f32(c, c->d_psim1, c->d_psim132), "mw3_state_put: FP32 copy");
   if (psi0) {
@@ -1119,6 +1023,7 @@ int32_t mw3_set_option(mw3_ctx* ctx, int32_t option, int32_t value) {
   if (!c) return MW3_EINVAL;
   int rc = flush_ring(c, nullptr, nullptr);  // no step of the old setting left pending
   if (rc) return rc;
+  c->g_fresh = false;
   switch (option) {
     case MW3_OPT_GRAPHS:
       if (value != 0 && value != 1) return seterr(c, MW3_EINVAL, "mw3_set_option: graphs 0 or 1");
@@ -1164,11 +1069,11 @@ int32_t mw3_set_option(mw3_ctx* ctx, int32_t option, int32_t value) {
 }
 
 // the variant each option value selects in this context (the fallback where
-// the kernel of that value is not built): radial 1 needs the persistent R
-// passes or the fused r passes; angular 0 the folded kernel, 1 a one-pass one
+// the kernel of that value is not built): radial 1 needs the low modes to fit
+// the update's tiles or one of the low-mode passes; angular 0 the folded kernel, 1 a one-pass one
 static void effective_options(const Ctx* c, int32_t* out) {
   out[MW3_OPT_GRAPHS] = c->graph_mode;
-  out[MW3_OPT_RADIAL] = c->opt_radial && (c->rad_nitems || c->mid_nitems) ? 1 : 0;
+  out[MW3_OPT_RADIAL] = c->opt_radial && (c->up_nk1 || c->rad_nitems || c->mid_nitems) ? 1 : 0;
   int a = c->opt_angular;
   const bool cor_fold = c->ang_fold_cor && c->precision == MW3_MIXED && c->opt_fp16;
   if (a == 0 && !c->ang_fold && !cor_fold) a = 1;
@@ -1176,11 +1081,7 @@ static void effective_options(const Ctx* c, int32_t* out) {
   if (a == 1 && !c->ang_nt) a = 0;
   out[MW3_OPT_ANGULAR] = a;
   out[MW3_OPT_SIDE_STREAM] = c->opt_side;
-  // the grid divisor applies to the staged R-pass kernels only: the FP32
-  // passes, and the FP64 ones with their table split over block pairs, run
-  // with the table in LDS on a grid of their own
-  const bool staged = c->precision != MW3_MIXED && !c->rad_lds64;
-  out[MW3_OPT_RADIAL_GRID] = c->rad_nitems && c->opt_radial && staged ? c->opt_rad_grid : 1;
+  out[MW3_OPT_RADIAL_GRID] = 1;  // no radial kernel has a grid to divide
   out[MW3_OPT_ANGULAR_GRID] =
       (c->ang_fold || cor_fold) && out[MW3_OPT_ANGULAR] == 0 ? c->opt_ang_grid : 1;
   out[MW3_OPT_FP16_PRODUCTS] = c->precision == MW3_MIXED ? c->opt_fp16 : 0;
@@ -1284,6 +1185,7 @@ int32_t mw3_autotune(mw3_ctx* ctx, int32_t trial_steps, int32_t* chosen, double*
   for (const auto& key : cands) {
     drop_graphs(c);
     apply(key);
+    c->g_fresh = false;
     double ms = 0;
     rc = trial_ms(c, n, e0, e1, &ms);
     if (rc) break;
@@ -1303,8 +1205,7 @@ int32_t mw3_autotune(mw3_ctx* ctx, int32_t trial_steps, int32_t* chosen, double*
   c->k = k0;
   c->ring_k0 = rk0;
   c->ring_fill = 0;
-  c->deferred_slot = -1;
-  c->slice_fresh = false;
+  c->g_fresh = false;
   HIPCHK(c, hipMemcpyAsync(c->d_psi, c->d_hout, bytes, hipMemcpyDeviceToDevice, c->stream),
          "mw3_autotune: restore");
   HIPCHK(c, hipMemcpyAsync(c->d_psim1, c->d_scratch, bytes, hipMemcpyDeviceToDevice, c->stream),

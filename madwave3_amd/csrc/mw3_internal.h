@@ -115,33 +115,35 @@ struct Ctx {
   HostTables t;
   std::string err;
   hipStream_t stream = nullptr;
-  // second stream (default priority) for the reactant-state sums, which then
-  // overlap the next step's H psi: ev_slice orders them after the update that
-  // wrote the slice, ev_cvj orders the next update and the ring flush after them
-  hipStream_t aux = nullptr;
-  hipEvent_t ev_slice = nullptr, ev_cvj = nullptr;
-  // third stream: the angular term runs beside the radial passes; ev_psi
+  // second stream (option): the angular term beside the radial passes; ev_psi
   // orders it after the update that wrote psi, ev_ang the next update after it
   hipStream_t side = nullptr;
   hipEvent_t ev_psi = nullptr, ev_ang = nullptr;
-  bool cvj_pending = false;
-  // step loop only: ev_slice follows main's last write of psi (the update),
-  // so the next H psi's third stream waits on it instead of a new record
-  bool slice_fresh = false;
-  bool cvj_joined = false;  // the third stream waited ev_cvj before ev_ang
   int device = 0;
 
   // device buffers
   uint32_t* d_pt_dense = nullptr;
   uint8_t* d_mask = nullptr;
-  // update work items (see mw3_create): rows and mask words of each
-  // (angle, 64-R chunk), items [nitems][4], item range per (channel, angle,
-  // chunk), flux partials [nitems][3][64]
-  int32_t* d_uw_row = nullptr;
-  uint64_t* d_uw_word = nullptr;
-  int32_t* d_uw_item = nullptr;
-  int32_t* d_uw_gfirst = nullptr;
-  double* d_uw_part = nullptr;
+  // update: strips of 16 up_nt consecutive R of one (channel, angle), their
+  // 16-row tiles with a kept point in runs of up_tmax per wave, and the radial
+  // tables (mw3_step.h)
+  void* d_up_wave = nullptr;        // [up_nwaves] step::UpWave
+  void* d_up_seg = nullptr;         // [up_nseg] step::UpSeg
+  uint32_t* d_up_tile = nullptr;    // [up_nwaves][up_tmax][64]
+  int32_t* d_up_sfirst = nullptr;   // [nc na up_ns + 1] first segment of each strip
+  double* d_up_part = nullptr;      // [kRing][up_nseg][4][16 up_nt] sums over r
+  int up_nwaves = 0, up_nseg = 0, up_tmax = 0, up_nt = 1, up_ns = 0, up_segmax = 0;
+  int up_nk1 = 0;                 // 16-mode tiles of the low r modes (0: radial GEMMs only)
+  int up_kst = 0;                 // low r modes kept of G, G2
+  int rr_np = 0, rr_nb = 0;       // k2 tiles per parity, 16-R blocks of a half row
+  double* d_up_row = nullptr;     // [16 ceil(n1/16)][4] absfr1, zAR1flux
+  void* d_up_tab = nullptr;       // S(r, k1) per r size
+  void* d_rr_f = nullptr;         // S(R, k2) by parity, forward and back order
+  void* d_rr_b = nullptr;
+  void* d_rr_w = nullptr;         // weights (radcut - E)_+ divi
+  void* d_g1 = nullptr;           // G of psi_k, segment sums [up_nseg][up_kst][16 up_nt]
+  void* d_g2 = nullptr;           // [nc na][up_ns][up_kst][16 up_nt]
+  bool g_fresh = false;           // d_g1 is G of d_psi
   void* d_v = nullptr;  // double or float dense V
   double* d_absfr1 = nullptr;
   double* d_absfr2 = nullptr;
@@ -175,7 +177,7 @@ struct Ctx {
   int32_t* d_nbr = nullptr;
   // projections
   uint32_t* d_flux_dense = nullptr;
-  uint32_t* d_flux_col = nullptr;
+  uint32_t* d_flux_col = nullptr; // [nflux] dense index of (c, ia, 0, ir2)
   double* d_zar1flux = nullptr;
   double* d_ring_zr = nullptr;   // [kRing][nflux]
   double* d_ring_zdr = nullptr;  // [kRing][nflux][2]
@@ -187,11 +189,10 @@ struct Ctx {
   double* d_fdv = nullptr;
   double* d_dcvj = nullptr;
   uint8_t* d_cvj_skip = nullptr; // [ncvj] 1 if the reference state (kminelastic)
-  double* d_norm_part = nullptr; // partial sums [nblocks][2]
+  double* d_norm_part = nullptr; // update wave sums [kRing][up_nwaves][2]
   double* d_ring_norm = nullptr; // [kRing][2] (norm, autocorrelation)
   double* d_efe = nullptr;
   double* d_zfe = nullptr;       // [nofe][nc*nslab][2] dense
-  int nnorm_blocks = 0;  // update work items (norm partials)
   int ring_fill = 0;             // steps buffered in the ring
   int ring_k0 = 0;               // k of ring slot 0
   std::vector<double> host_norms;
@@ -203,11 +204,9 @@ struct Ctx {
 
   // GEMM passes: R rows, r columns, angular forward, angular back
   GemmPlan p_dstR, p_dstr, p_dstr2, p_dstRi, p_angF, p_angB;
-  bool ang_fused = false;  // FBR coefficients applied in the forward GEMM (no Coriolis)
-  int ang_nt = 0;          // 16-row tiles of the one-pass angular kernel (0: two GEMMs)
   int32_t* d_rad_items = nullptr;  // R-pass work items {channel-angle, 16-row tile, nn1, k2lo}
   int rad_nitems = 0;              // 0: the R passes run as GEMMs
-  int rad_grid[2] = {0, 0};        // persistent blocks of the forward / inverse R pass
+  int rad_ncu = 1;                 // compute units
   void* d_lowT = nullptr;          // transposed low-mode r tables of k_rad_mid
   int32_t* d_mid_items = nullptr;  // its work items (int4)
   int32_t* d_mid_sizes = nullptr;  // its per-size table records (int4)
@@ -216,9 +215,8 @@ struct Ctx {
   int mid_rbw = 0;                 // r blocks per wave of the FP32 kernel
   int mid_nitems = 0;              // 0: the r passes run as two GEMMs
   int mid_nk1 = 0;                 // 16-row tiles of the low r modes
-  int rad_ncu = 1;                 // compute units (the LDS-table R passes)
-  bool rad_lds64 = false;          // FP64 R passes with the table split over block pairs
-  bool rad_inv_h = false;          // FP32 inverse R pass with compensated FP16 products
+  bool ang_fused = false;  // FBR coefficients applied in the forward GEMM (no Coriolis)
+  int ang_nt = 0;          // 16-row tiles of the one-pass angular kernel (0: two GEMMs)
   bool ang_fold_h = false;         // FP32 folded angular kernel with compensated FP16 products
   int ang_fold_h_nbc = 0;          // its blocks per channel
   int ang_fold_cor = 0;            // tiles of the folded forward / back parts with Coriolis (mixed)
@@ -252,16 +250,16 @@ struct Ctx {
 
   int32_t* d_fmap = nullptr;     // [nc][na][n2] flux point index or -1
   int32_t* d_ir1flux = nullptr;  // [na]
-  double* d_slice = nullptr;     // [nc][na][n1] psi at R = ir2abs / sqrt(ah2)
+  double* d_ring_slice = nullptr; // [kRing][nc][na][n1] psi at R = ir2abs / sqrt(ah2)
 
   // product-state projection (iprod = 2, mw3_prod_attach).  Per step, the
-  // update sums T psi_new over r into d_ppart (T = transRgjac on the dense
-  // grid); k_prod_fun reduces them to funprod(c, l), l = (angle, R) of the
-  // projection range, rotates by dtrans and sums the channels of each
-  // electronic state into the ring d_ring_prod[slot][Omega'][e][l].  At each
-  // ring flush one split-K GEMM per Omega' projects the ring on prodwf:
-  // Cvjprod[s][Omega'][j'v'] (partials [Omega'][chunk][kRing][nvj]), then the
-  // energy accumulation adds C_k(E) Cvjprod to zS2prod.
+  // update leaves funprod(c, l) = sum_r T psi_new (T = transRgjac on the dense
+  // grid), l = (angle, R) of the projection range, in its segment sums.  At
+  // each ring flush dtrans rotates it and the channels of each electronic
+  // state are summed into d_ring_prod[slot][Omega'][e][l], one split-K GEMM
+  // per Omega' projects that on prodwf: Cvjprod[s][Omega'][j'v'] (partials
+  // [Omega'][chunk][kRing][nvj]), and the energy accumulation adds
+  // C_k(E) Cvjprod to zS2prod.
   bool prod_on = false;
   int pr_n2p0 = 0, pr_nap0 = 0, pr_n2p = 0, pr_nap = 0, pr_nomb = 0, pr_nvj = 0;
   int pr_nchunk = 0, pr_kc = 0;
@@ -269,7 +267,6 @@ struct Ctx {
   int64_t pr_tstride = 0;        // channel stride of d_tprod (0: one table for all)
   std::vector<int32_t> pr_shape; // iomminprod, iommaxprod, nviniprod, nvmaxprod, jiniprod, jmaxprod
   void* d_tprod = nullptr;       // T or float dense [nct][na][n1][n2]
-  double* d_ppart = nullptr;     // [nitems][64]
   double* d_dtrans = nullptr;    // [nc][nomb][L]
   double* d_ring_prod = nullptr; // [kRing][nomb][ne][L]
   double* d_prodwf = nullptr;    // [nomb][nvj][ne][L]
@@ -283,10 +280,10 @@ struct Ctx {
   int k = 0;
   bool begun = false;
 
-  // captured steps (hipGraph): graph[q] is one step -- the projection sums of
-  // the step before on the second stream beside this step's H psi, then the
-  // update -- for psi in buffer q (0: the buffer d_psi held at creation);
-  // d_slot is the ring slot of those projection sums, advanced by the graph
+  // captured steps (hipGraph): graph[q] is one step for psi in buffer q (0:
+  // the buffer d_psi held at creation); d_slot[q] is the ring slot of the step,
+  // left there by the captured step before it; dslot_host the slot that was
+  // left last
   int graph_mode = 1;             // 0: off; 1: on when the context allows it
   // execution options (include/mw3.h MW3_OPT_*): radial passes as the
   // persistent low-mode kernels (1) or as GEMMs (0); angular term by the
@@ -294,7 +291,7 @@ struct Ctx {
   // GEMMs (2), each falling back to the next where not built; the angular
   // term on the third stream (1) or the main one (0)
   int opt_radial = 1, opt_angular = 0, opt_side = 0;
-  int opt_rad_grid = 1;           // persistent radial grids: resident blocks / this
+  int opt_rad_grid = 1;           // accepted; no kernel has a radial grid to divide
   int opt_ang_grid = 1;           // folded angular kernel: blocks per channel / this
   int flux_etest = 1;             // E > V(flux point) test when the flux sums are read
   bool trial = false;             // autotuner trial steps: no ring flush, no psi(E)
@@ -302,8 +299,7 @@ struct Ctx {
   hipGraphExec_t graph[2] = {nullptr, nullptr};
   double* graph_psi0 = nullptr;   // d_psi at creation (buffer 0)
   int32_t* d_slot = nullptr;
-  int deferred_slot = -1;         // ring slot whose projection sums are not yet enqueued
-  hipEvent_t ev_fork = nullptr;
+  int dslot_host = -2;
 
   // timing
   bool timing = false;
@@ -329,8 +325,7 @@ hipError_t launch_spectrum(hipStream_t s, const double* d_auto, double* d_a, int
                            double delta2, double* d_spec);  // T, V and angular terms into work slabs
 // 0: H psi into d_hout, 1: first step, 2: damped step (psi_new into d_psim1)
 hipError_t launch_update(Ctx* c, int mode, const double* psi, bool proj = false);
-hipError_t launch_projections(Ctx* c, int slot);
-hipError_t launch_tail_sums(Ctx* c, int slot, hipStream_t st);
+hipError_t launch_ring_sums(Ctx* c);
 hipError_t launch_energy_accum(Ctx* c);
 hipError_t launch_psie(Ctx* c, int k);
 hipError_t launch_zero(Ctx* c, void* p, size_t bytes);
@@ -339,10 +334,9 @@ void free_plans(Ctx* c);
 hipError_t launch_flux_result(Ctx* c, double* d_out /* [(1+ne)][netot] */);
 // product projection: plan of the flush GEMM, per-step reduction into the ring
 hipError_t build_prod_plan(Ctx* c);
-hipError_t launch_prod_step(Ctx* c, int slot, hipStream_t s);
+hipError_t launch_prod_sums(Ctx* c);
 hipError_t launch_prod_flush(Ctx* c);
 
-constexpr int kUpdRows = 32;  // rows per update work item
 // most channels of one product-state context (LDS of the per-step product
 // reduction: 64 doubles per channel)
 constexpr int kProdMaxCh = 64;
@@ -368,13 +362,21 @@ enum KernelId {
   K_PROJ = 6,
   K_ENERGY = 7,
   K_CORIOLIS = 8,  // FBR coefficients with the Omega +- 1 Coriolis stencil (k_fbr_coef)
-  K_PROD = 9,      // product projection: per-step reduction (the flush GEMM is in K_ENERGY)
-  K_UPDATE_TAIL = 10,  // flux columns and norm from the update partials (second stream)
+  K_PROD = 9,      // product projection: rotation and channel sums of a ring (the GEMM is in K_ENERGY)
+  K_UPDATE_TAIL = 10,  // norms of a ring from the update block sums
 };
 
-hipError_t launch_update_tail(Ctx* c, int mode, int slot, bool proj, hipStream_t st);
-hipError_t launch_slot_set(Ctx* c, int v, hipStream_t st);
-hipError_t launch_slot_next(Ctx* c, hipStream_t st);
+hipError_t launch_slot_set(Ctx* c, int q, int v);
+namespace step {
+struct UpArgs;
+struct RrArgs;
+}
+// mw3_step_f32.hip, mw3_step_f64.hip
+hipError_t step_build_f32(Ctx* c);
+hipError_t step_build_f64(Ctx* c);
+hipError_t step_update_f32(Ctx* c, const step::UpArgs& a, int nk1, int cpl, int aux, int mode);
+hipError_t step_update_f64(Ctx* c, const step::UpArgs& a, int nk1, int cpl, int aux, int mode);
+hipError_t step_rad_rr_f64(Ctx* c, const step::RrArgs& a);
 void timer_begin(Ctx* c, int id, hipStream_t s = nullptr);
 void timer_end(Ctx* c, int id, hipStream_t s = nullptr);
 

@@ -2,26 +2,27 @@
 //
 // One Chebyshev step of SRC/main_madwave3.f:324-353 is:
 //   radial kinetic  (SRC/mod_Hphi_01y2.f:762-832): 2-D DST-I, scale, 2-D DST-I
-//                   as three passes over the dense slabs (R rows, r columns
-//                   with scaling, R rows);
+//                   on its low modes: products over r in the update kernels,
+//                   over R between them (mw3_step.h), or four batched GEMMs;
 //   angular term    (SRC/mod_Hphi_01y2.f:859-902) in factor form:
 //                   FBR = D^T psi, stencil over Omega with the j^2 / l^2
 //                   coefficients, back with D;
 //   fused update    V psi (SRC/mod_Hphi_01y2.f:838-853), compressed-grid
 //                   projection, damped three-term update
-//                   (SRC/main_madwave3.f:332-339), norm partial sums;
-//   projections     flux-line samples (SRC/mod_flux_01y2.f:598-628) and
-//                   reactant-state amplitudes (SRC/mod_flux_01y2.f:672-702)
-//                   into a ring of kRing steps; the energy sums
-//                   sum_k C_k(E) x_k (CoefEcheby, SRC/main_madwave3.f:462-490)
-//                   run once per ring as a complex GEMM.
+//                   (SRC/main_madwave3.f:332-339), the sums over r of the
+//                   per-step projections (mw3_step.h);
+//   once per ring of kRing steps: norms, flux-line samples
+//                   (SRC/mod_flux_01y2.f:598-628), reactant- and product-state
+//                   amplitudes (SRC/mod_flux_01y2.f:672-702), and the energy
+//                   sums sum_k C_k(E) x_k (CoefEcheby,
+//                   SRC/main_madwave3.f:462-490) as complex products.
 #include <hip/hip_runtime.h>
 
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
 
-#include "mw3_internal.h"
+#include "mw3_step.h"
 
 namespace mw3 {
 
@@ -523,29 +524,6 @@ __global__ void k_zero(uint32_t* p, int64_t nwords) {
 }
 
 // ---------------------------------------------------------------------------
-// kinetic scaling between the forward and inverse r transforms
-// ---------------------------------------------------------------------------
-template <typename T>
-__global__ void k_kin_scale(T* __restrict__ x, const int32_t* __restrict__ nn1,
-                            const double* __restrict__ p2r1, const double* __restrict__ p2r2,
-                            const double* __restrict__ divi, double radcut, int nc, int na, int n1,
-                            int n2) {
-  // one block row per (c, ia, k1)
-  int64_t row = blockIdx.x;
-  int k1 = row % n1;
-  int ia = (row / n1) % na;
-  if (k1 >= nn1[ia]) return;
-  T* xr = x + row * n2;
-  double p1 = p2r1[(int64_t)ia * n1 + k1];
-  double dv = divi[ia];
-  for (int k2 = threadIdx.x; k2 < n2; k2 += blockDim.x) {
-    double e = p1 + p2r2[k2];
-    if (e > radcut) e = radcut;
-    xr[k2] = (T)((double)xr[k2] * e * dv);
-  }
-}
-
-// ---------------------------------------------------------------------------
 // angular stencil in the FBR: phi_t = (a_t(r) + b_t0(R)) f_t + b_t-(R) f_s- + b_t+(R) f_s+
 // ---------------------------------------------------------------------------
 template <typename T>
@@ -628,325 +606,41 @@ __global__ __launch_bounds__(FBR_THREADS) void k_fbr_coef_all(const T* __restric
 }
 
 // ---------------------------------------------------------------------------
-// Fused V psi + compressed-grid projection + damped update
-// (SRC/mod_Hphi_01y2.f:838-853, SRC/main_madwave3.f:245-248, 332-339) with the
-// per-step projections of the new psi (SRC/mod_flux_01y2.f:598-628, 672-702).
-// Block = one (channel, angle) and 64 consecutive R; its 8 waves take the r
-// rows r = w, w+8, ...; lane = R, so every row access is one contiguous run.
-// Points outside the compressed grid are neither read nor written: every
-// state buffer is zero there and stays zero.  mode 0: hout = H psi;
-// mode 1: out = H_norm psi (first step, undamped); mode 2: damped update.
-// proj: also sum zAR1flux(r) psi_new(r, R) and take psi_new(ir1flux, R) for the
-// flux columns, and psi_new(r, ir2abs) / sqrt(ah2) for the reactant slice.
-struct UpdArgs {
-  const int32_t* items;  // [nitems][4]: group (c, ia, R chunk), first row entry, count, 0
-  const int32_t* urow;   // listed rows r
-  const uint64_t* uword; // their mask words
-  double* upart;         // [nitems][3][64] flux partials (sum zAR1flux psi: re, im; psi at ir1flux)
-  int nitems;
-  const int32_t* nn1;
-  const double* absfr1;
-  const double* absfr2;
-  const int32_t* ch_elec;
-  const int32_t* ch_omega;
-  const int32_t* ch_cpl;  // [nc][4] coupled channels (CPL4 kernels)
-  const double* psi0;  // autocorrelation reference (null: none)
-  double* part;        // per-block (norm, autocorrelation) partials
-  int nc, ne, na, n1, n2;
-  double emindlt, rdelta2, radcut;
-  int mode, pflux;  // pflux: flux-column projections on
-  // projections (slice non-null: reactant slice on)
-  const int32_t* fmap;
-  const int32_t* ir1flux;
-  const double* zar;
-  double* zr;
-  double* zdr;
-  double* slice;
-  float* out32;  // FP32 copy of the new psi (mixed precision), or null
-  // mixed precision, damped update: psi_k enters only through the operator
-  // (its diagonal V, radcut and emindlt terms), so it is read from its FP32
-  // copy like every other operator input
-  const float* psi32;
-  int ir2abs;
-  double rsah2;
-  // product projection: per item and lane (R), sum over the item's rows of
-  // T(c, ia, r, R) psi_new (T = transRgjac, operator precision)
-  const void* tprod;
-  int64_t tp_cstride;
-  double* ppart;  // [nitems][64]
-};
-
-
-// MODE 0: hout = H psi; 1: first step (undamped); 2: damped update.  SINGLE:
-// one electronic state (V diagonal; any number of Omega channels).  PROJ: flux columns and reactant
-// slice.  AUTO: <psi_0|psi_new> partials.  PRODP: product-projection partials.
-// All are template parameters so that no load sits behind a runtime branch
-// (the compiler waits for every load at the join of such a branch, which
-// serialises the batch).
-// CPL4 (several states): at most 4 channels share an Omega; their V and psi
-// values are loaded with the row's other loads, from the host-built list.
-template <typename TT, typename TV, int MODE, bool SINGLE, bool PROJ, bool AUTO, bool PRODP,
-          bool CPL4 = false>
-__global__ __launch_bounds__(256) void k_update(const double* __restrict__ psi,
-                                               double* __restrict__ out_buf,
-                                               const TT* __restrict__ tkin,
-                                               const TT* __restrict__ ang,
-                                               const TV* __restrict__ vd, UpdArgs a) {
-  const int64_t plane = (int64_t)a.n1 * a.n2, slab = (int64_t)a.na * plane;
-  const int nrc = (a.n2 + 63) / 64;
-  const int lane = threadIdx.x & 63;
-  const int item = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * 4 + (threadIdx.x >> 6)));
-  if (item >= a.nitems) return;  // no block-level synchronisation in this kernel
-  const int g = a.items[4 * item], off = a.items[4 * item + 1], cnt = a.items[4 * item + 2];
-  const int rc = g % nrc, cia = g / nrc;
-  const int ia = cia % a.na, c = cia / a.na;
-  const int R = rc * 64 + lane;
-  const bool inR = R < a.n2;
-  const int Ra = inR ? R : a.n2 - 1;  // address of lanes past the grid (never used)
-  const int nn = a.nn1[ia];
-  const int et = a.ch_elec[c], om = a.ch_omega[c];
-  const double f2 = a.absfr2[Ra];
-  const int rflux = PROJ ? a.ir1flux[ia] - 1 : -1;
-  const bool cvjcol = PROJ && a.slice && R == a.ir2abs - 1;
-  double s_norm = 0.0, s_auto = 0.0, zre = 0.0, zim = 0.0, zval = 0.0, sprod = 0.0;
-  const TT* tprod = PRODP ? (const TT*)a.tprod + (int64_t)c * a.tp_cstride : nullptr;
-  constexpr bool P32 = MODE == 2 && sizeof(TT) == 4;  // psi_k from its FP32 copy
-  // the item's rows, four at a time: the loads of the four rows and their
-  // per-row tables are issued before any is used, with no branch around them
-  constexpr int NK = CPL4 ? 4 : 1;
-  // coupled channels: V and psi offsets and the 0 / 1 weight (entries past
-  // the count repeat the channel itself with weight 0), once per wave
-  int64_t cvo[NK], cpo[NK];
-  double cw[NK];
-#pragma unroll
-  for (int k = 0; k < NK; k++) {
-    const int s2r = CPL4 ? a.ch_cpl[4 * c + k] : c;
-    const int s2 = s2r >= 0 ? s2r : c;
-    cvo[k] = CPL4 ? ((int64_t)et * a.ne + a.ch_elec[s2]) * slab : 0;
-    cpo[k] = (int64_t)s2 * slab;
-    cw[k] = s2r >= 0 ? 1.0 : 0.0;
-  }
-  for (int b = 0; b < cnt; b += 4) {
-    bool act[4];
-    int rr[4];
-    int64_t pl[4];
-    double p[4], ob[4], tk[4], an[4], vv[4], f1[4], za[4], zb[4], p0[4], tp[4];
-    double cv[4][NK], cp[4][NK];
-#pragma unroll
-    for (int u = 0; u < 4; u++) {
-      const int idx = b + u < cnt ? b + u : cnt - 1;
-      rr[u] = a.urow[off + idx];
-      const uint64_t w = a.uword[off + idx];
-      const bool kept = (w >> lane) & 1ull;
-      act[u] = b + u < cnt && inR && kept;
-      // lanes without a kept point read the row's first kept point instead
-      // of their own: the row's loads then touch only the cache lines that
-      // hold kept points (the values they load are not used)
-      const int Ru = kept ? Ra : rc * 64 + (w ? (int)__builtin_ctzll(w) : 0);
-      pl[u] = (int64_t)ia * plane + (int64_t)rr[u] * a.n2 + Ru;
-    }
-#pragma unroll
-    for (int u = 0; u < 4; u++) {
-      const int r = rr[u];
-      const int64_t ie = (int64_t)c * slab + pl[u];
-      p[u] = P32 ? (double)a.psi32[ie] : psi[ie];
-      tk[u] = (double)tkin[ie];
-      an[u] = (double)ang[ie];
-      vv[u] = SINGLE ? (double)vd[pl[u]] : 0.0;
-      ob[u] = MODE == 2 ? out_buf[ie] : 0.0;
-      f1[u] = MODE == 2 ? a.absfr1[r] : 0.0;
-      za[u] = PROJ ? a.zar[2 * r] : 0.0;
-      zb[u] = PROJ ? a.zar[2 * r + 1] : 0.0;
-      p0[u] = AUTO ? a.psi0[ie] : 0.0;
-      tp[u] = PRODP ? (double)tprod[pl[u]] : 0.0;
-      if (CPL4) {
-#pragma unroll
-        for (int k = 0; k < NK; k++) {
-          cv[u][k] = (double)vd[cvo[k] + pl[u]];
-          cp[u][k] = P32 ? (double)a.psi32[cpo[k] + pl[u]] : psi[cpo[k] + pl[u]];
-        }
-      }
-    }
-#pragma unroll
-    for (int u = 0; u < 4; u++) {
-      if (!act[u]) continue;
-      const int r = rr[u];
-      const int64_t i = (int64_t)c * slab + pl[u];
-      // T psi = radcut psi - low-mode correction on r < nn1; psi beyond (Q1)
-      double h = (r < nn ? a.radcut * p[u] - tk[u] : p[u]) + an[u];
-      if (SINGLE) {
-        h += p[u] * vv[u];
-      } else if (CPL4) {
-#pragma unroll
-        for (int k = 0; k < NK; k++) h += cp[u][k] * (cv[u][k] * cw[k]);
-      } else {
-        for (int s2 = 0; s2 < a.nc; s2++) {
-          if (a.ch_omega[s2] != om) continue;
-          const int es = a.ch_elec[s2];
-          const double v = (double)vd[((int64_t)et * a.ne + es) * slab + pl[u]];
-          const int64_t is2 = (int64_t)s2 * slab + pl[u];
-          const double ps = (s2 == c) ? p[u] : (P32 ? (double)a.psi32[is2] : psi[is2]);
-          h += ps * v;
-        }
-      }
-      if (MODE == 0) {
-        out_buf[i] = h;
-        continue;
-      }
-      const double hn = (h - a.emindlt * p[u]) * a.rdelta2;
-      double o;
-      if (MODE == 1) {
-        o = hn;
-      } else {
-        const double f = f1[u] * f2;
-        o = (2.0 * hn - f * ob[u]) * f;
-      }
-      out_buf[i] = o;
-      if (a.out32) a.out32[i] = (float)o;
-      s_norm += o * o;
-      if (AUTO) s_auto += p0[u] * o;
-      if (PRODP) sprod += tp[u] * o;
-      if (PROJ) {
-        zre += za[u] * o;
-        zim += zb[u] * o;
-        if (r == rflux) zval = o;
-        if (cvjcol) a.slice[((int64_t)c * a.na + ia) * a.n1 + r] = o * a.rsah2;
-      }
-    }
-  }
-  if (PROJ) {
-    double* up = a.upart + (int64_t)item * 3 * 64;
-    up[lane] = zre;
-    up[64 + lane] = zim;
-    up[128 + lane] = zval;
-  }
-  if (PRODP) a.ppart[(int64_t)item * 64 + lane] = sprod;
-  if (a.part) {
-    for (int o2 = 32; o2 > 0; o2 >>= 1) {
-      s_norm += __shfl_xor(s_norm, o2);
-      s_auto += __shfl_xor(s_auto, o2);
-    }
-    if (lane == 0) {
-      a.part[2 * item] = s_norm;
-      a.part[2 * item + 1] = s_auto;
-    }
-  }
-}
-
-// flux columns of each (channel, angle, 64-R chunk) from the partials of its
-// work items (in item order); chunks with no listed rows write zeros
-// ring slot of a per-step projection kernel: `s`, or, inside a captured step
-// (one graph serves every slot), the value a device counter holds when the
-// kernel runs; the counter advances after the step's last projection kernel
-struct RingSlot {
-  const int32_t* d;
-  int32_t s;
-  __device__ int64_t get() const { return d ? (int64_t)*d : (int64_t)s; }
-};
-
-static RingSlot ring_slot(const Ctx* c, int slot) {
-  return RingSlot{c->graph_slot_dev ? c->d_slot : nullptr, slot};
-}
-
+// ring slot of a captured step (one graph per psi buffer serves every slot):
+// the step for buffer q reads d_slot[q], and its update writes the next slot
+// to d_slot[1 - q], which the step after it reads
+// ---------------------------------------------------------------------------
 __global__ void k_slot_set(int32_t* d, int32_t v) {
   if (threadIdx.x == 0 && blockIdx.x == 0) *d = v;
 }
 
-__global__ void k_slot_next(int32_t* d) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) *d = *d + 1;
-}
-
-hipError_t launch_slot_set(Ctx* c, int v, hipStream_t st) {
-  hipLaunchKernelGGL(k_slot_set, dim3(1), dim3(64), 0, st, c->d_slot, v);
+hipError_t launch_slot_set(Ctx* c, int q, int v) {
+  hipLaunchKernelGGL(k_slot_set, dim3(1), dim3(64), 0, c->stream, c->d_slot + q, v);
   return hipGetLastError();
 }
 
-hipError_t launch_slot_next(Ctx* c, hipStream_t st) {
-  hipLaunchKernelGGL(k_slot_next, dim3(1), dim3(64), 0, st, c->d_slot);
-  return hipGetLastError();
-}
-
-__global__ __launch_bounds__(64) void k_update_flux(const double* __restrict__ upart,
-                                                    const int32_t* __restrict__ gfirst,
-                                                    const int32_t* __restrict__ fmap,
-                                                    double* __restrict__ zr_ring,
-                                                    double* __restrict__ zdr_ring, int n2,
-                                                    int64_t nflux, RingSlot rs) {
-  const int64_t slot = rs.get();
-  double* __restrict__ zr = zr_ring + slot * nflux;
-  double* __restrict__ zdr = zdr_ring + 2 * slot * nflux;
-  const int g = blockIdx.x, lane = threadIdx.x;
-  const int nrc = (n2 + 63) / 64;
-  const int rc = g % nrc, cia = g / nrc;
-  const int R = rc * 64 + lane;
-  if (R >= n2) return;
-  double re = 0.0, im = 0.0, zv = 0.0;
-  const int i0 = gfirst[g], i1 = gfirst[g + 1];
-#pragma unroll 4
-  for (int it = i0; it < i1; it++) {
-    const double* up = upart + (int64_t)it * 3 * 64;
-    re += up[lane];
-    im += up[64 + lane];
-    zv += up[128 + lane];
-  }
-  const int f = fmap[(int64_t)cia * n2 + R];
-  if (f >= 0) {
-    zdr[2 * (int64_t)f] = re;
-    zdr[2 * (int64_t)f + 1] = im;
-    zr[f] = zv;
-  }
-}
-
-template <typename T, int MODE, bool SINGLE, bool PROJ, bool AUTO, bool PRODP = false,
-          bool CPL4 = false>
-static void launch_update_kernel(Ctx* c, unsigned nb, const double* psi, double* out,
-                                 const UpdArgs& a) {
-  hipLaunchKernelGGL((k_update<T, T, MODE, SINGLE, PROJ, AUTO, PRODP, CPL4>), dim3(nb), dim3(256), 0,
-                     c->stream, psi, out, (const T*)c->d_t2, (const T*)c->d_ang,
-                     (const T*)c->d_v, a);
-}
-
-// prodp (product projection) runs with the projection variant (PROJ) only
-template <typename T, bool SINGLE, bool CPL4>
-static void dispatch_update(Ctx* c, unsigned nb, const double* psi, double* out, const UpdArgs& a,
-                            bool proj, bool autoc, bool prodp) {
-  if (a.mode == 0)
-    launch_update_kernel<T, 0, SINGLE, false, false, false, CPL4>(c, nb, psi, out, a);
-  else if (a.mode == 1)
-    autoc ? launch_update_kernel<T, 1, SINGLE, false, true, false, CPL4>(c, nb, psi, out, a)
-          : launch_update_kernel<T, 1, SINGLE, false, false, false, CPL4>(c, nb, psi, out, a);
-  else if (prodp)
-    autoc ? launch_update_kernel<T, 2, SINGLE, true, true, true, CPL4>(c, nb, psi, out, a)
-          : launch_update_kernel<T, 2, SINGLE, true, false, true, CPL4>(c, nb, psi, out, a);
-  else if (proj)
-    autoc ? launch_update_kernel<T, 2, SINGLE, true, true, false, CPL4>(c, nb, psi, out, a)
-          : launch_update_kernel<T, 2, SINGLE, true, false, false, CPL4>(c, nb, psi, out, a);
-  else
-    autoc ? launch_update_kernel<T, 2, SINGLE, false, true, false, CPL4>(c, nb, psi, out, a)
-          : launch_update_kernel<T, 2, SINGLE, false, false, false, CPL4>(c, nb, psi, out, a);
-}
-
-__global__ void k_reduce_parts(const double* __restrict__ part, int nb,
-                               double* __restrict__ out_ring, RingSlot rs) {
-  double* __restrict__ out = out_ring + 2 * (int64_t)rs.get();
-  __shared__ double sh[2][256];
-  // four independent partial sums per thread, so that four loads are in
-  // flight at a time instead of one
+// ---------------------------------------------------------------------------
+// sums over a ring of steps that the update leaves per block, per reactant
+// slice and per channel.  They run once per ring, one block (or grid row) per
+// step, instead of as small kernels after every update.
+// ---------------------------------------------------------------------------
+// (norm, autocorrelation) of step blockIdx.x from the update's block sums
+__global__ __launch_bounds__(256) void k_norm_ring(const double* __restrict__ part_ring, int nb,
+                                                   double* __restrict__ out_ring) {
   typedef double d2 __attribute__((ext_vector_type(2)));
-  const d2* p2 = (const d2*)part;
-  d2 s0 = {0, 0}, s1 = {0, 0}, s2 = {0, 0}, s3 = {0, 0};
+  const d2* p2 = (const d2*)part_ring + (int64_t)blockIdx.x * nb;
+  double* __restrict__ out = out_ring + 2 * (int64_t)blockIdx.x;
+  __shared__ double sh[2][256];
+  d2 s0 = {0, 0}, s1 = {0, 0};
   int i = threadIdx.x;
-  for (; i + 3 * (int)blockDim.x < nb; i += 4 * blockDim.x) {
+  for (; i + (int)blockDim.x < nb; i += 2 * blockDim.x) {  // two loads in flight
     s0 += p2[i];
     s1 += p2[i + blockDim.x];
-    s2 += p2[i + 2 * blockDim.x];
-    s3 += p2[i + 3 * blockDim.x];
   }
-  for (; i < nb; i += blockDim.x) s0 += p2[i];
-  const d2 st = (s0 + s1) + (s2 + s3);
-  double a = st.x, b = st.y;
-  sh[0][threadIdx.x] = a;
-  sh[1][threadIdx.x] = b;
+  if (i < nb) s0 += p2[i];
+  const d2 st = s0 + s1;
+  sh[0][threadIdx.x] = st.x;
+  sh[1][threadIdx.x] = st.y;
   __syncthreads();
   for (int w = 128; w > 0; w >>= 1) {
     if (threadIdx.x < w) {
@@ -961,61 +655,86 @@ __global__ void k_reduce_parts(const double* __restrict__ part, int nb,
   }
 }
 
-// ---------------------------------------------------------------------------
-// per-step projections into the ring.  The flux line (every (c, ia, R)
-// column: zdR = sum_r zAR1flux(r) psi(c,ia,r,R), the full-state derivative of
-// totalflux_k, SRC/mod_flux_01y2.f:598-609, and zR = psi at r = ir1flux(ia),
-// stored at flux points f = fmap(c,ia,R) >= 0) and the reactant slice at
-// R = ir2abs are taken inside k_update.
-// ---------------------------------------------------------------------------
-// Cvj(c, j, v) = sum_r fd(r, v, j) sum_ia slice(c, ia, r) D(ia, j); block per (c, jj)
-// (Cvjflux_k, SRC/mod_flux_01y2.f:672-702; slice = psi at R = ir2abs / sqrt(ah2)).
-// 16 waves: the angle sum is split over the waves (lanes over r), then each
-// wave takes some of the v sums.
-constexpr int CVJ_WAVES = 16;
-__global__ __launch_bounds__(64 * CVJ_WAVES) void k_cvj(const double* __restrict__ slice,
-                                                        const double* __restrict__ dcvj,
-                                                        const double* __restrict__ fdv,
-                                                        double* __restrict__ cvj_ring, int nj,
-                                                        int nv, int na, int n1, int64_t ncvj,
-                                                        RingSlot rs) {
-  double* __restrict__ cvj = cvj_ring + (int64_t)rs.get() * ncvj;
-  const int c = blockIdx.x / nj, jj = blockIdx.x % nj;
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  extern __shared__ double xj[];  // [n1]
-  __shared__ double part[CVJ_WAVES][64];
-  const double* dj = dcvj + ((int64_t)c * nj + jj) * na;
-  const double* sl = slice + (int64_t)c * na * n1;
-  for (int r0 = 0; r0 < n1; r0 += 64) {
-    const int r = r0 + lane;
-    double s = 0, s1 = 0;
-    if (r < n1) {
-      int ia = wv;
-      for (; ia + CVJ_WAVES < na; ia += 2 * CVJ_WAVES) {  // two loads in flight
-        s += sl[(int64_t)ia * n1 + r] * dj[ia];
-        s1 += sl[(int64_t)(ia + CVJ_WAVES) * n1 + r] * dj[ia + CVJ_WAVES];
-      }
-      if (ia < na) s += sl[(int64_t)ia * n1 + r] * dj[ia];
-      s += s1;
-    }
-    part[wv][lane] = s;
-    __syncthreads();
-    if (wv == 0 && r < n1) {
-      double t = 0;
-      for (int q = 0; q < CVJ_WAVES; q++) t += part[q][lane];
-      xj[r] = t;
-    }
-    __syncthreads();
+// flux samples of step blockIdx.y: the sums over r that the update left per
+// segment, added over the segments of the point's strip
+__global__ __launch_bounds__(256) void k_flux_ring(const double* __restrict__ upart,
+                                                   const int32_t* __restrict__ sfirst,
+                                                   const uint32_t* __restrict__ col,
+                                                   double* __restrict__ zr,
+                                                   double* __restrict__ zdr, int64_t nflux,
+                                                   int nseg, int n2, int64_t plane, int ns,
+                                                   int sw) {
+  const int64_t f = (int64_t)blockIdx.x * blockDim.x + threadIdx.x, slot = blockIdx.y;
+  if (f >= nflux) return;
+  const int64_t cia = col[f] / plane;
+  const int R = col[f] % n2, s = R / sw, x = R - s * sw;
+  double re = 0.0, im = 0.0, zv = 0.0;
+  for (int k = sfirst[cia * ns + s]; k < sfirst[cia * ns + s + 1]; k++) {
+    const double* up = upart + ((slot * nseg + k) * 4) * sw + x;
+    re += up[0];
+    im += up[sw];
+    zv += up[2 * sw];
   }
-  for (int v = wv; v < nv; v += CVJ_WAVES) {
-    const double* f = fdv + (((int64_t)c * nj + jj) * nv + v) * n1;
+  zdr[2 * (slot * nflux + f)] = re;
+  zdr[2 * (slot * nflux + f) + 1] = im;
+  zr[slot * nflux + f] = zv;
+}
+
+// Cvj(c, j, v) = sum_r fd(r, v, j) sum_ia slice(c, ia, r) D(ia, j) of step
+// blockIdx.y (Cvjflux_k, SRC/mod_flux_01y2.f:672-702; slice = psi at
+// R = ir2abs / sqrt(ah2)).  Block = (channel, jb <= CVJ_J values of j), a
+// thread per r: each slice value is read once for the jb angular sums.
+constexpr int CVJ_J = 8;
+__global__ __launch_bounds__(256) void k_cvj_ring(const double* __restrict__ slice_ring,
+                                                  const double* __restrict__ dcvj,
+                                                  const double* __restrict__ fdv,
+                                                  double* __restrict__ cvj_ring, int nc, int nj,
+                                                  int nv, int na, int n1, int jb, int64_t ncvj) {
+  const int njb = (nj + jb - 1) / jb;
+  const int c = blockIdx.x / njb, j0 = (blockIdx.x - c * njb) * jb;
+  const int64_t slot = blockIdx.y;
+  const double* __restrict__ sl = slice_ring + (slot * nc + c) * (int64_t)na * n1;
+  double* __restrict__ cvj = cvj_ring + slot * ncvj + ((int64_t)c * nj + j0) * nv;
+  extern __shared__ double xj[];  // [jb][n1]
+  const double* dj[CVJ_J];
+#pragma unroll
+  for (int q = 0; q < CVJ_J; q++)
+    dj[q] = dcvj + ((int64_t)c * nj + (j0 + q < nj ? j0 + q : nj - 1)) * na;
+  for (int r = threadIdx.x; r < n1; r += blockDim.x) {
+    double s[CVJ_J] = {};
+    int ia = 0;
+    for (; ia + 4 <= na; ia += 4) {  // four loads in flight
+      double x[4];
+#pragma unroll
+      for (int u = 0; u < 4; u++) x[u] = sl[(int64_t)(ia + u) * n1 + r];
+#pragma unroll
+      for (int u = 0; u < 4; u++)
+#pragma unroll
+        for (int q = 0; q < CVJ_J; q++) s[q] += x[u] * dj[q][ia + u];
+    }
+    for (; ia < na; ia++) {
+      const double x = sl[(int64_t)ia * n1 + r];
+#pragma unroll
+      for (int q = 0; q < CVJ_J; q++) s[q] += x * dj[q][ia];
+    }
+#pragma unroll
+    for (int q = 0; q < CVJ_J; q++)
+      if (q < jb) xj[q * n1 + r] = s[q];
+  }
+  __syncthreads();
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int nq = (j0 + jb < nj ? jb : nj - j0) * nv;
+  for (int k = wv; k < nq; k += 4) {
+    const int q = k / nv, v = k - q * nv;
+    const double* f = fdv + (((int64_t)c * nj + j0 + q) * nv + v) * n1;
     double s = 0;
-    for (int r = lane; r < n1; r += 64) s += xj[r] * f[r];
+    for (int r = lane; r < n1; r += 64) s += xj[q * n1 + r] * f[r];
     for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off);
-    if (lane == 0) cvj[((int64_t)c * nj + jj) * nv + v] = s;
+    if (lane == 0) cvj[k] = s;
   }
 }
 
+// ---------------------------------------------------------------------------
 // ---------------------------------------------------------------------------
 // energy accumulation over a ring of steps k0 .. k0+ns-1
 //   acc[x][E] += sum_s C_{k0+s}(E) z[s][x],  C_k(E) = 2 hbr/delta e^{-i k acos Es}/sqrt(1-Es^2)
@@ -2420,256 +2139,22 @@ static hipError_t ang_fused_setup(Ctx* c, int nt) {
 }
 
 // ---------------------------------------------------------------------------
-// First and last passes of the radial correction over R, for n2 = 32 HB with
-// HB in {8, 10, 12, 16}, on work items of 16 rows r < nn1(ia) of one
-// (channel, angle): int4 {channel * na + angle, row tile, nn1, k2lo}.
-// With h = n2 / 2 and S(n2-1-R, k) = (-1)^k S(R, k):
-//   k_rad_fwd: t1[r][k2] = sum_R S(R, k2) psi[r][R] for k2 < k2lo(ia), as
+// First and last passes of the radial correction over R, R products first (FP32
+// operator terms, and FP64 where the low r modes do not fit the update's
+// tiles), for n2 = 32 HB with HB in {8, 10, 12, 16}, on work items of 16 rows
+// r < nn1(ia) of one (channel, angle): int4 {channel * na + angle, row tile,
+// nn1, k2lo | active pairs << 16}.  With h = n2 / 2 and
+// S(n2-1-R, k) = (-1)^k S(R, k):
+//   forward: t1[r][k2] = sum_R S(R, k2) psi[r][R] for k2 < k2lo(ia), as
 //     even k2: sum_{j<h} (psi[j] + psi[n2-1-j]) S(j, k2)
 //     odd  k2: sum_{j<h} (psi[j] - psi[n2-1-j]) S(j, k2);
-//   k_rad_inv: corr[r][R] = E + O and corr[r][n2-1-R] = E - O for R < h,
+//   inverse: corr[r][R] = E + O and corr[r][n2-1-R] = E - O for R < h,
 //     E / O the sums of t1[r][k2] S(R, k2) over even / odd k2 < k2lo(ia)
 //     (half the MFMAs of the unfolded product, every output written once).
-// Both are persistent: each wave keeps its slice of the sine table in
-// registers for the whole launch (the forward pass: one 16-wide k2 tile of
-// one parity, all j; the inverse pass: one pair of 16-wide R tiles, all
-// k2), and the block walks the work items with the item's 16-row tile staged
-// in LDS (the forward pass stages it folded, psi[j] +- psi[n2-1-j]); the
-// next items' tiles load into registers during the MFMAs.
 // MFMA k index of lane group g at step s: j = 16 kb + 4 g + s (forward) and
 // k2 = 32 kb + 8 g + 2 s + parity (inverse), so a lane's operands for four
 // steps are one 16-byte read.
 // ---------------------------------------------------------------------------
-template <typename T>
-struct RadPad;  // LDS row padding (elements): rows start 4 banks apart
-template <>
-struct RadPad<float> {
-  static constexpr int v = 4;
-};
-template <>
-struct RadPad<double> {
-  static constexpr int v = 2;
-};
-
-// waves of k_rad_fwd per (parity, k' tile): two in FP32 when HB is a
-// multiple of 4, each over half the j range (the block then has 12 waves for
-// three k' tiles, three per SIMD); one otherwise, and in FP64, whose table
-// slice leaves no room for more waves
-template <typename T, int HB>
-struct RadSplit {
-  static constexpr int v = sizeof(T) == 4 && HB % 4 == 0 ? 2 : 1;
-};
-
-// work items per block of k_rad_fwd / k_rad_inv (the grid is raised to keep
-// each block's list within it)
-constexpr int kRadMaxItems = 256;
-
-// items of k_rad_fwd whose loads are in flight while a wave multiplies: two
-// in FP32; one in FP64, whose registers hold no second set
-template <typename T>
-struct RadDepth {
-  static constexpr int v = sizeof(T) == 4 ? 2 : 1;
-};
-
-template <typename T, int NKB, int HB, bool FULL>
-__global__ __launch_bounds__(128 * NKB * (RadSplit<T, HB>::v)) void k_rad_fwd(
-    const T* __restrict__ psi, const T* __restrict__ Tt, T* __restrict__ t1,
-    const int4* __restrict__ items, int nitems, int n1) {
-  typedef MfmaAcc<T> M;
-  typedef typename M::V V;
-  constexpr int KS = RadSplit<T, HB>::v, HBW = HB / KS;  // j blocks per wave (even)
-  constexpr int N2 = 32 * HB, H = N2 / 2, NT = 128 * NKB * KS;  // threads
-  constexpr int LP = H + RadPad<T>::v;
-  // the tile is staged folded: fold[0][row][j] = psi[j] + psi[n2-1-j] and
-  // fold[1][row][j] = psi[j] - psi[n2-1-j], j < h; a thread loads the
-  // vectors at j and at its mirror and folds them as it stores
-  constexpr int NP = 16 * H / 4, PER = (NP + NT - 1) / NT;
-  __shared__ __align__(16) T fold[2][2][16 * LP];  // [buffer][parity]
-  // partial tiles of both j halves, by buffer (KS = 2)
-  __shared__ V red[KS == 2 ? 2 : 1][KS == 2 ? 2 : 1][KS == 2 ? 2 * NKB : 1][64];
-  const int lane = threadIdx.x & 63, g = lane >> 4, i = lane & 15, wave = threadIdx.x >> 6;
-  const int kh = wave / (2 * NKB), w2 = wave - kh * 2 * NKB;  // j half, tile index
-  const int p = w2 / NKB, t = w2 - p * NKB;  // parity and k' tile of this wave
-  const int64_t plane = (int64_t)n1 * N2;
-  // b[kb][s] = S(16 (kh HBW + kb) + 4 g + s, 2 (16 t + i) + p) over this
-  // wave's j blocks
-  T b[HBW][4];
-  {
-    const T* trow = Tt + (int64_t)(2 * (16 * t + i) + p) * H + 16 * kh * HBW + 4 * g;
-#pragma unroll
-    for (int kb = 0; kb < HBW; kb++) ld4(trow + 16 * kb, b[kb]);
-  }
-  auto fetch = [&](const int4& it, T(&pf)[PER][2][4]) {
-#pragma unroll
-    for (int l = 0; l < PER; l++) {
-      int v = threadIdx.x + NT * l;
-      v = v < NP ? v : NP - 1;  // spare threads repeat the last pair
-      const int row = v / (H / 4), c4 = v - row * (H / 4);
-      int r = 16 * it.y + row;
-      r = r < it.z ? r : it.z - 1;
-      const T* src = psi + it.x * plane + (int64_t)r * N2;
-      ld4(src + 4 * c4, pf[l][0]);               // psi[j .. j+3], j = 4 c4
-      ld4(src + (N2 - 4 - 4 * c4), pf[l][1]);    // psi[n2-4-j .. n2-1-j]
-    }
-  };
-  auto put = [&](const T(&pf)[PER][2][4], int buf) {
-#pragma unroll
-    for (int l = 0; l < PER; l++) {
-      int v = threadIdx.x + NT * l;
-      v = v < NP ? v : NP - 1;
-      const int row = v / (H / 4), c4 = v - row * (H / 4);
-      T e[4], o[4];
-#pragma unroll
-      for (int q = 0; q < 4; q++) {
-        e[q] = pf[l][0][q] + pf[l][1][3 - q];
-        o[q] = pf[l][0][q] - pf[l][1][3 - q];
-      }
-      st4(&fold[buf][0][row * LP + 4 * c4], e);
-      st4(&fold[buf][1][row * LP + 4 * c4], o);
-    }
-  };
-  auto mult = [&](int buf) {
-    // two accumulator chains (even and odd j blocks), summed at the end;
-    // the operands of the next pair of j blocks are read from LDS before the
-    // MFMAs of this pair are issued (the scheduling barrier keeps that
-    // order), so the LDS latency hides behind the matrix work
-    V acc0 = (V){0, 0, 0, 0}, acc1 = (V){0, 0, 0, 0};
-    const T* frow = &fold[buf][p][i * LP + 16 * kh * HBW + 4 * g];
-    T x[2][2][4];
-    ld4(frow, x[0][0]);
-    ld4(frow + 16, x[0][1]);
-#pragma unroll
-    for (int kb = 0; kb < HBW; kb += 2) {
-      const int c = (kb >> 1) & 1;
-      if (kb + 2 < HBW) {
-        ld4(frow + 16 * (kb + 2), x[c ^ 1][0]);
-        ld4(frow + 16 * (kb + 3), x[c ^ 1][1]);
-      }
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int s = 0; s < 4; s++) {
-        acc0 = M::mma(x[c][0][s], b[kb][s], acc0);
-        acc1 = M::mma(x[c][1][s], b[kb + 1][s], acc1);
-      }
-    }
-    V acc;
-#pragma unroll
-    for (int rr = 0; rr < 4; rr++) acc[rr] = acc0[rr] + acc1[rr];
-    return acc;
-  };
-  // With FULL (n1 a multiple of 16) every lane stores, with no branch:
-  // rows nn1 .. 16 ceil(nn1 / 16) - 1 (< n1) and columns k2lo .. 32 NKB - 1
-  // then hold finite values that no later pass uses (the r-pass tables are
-  // zero on those rows, the r-pass factor (radcut - E)_+ is zero on those
-  // columns and the inverse pass reads them as zero).  Otherwise rows past
-  // n1 are not stored.  With KS = 2 the two halves' tiles meet in LDS (left
-  // there by the previous item) and each half stores two of a lane's four
-  // rows: every wave runs the same stores, so no branch leaves the compiler
-  // unsure how many stores are in flight when it waits for the next loads.
-  auto store = [&](const V& acc, const int4& it, int buf) {
-    T* orow = t1 + it.x * plane;
-    const int k2 = 2 * (16 * t + i) + p;
-    if constexpr (KS == 2) {
-      const V o = red[buf][kh ^ 1][w2][lane];
-      const T v0 = kh ? acc[2] + o[2] : acc[0] + o[0];
-      const T v1 = kh ? acc[3] + o[3] : acc[1] + o[1];
-      const int r0 = 16 * it.y + M::row(lane, 2 * kh), r1 = 16 * it.y + M::row(lane, 2 * kh + 1);
-      if (FULL || r0 < n1) orow[(int64_t)r0 * N2 + k2] = v0;
-      if (FULL || r1 < n1) orow[(int64_t)r1 * N2 + k2] = v1;
-    } else {
-#pragma unroll
-      for (int rr = 0; rr < 4; rr++) {
-        const int row = 16 * it.y + M::row(lane, rr);
-        if (FULL || row < n1) orow[(int64_t)row * N2 + k2] = acc[rr];
-      }
-    }
-  };
-  auto keep = [&](const V& acc, int buf) {  // this half's partial tile
-    if constexpr (KS == 2) red[buf][kh][w2][lane] = acc;
-  };
-  const int G = (int)gridDim.x;
-  if ((int)blockIdx.x >= nitems) return;  // block-uniform
-  // this block's items blockIdx.x + k G, k < K, copied to LDS once: read
-  // from there they cost an in-order LDS read, where a scalar load would make
-  // every later LDS wait a full one
-  __shared__ int4 its[kRadMaxItems];
-  const int K = (nitems - 1 - (int)blockIdx.x) / G + 1;  // <= kRadMaxItems (host)
-  for (int k = threadIdx.x; k < K; k += NT) its[k] = items[blockIdx.x + k * G];
-  __syncthreads();
-  auto at = [&](int k) { return its[k < K ? k : K - 1]; };
-  // Two LDS buffers, one barrier per item: while a wave multiplies item k
-  // out of one buffer it has stored item k + 1 (loaded into registers during
-  // an earlier item) into the other and issued the loads of a later item.
-  // The barrier at the end of an item frees its buffer and completes the
-  // other (and the partial tiles of that item).  Each item's results are
-  // stored at the start of the next one, before the tile is staged: the wait
-  // for the staged loads then leaves those stores in flight.  A prefetch past
-  // the last item re-reads the last item, unused; the scheduling barriers
-  // keep this order of issue.
-  if constexpr (RadDepth<T>::v == 2) {
-    // two register sets: the loads of item k are issued two items before its
-    // tile is staged, so two items' loads are in flight while a wave
-    // multiplies (the loop is unrolled by two so that each set has fixed
-    // registers)
-    T pa[PER][2][4], pb[PER][2][4];
-    fetch(at(0), pa);
-    put(pa, 0);
-    fetch(at(1), pa);
-    fetch(at(2), pb);
-    __syncthreads();
-    put(pa, 1);
-    fetch(at(3), pa);
-    __builtin_amdgcn_sched_barrier(0);
-    V acc = mult(0);
-    keep(acc, 0);
-    __syncthreads();
-    // item k is staged in buffer b; p holds item k + 1
-    auto body = [&](T(&p)[PER][2][4], int k, int b) {
-      store(acc, at(k - 1), b ^ 1);
-      __builtin_amdgcn_sched_barrier(0);
-      put(p, b ^ 1);
-      fetch(at(k + 3), p);
-      __builtin_amdgcn_sched_barrier(0);
-      acc = mult(b);
-      keep(acc, b);
-      __syncthreads();
-    };
-    int k = 1, last = 0;  // last: buffer of the last item multiplied
-    while (k < K) {
-      body(pb, k, 1);
-      last = 1;
-      if (++k >= K) break;
-      body(pa, k, 0);
-      last = 0;
-      ++k;
-    }
-    store(acc, at(k - 1), last);
-  } else {
-    T pf[PER][2][4];
-    fetch(at(0), pf);
-    put(pf, 0);
-    fetch(at(1), pf);
-    __syncthreads();
-    put(pf, 1);
-    fetch(at(2), pf);
-    __builtin_amdgcn_sched_barrier(0);
-    V acc = mult(0);
-    keep(acc, 0);
-    __syncthreads();
-    int k = 1, buf = 1;
-    for (; k < K; k++, buf ^= 1) {
-      store(acc, at(k - 1), buf ^ 1);
-      __builtin_amdgcn_sched_barrier(0);
-      put(pf, buf ^ 1);
-      fetch(at(k + 2), pf);
-      __builtin_amdgcn_sched_barrier(0);
-      acc = mult(buf);
-      keep(acc, buf);
-      __syncthreads();
-    }
-    store(acc, at(k - 1), buf ^ 1);
-  }
-}
 
 // ---------------------------------------------------------------------------
 // The forward R pass in FP32 with the sine table in LDS: the same sums as
@@ -3300,135 +2785,6 @@ __global__ __launch_bounds__(64 * kRadLds64Waves) void k_rad_inv_lds64(
   }
 }
 
-template <typename T, int NKB, int HB, bool FULL>
-__global__ __launch_bounds__(32 * HB) void k_rad_inv(const T* __restrict__ t1,
-                                                     const T* __restrict__ Ti,
-                                                     T* __restrict__ corr,
-                                                     const int4* __restrict__ items, int nitems,
-                                                     int n1) {
-  typedef MfmaAcc<T> M;
-  typedef typename M::V V;
-  constexpr int N2 = 32 * HB, NT = 32 * HB;  // one wave per pair of R tiles of the first half
-  constexpr int K2P = 32 * NKB, LP = K2P + RadPad<T>::v;
-  constexpr int NV4 = 16 * K2P / 4, PER = (NV4 + NT - 1) / NT;
-  __shared__ __align__(16) T tile[2][16 * LP];
-  const int lane = threadIdx.x & 63, g = lane >> 4, i = lane & 15, pair = threadIdx.x >> 6;
-  const int64_t plane = (int64_t)n1 * N2;
-  // b[q][kb][e] = S(R, 32 kb + 8 g + e), R = 16 (2 pair + q) + i
-  T b[2][NKB][2][4];
-#pragma unroll
-  for (int q = 0; q < 2; q++) {
-    const T* trow = Ti + (int64_t)(16 * (2 * pair + q) + i) * K2P + 8 * g;
-#pragma unroll
-    for (int kb = 0; kb < NKB; kb++) {
-      ld4(trow + 32 * kb, b[q][kb][0]);
-      ld4(trow + 32 * kb + 4, b[q][kb][1]);
-    }
-  }
-  T pf[PER][4];
-  auto fetch = [&](const int4& it) {
-#pragma unroll
-    for (int l = 0; l < PER; l++) {
-      int v = threadIdx.x + NT * l;
-      v = v < NV4 ? v : NV4 - 1;
-      const int row = v / (K2P / 4), c4 = v - row * (K2P / 4);
-      int r = 16 * it.y + row;
-      r = r < it.z ? r : it.z - 1;
-      ld4(t1 + it.x * plane + (int64_t)r * N2 + 4 * c4, pf[l]);
-    }
-  };
-  auto put = [&](const int4& it, int buf) {  // columns k2 >= k2lo enter as zero
-#pragma unroll
-    for (int l = 0; l < PER; l++) {
-      int v = threadIdx.x + NT * l;
-      v = v < NV4 ? v : NV4 - 1;
-      const int row = v / (K2P / 4), c4 = v - row * (K2P / 4);
-#pragma unroll
-      for (int e = 0; e < 4; e++)
-        if (4 * c4 + e >= (it.w & 0xffff)) pf[l][e] = 0;
-      st4(&tile[buf][row * LP + 4 * c4], pf[l]);
-    }
-  };
-  // pairs whose 16 rows hold no compressed-grid point in their columns or
-  // the mirrored ones: the update reads none of their output
-  auto active = [&](const int4& it) { return (it.w >> (16 + pair)) & 1; };
-  V E[2], O[2];
-  auto mult = [&](int buf) {
-    T a[NKB][2][4];
-#pragma unroll
-    for (int kb = 0; kb < NKB; kb++) {
-      ld4(&tile[buf][i * LP + 32 * kb + 8 * g], a[kb][0]);
-      ld4(&tile[buf][i * LP + 32 * kb + 8 * g + 4], a[kb][1]);
-    }
-#pragma unroll
-    for (int q = 0; q < 2; q++) {
-      E[q] = (V){0, 0, 0, 0};
-      O[q] = (V){0, 0, 0, 0};
-#pragma unroll
-      for (int kb = 0; kb < NKB; kb++)
-#pragma unroll
-        for (int s = 0; s < 4; s++) {
-          const int e0 = 2 * s, e1 = 2 * s + 1;
-          E[q] = M::mma(a[kb][e0 >> 2][e0 & 3], b[q][kb][e0 >> 2][e0 & 3], E[q]);
-          O[q] = M::mma(a[kb][e1 >> 2][e1 & 3], b[q][kb][e1 >> 2][e1 & 3], O[q]);
-        }
-    }
-  };
-  // With FULL (n1 a multiple of 16) rows nn1 .. 16 ceil(nn1 / 16) - 1 are
-  // stored too (below n1; the update reads no row past nn1), with no
-  // per-lane branch; otherwise rows past nn1 are not stored.
-  auto store = [&](const int4& it) {
-    T* ob = corr + it.x * plane;
-#pragma unroll
-    for (int q = 0; q < 2; q++) {
-      const int R = 16 * (2 * pair + q) + i;
-#pragma unroll
-      for (int rr = 0; rr < 4; rr++) {
-        const int row = 16 * it.y + M::row(lane, rr);
-        if (FULL || row < it.z) {
-          ob[(int64_t)row * N2 + R] = E[q][rr] + O[q][rr];
-          ob[(int64_t)row * N2 + (N2 - 1 - R)] = E[q][rr] - O[q][rr];
-        }
-      }
-    }
-  };
-  const int G = (int)gridDim.x;
-  if ((int)blockIdx.x >= nitems) return;  // block-uniform
-  // this block's items in LDS, as in k_rad_fwd
-  __shared__ int4 its[kRadMaxItems];
-  const int K = (nitems - 1 - (int)blockIdx.x) / G + 1;  // <= kRadMaxItems (host)
-  for (int k = threadIdx.x; k < K; k += NT) its[k] = items[blockIdx.x + k * G];
-  __syncthreads();
-  auto at = [&](int k) { return its[k < K ? k : K - 1]; };
-  // Two LDS buffers, one barrier per item, as in k_rad_fwd: item k is
-  // multiplied out of one buffer after item k + 1 has been staged into the
-  // other and the loads of item k + 2 issued; its results are stored at the
-  // start of the next item, after the staging.  A prefetch past the last
-  // item re-reads the last item, unused.
-  int4 cur = at(0);
-  fetch(cur);
-  put(cur, 0);
-  int4 nxt = at(1);
-  fetch(nxt);
-  __syncthreads();
-  int4 prev = cur;
-  bool have = false;  // results of prev in E, O
-  for (int k = 0, buf = 0; k < K; k++, buf ^= 1) {
-    put(nxt, buf ^ 1);
-    if (have && active(prev)) store(prev);
-    const int4 nn = at(k + 2);
-    fetch(nn);
-    __builtin_amdgcn_sched_barrier(0);  // issue the loads before the MFMAs
-    if (active(cur)) mult(buf);
-    have = true;
-    __syncthreads();
-    prev = cur;
-    cur = nxt;
-    nxt = nn;
-  }
-  if (active(prev)) store(prev);
-}
-
 // ---------------------------------------------------------------------------
 // The two r passes of the radial correction in one kernel, one block of four
 // waves per work item = (channel-angle, 16 columns k2 of the low R modes):
@@ -3800,120 +3156,35 @@ static hipError_t build_rad_mid(Ctx* c) {
   return hipSuccess;
 }
 
-template <typename K>
-static hipError_t persistent_grid(K kernel, int threads, int* blocks) {
-  int nb = 0, dev = 0, ncu = 0;
-  hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, kernel, threads, 0);
-  if (e != hipSuccess) return e;
-  if ((e = hipGetDevice(&dev)) != hipSuccess) return e;
-  if ((e = hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev)) != hipSuccess)
-    return e;
-  *blocks = (nb > 0 ? nb : 1) * ncu;
-  return hipSuccess;
-}
-
-// launch (or, with setup, size the grids of) the R passes for NKB, HB
+// launch the R passes for NKB, HB
 template <typename T, int NKB, int HB>
 static hipError_t rad_nkb_hb(Ctx* c, const T* psi, T* t1, T* corr, int mode) {
   const HostTables& t = c->t;
   const T* tab = (const T*)c->d_dst_tables;
   const int4* items = (const int4*)c->d_rad_items;
-  if (mode == 2) {
-    int dev = 0;
-    hipError_t e = hipGetDevice(&dev);
-    if (e == hipSuccess) e = hipDeviceGetAttribute(&c->rad_ncu, hipDeviceAttributeMultiprocessorCount, dev);
-    if (e != hipSuccess) return e;
-    // FP64 passes with the table split over block pairs (whole 16-block
-    // groups; the HB R tiles of the first half split in two)
-    c->rad_lds64 = sizeof(T) == 8 && c->rad_ncu >= 16 && HB % 2 == 0;
-    c->rad_inv_h = sizeof(T) == 4;
-    e = t.n1 % 16 == 0
-                       ? persistent_grid(k_rad_fwd<T, NKB, HB, true>, 128 * NKB * RadSplit<T, HB>::v,
-                                         &c->rad_grid[0])
-                       : persistent_grid(k_rad_fwd<T, NKB, HB, false>, 128 * NKB * RadSplit<T, HB>::v,
-                                         &c->rad_grid[0]);
-    if (e != hipSuccess) return e;
-    return t.n1 % 16 == 0 ? persistent_grid(k_rad_inv<T, NKB, HB, true>, 32 * HB, &c->rad_grid[1])
-                          : persistent_grid(k_rad_inv<T, NKB, HB, false>, 32 * HB, &c->rad_grid[1]);
-  }
   const int n = c->rad_nitems;
-  // the grid: the resident blocks divided by the grid option (each block
-  // loads its waves' table slices once, so fewer blocks read fewer table
-  // bytes and walk more items each)
-  const int gdiv = c->opt_rad_grid > 0 ? c->opt_rad_grid : 1;
-  const int gmin = (n + kRadMaxItems - 1) / kRadMaxItems;  // each block's list fits its LDS copy
-  const int g0 = std::max(std::max(c->rad_grid[0] / gdiv, 1), gmin);
-  const int g1 = std::max(std::max(c->rad_grid[1] / gdiv, 1), gmin);
-  if (mode == 0) {
-    if constexpr (sizeof(T) == 4) {  // the table in LDS, one block per CU
-      const int nb = std::max(1, std::min(c->rad_ncu, n));
-      if (t.n1 % 16 == 0)
-        hipLaunchKernelGGL((k_rad_fwd_lds<NKB, HB, true>), dim3(nb), dim3(64 * kFwdLdsWaves), 0,
-                           c->stream, psi, tab + t.rad_tt_off, t1, items, n, t.n1);
-      else
-        hipLaunchKernelGGL((k_rad_fwd_lds<NKB, HB, false>), dim3(nb), dim3(64 * kFwdLdsWaves), 0,
-                           c->stream, psi, tab + t.rad_tt_off, t1, items, n, t.n1);
-      return hipGetLastError();
-    }
-    if constexpr (sizeof(T) == 8) {
-      if (c->rad_lds64) {  // pairs of blocks split the table (16-block groups)
-        const int nb = c->rad_ncu / 16 * 16;
-        if (t.n1 % 16 == 0)
-          hipLaunchKernelGGL((k_rad_fwd_lds64<NKB, HB, true>), dim3(nb), dim3(64 * kRadLds64Waves),
-                             0, c->stream, psi, tab + t.rad_tt_off, t1, items, n, t.n1);
-        else
-          hipLaunchKernelGGL((k_rad_fwd_lds64<NKB, HB, false>), dim3(nb), dim3(64 * kRadLds64Waves),
-                             0, c->stream, psi, tab + t.rad_tt_off, t1, items, n, t.n1);
-        return hipGetLastError();
-      }
-    }
-    const int nt = 128 * NKB * RadSplit<T, HB>::v;
-    if (t.n1 % 16 == 0)
-      hipLaunchKernelGGL((k_rad_fwd<T, NKB, HB, true>), dim3(n < g0 ? n : g0), dim3(nt), 0,
-                         c->stream, psi, tab + t.rad_tt_off, t1, items, n, t.n1);
-    else
-      hipLaunchKernelGGL((k_rad_fwd<T, NKB, HB, false>), dim3(n < g0 ? n : g0), dim3(nt), 0,
-                         c->stream, psi, tab + t.rad_tt_off, t1, items, n, t.n1);
-  } else {
-    if constexpr (sizeof(T) == 4) {  // the table in LDS, one block per CU
-      const int nb = std::max(1, std::min(c->rad_ncu, n));
-      if (c->rad_inv_h && c->opt_fp16) {  // products on the FP16 matrix cores, compensated
-        if (t.n1 % 16 == 0)
-          hipLaunchKernelGGL((k_rad_inv_h<NKB, HB, true>), dim3(nb), dim3(64 * kInvLdsWaves), 0,
-                             c->stream, t1, tab + t.rad_ti_off, corr, items, n, t.n1);
-        else
-          hipLaunchKernelGGL((k_rad_inv_h<NKB, HB, false>), dim3(nb), dim3(64 * kInvLdsWaves), 0,
-                             c->stream, t1, tab + t.rad_ti_off, corr, items, n, t.n1);
-        return hipGetLastError();
-      }
-      if (t.n1 % 16 == 0)
-        hipLaunchKernelGGL((k_rad_inv_lds<NKB, HB, true>), dim3(nb), dim3(64 * kInvLdsWaves), 0,
-                           c->stream, t1, tab + t.rad_ti_off, corr, items, n, t.n1);
-      else
-        hipLaunchKernelGGL((k_rad_inv_lds<NKB, HB, false>), dim3(nb), dim3(64 * kInvLdsWaves), 0,
-                           c->stream, t1, tab + t.rad_ti_off, corr, items, n, t.n1);
-      return hipGetLastError();
-    }
-    if constexpr (sizeof(T) == 8) {
-      if (c->rad_lds64) {
-        const int nb = c->rad_ncu / 16 * 16;
-        if (t.n1 % 16 == 0)
-          hipLaunchKernelGGL((k_rad_inv_lds64<NKB, HB, true>), dim3(nb), dim3(64 * kRadLds64Waves),
-                             0, c->stream, t1, tab + t.rad_ti_off, corr, items, n, t.n1);
-        else
-          hipLaunchKernelGGL((k_rad_inv_lds64<NKB, HB, false>), dim3(nb), dim3(64 * kRadLds64Waves),
-                             0, c->stream, t1, tab + t.rad_ti_off, corr, items, n, t.n1);
-        return hipGetLastError();
-      }
-    }
-    if (t.n1 % 16 == 0)
-      hipLaunchKernelGGL((k_rad_inv<T, NKB, HB, true>), dim3(n < g1 ? n : g1), dim3(32 * HB), 0,
-                         c->stream, t1, tab + t.rad_ti_off, corr, items, n, t.n1);
-    else
-      hipLaunchKernelGGL((k_rad_inv<T, NKB, HB, false>), dim3(n < g1 ? n : g1), dim3(32 * HB), 0,
-                         c->stream, t1, tab + t.rad_ti_off, corr, items, n, t.n1);
+#define MW3_RAD(K, NB, NT, ...)                                                               \
+  do {                                                                                       \
+    if (t.n1 % 16 == 0)                                                                       \
+      hipLaunchKernelGGL((K<NKB, HB, true>), dim3(NB), dim3(NT), 0, c->stream, __VA_ARGS__,   \
+                         items, n, t.n1);                                                     \
+    else                                                                                     \
+      hipLaunchKernelGGL((K<NKB, HB, false>), dim3(NB), dim3(NT), 0, c->stream, __VA_ARGS__,  \
+                         items, n, t.n1);                                                     \
+    return hipGetLastError();                                                                 \
+  } while (0)
+  if constexpr (sizeof(T) == 4) {  // the table in LDS, one block per CU
+    const int nb = std::max(1, std::min(c->rad_ncu, n));
+    if (mode == 0) MW3_RAD(k_rad_fwd_lds, nb, 64 * kFwdLdsWaves, psi, tab + t.rad_tt_off, t1);
+    if (c->opt_fp16)  // products on the FP16 matrix cores, compensated
+      MW3_RAD(k_rad_inv_h, nb, 64 * kInvLdsWaves, t1, tab + t.rad_ti_off, corr);
+    MW3_RAD(k_rad_inv_lds, nb, 64 * kInvLdsWaves, t1, tab + t.rad_ti_off, corr);
+  } else {  // pairs of blocks split the table (16-block groups)
+    const int nb = c->rad_ncu / 16 * 16;
+    if (mode == 0) MW3_RAD(k_rad_fwd_lds64, nb, 64 * kRadLds64Waves, psi, tab + t.rad_tt_off, t1);
+    MW3_RAD(k_rad_inv_lds64, nb, 64 * kRadLds64Waves, t1, tab + t.rad_ti_off, corr);
   }
-  return hipGetLastError();
+#undef MW3_RAD
 }
 
 template <typename T, int NKB>
@@ -3927,8 +3198,7 @@ static hipError_t rad_nkb(Ctx* c, const T* psi, T* t1, T* corr, int mode) {
   }
 }
 
-// mode 0: forward R pass (psi -> t1); 1: inverse (t1 -> corr); 2: size the
-// persistent grids
+// mode 0: forward R pass (psi -> t1); 1: inverse (t1 -> corr)
 template <typename T>
 static hipError_t run_rad(Ctx* c, const T* psi, T* t1, T* corr, int mode) {
   switch (c->t.rad_nkb) {
@@ -3939,7 +3209,6 @@ static hipError_t run_rad(Ctx* c, const T* psi, T* t1, T* corr, int mode) {
     default: return hipErrorInvalidValue;
   }
 }
-
 
 // block order of each plan; every vectorised plan runs the 64 x 64 block tile
 // (2 x 2 waves of 2 x 2 MFMA tiles), which beat 128 x 64, 64 x 128 and
@@ -4116,11 +3385,23 @@ hipError_t build_plans(Ctx* c) {
     if ((e = upload_plan(&c->p_angB, d, true)) != hipSuccess) return e;
   }
   plan_tiles(c);
-  // the two r passes in one kernel where the low r modes fit its tiles
-  if ((e = build_rad_mid(c)) != hipSuccess) return e;
+  // strips, tiles and (FP64) radial tables of the update
+  e = c->precision == MW3_MIXED ? step_build_f32(c) : step_build_f64(c);
+  if (e != hipSuccess) return e;
+  // else the R products first: the two r passes in one kernel where the low r
+  // modes fit its tiles
+  if (!c->up_nk1 && (e = build_rad_mid(c)) != hipSuccess) return e;
   // R passes one wave per 16-row tile when their tables were built
   c->rad_nitems = 0;
-  if (t.rad_nkb > 0 && (t.n2 == 256 || t.n2 == 320 || t.n2 == 384 || t.n2 == 512)) {
+  {
+    int dev = 0;
+    if ((e = hipGetDevice(&dev)) != hipSuccess) return e;
+    if ((e = hipDeviceGetAttribute(&c->rad_ncu, hipDeviceAttributeMultiprocessorCount, dev)) !=
+        hipSuccess)
+      return e;
+  }
+  if (!c->up_nk1 && t.rad_nkb > 0 && (c->precision == MW3_MIXED || c->rad_ncu >= 16) &&
+      (t.n2 == 256 || t.n2 == 320 || t.n2 == 384 || t.n2 == 512)) {
     // items {channel * na + angle, row tile, nn1, k2lo | active R-tile pairs << 16}
     std::vector<int32_t> items;
     for (int ch = 0; ch < t.nc; ch++)
@@ -4149,9 +3430,6 @@ hipError_t build_plans(Ctx* c) {
                        hipMemcpyHostToDevice)) != hipSuccess)
       return e;
     c->rad_nitems = (int)(items.size() / 4);
-    e = c->precision == MW3_MIXED ? run_rad<float>(c, nullptr, nullptr, nullptr, 2)
-                                  : run_rad<double>(c, nullptr, nullptr, nullptr, 2);
-    if (e != hipSuccess) return e;
   }
   // one-pass angular kernel when both products fit its register tiles
   c->ang_nt = 0;
@@ -4271,58 +3549,93 @@ const float* op_psi<float>(Ctx* c, const double* psi) {
   return psi_shadow(c, psi);
 }
 
-template <typename T>
-static hipError_t hpsi_impl(Ctx* c, const double* psi64) {
-  const T* psi = op_psi<T>(c, psi64);
-  if (!psi) return hipErrorInvalidValue;
+// the update's arguments for psi; mode 3: G of psi only
+static step::UpArgs update_args(Ctx* c, int mode, const double* psi, bool proj) {
   const HostTables& t = c->t;
-  hipStream_t s = c->stream;
-  T* t1 = (T*)c->d_t1;
-  T* t2 = (T*)c->d_t2;
-  const T* tab = (const T*)c->d_dst_tables;
-  hipError_t e;
-  // mixed precision: the angular term on the third stream, beside the radial
-  // passes (it reads psi, written by the previous update on the main stream,
-  // and writes only its own slabs, which the next update reads after ev_ang);
-  // measured 3.5% faster per step than one stream at configuration 2, while
-  // the FP64 pair ran 2% slower side by side (its angular kernel holds a
-  // whole CU's LDS)
-  hipStream_t sa = c->opt_side ? c->side : s;
-  // kernel variants of this context's options (the autotuner's choices)
-  const bool use_rad = c->rad_nitems && c->opt_radial;
-  const bool use_mid = c->mid_nitems && c->opt_radial;
-  const bool use_fold = c->ang_fold && c->opt_angular == 0;
-  const bool use_one = c->ang_nt && c->opt_angular <= 1 && !use_fold;
-  // folded parts beside the Coriolis pass (mixed precision, FP16 products)
-  const bool use_cor = sizeof(T) == 4 && c->ang_fold_cor && c->opt_angular == 0 && c->opt_fp16 &&
-                       !use_fold && !use_one && !c->ang_fused;
-  // (its back part forms the coefficients and the Omega +- 1 terms itself:
-  // no coefficient pass)
-  const bool use_cor3 = use_cor;
-  // the forward R pass first (measured 1.3% faster per FP64 step than after
-  // the angular term)
-  timer_begin(c, K_DST_R);
-  e = use_rad ? run_rad<T>(c, psi, t1, t2, 0)
-              : run_gemm<G_DST_R, T, T, T, T>(s, psi, tab, t1, c->p_dstR);
-  if (e != hipSuccess) return e;
-  timer_end(c, K_DST_R);
-  if (sa != s) {
-    if (c->slice_fresh) {  // recorded after the update that wrote psi, nothing writing it since
-      if ((e = hipStreamWaitEvent(sa, c->ev_slice, 0)) != hipSuccess) return e;
-    } else {
-      if ((e = hipEventRecord(c->ev_psi, s)) != hipSuccess) return e;
-      if ((e = hipStreamWaitEvent(sa, c->ev_psi, 0)) != hipSuccess) return e;
+  const bool mixed = c->precision == MW3_MIXED;
+  step::UpArgs a{};
+  a.waves = (const step::UpWave*)c->d_up_wave;
+  a.segs = (const step::UpSeg*)c->d_up_seg;
+  a.tiles = c->d_up_tile;
+  a.nwaves = c->up_nwaves;
+  a.nseg = c->up_nseg;
+  a.tmax = c->up_tmax;
+  a.absfr2 = c->d_absfr2;
+  a.rowtab = c->d_up_row;
+  a.tab = c->d_up_tab;
+  a.g1 = c->d_g1;
+  a.g2 = c->d_g2;
+  a.ns = c->up_ns;
+  a.kst = c->up_kst;
+  a.psi = psi;
+  a.psi32 = mixed ? psi_shadow(c, psi) : nullptr;
+  a.out = mode == 0 ? c->d_hout : c->d_psim1;
+  a.out32 = mixed && mode != 0 ? psi_shadow(c, c->d_psim1) : nullptr;
+  a.tkin = c->d_t2;
+  a.ang = c->d_ang;
+  a.v = c->d_v;
+  a.psi0 = c->s.iphoto >= 1 ? c->d_psi0 : nullptr;
+  a.ch_elec = c->d_ch_elec;
+  a.ch_omega = c->d_ch_omega;
+  a.ch_cpl = c->d_ch_cpl;
+  a.nc = t.nc;
+  a.ne = t.ne;
+  a.na = t.na;
+  a.n1 = t.n1;
+  a.n2 = t.n2;
+  a.emindlt = c->s.emindlt;
+  a.rdelta2 = 1.0 / c->s.delta2;
+  a.radcut = t.radcut;
+  a.rsah2 = 1.0 / std::sqrt(c->s.ah2);
+  a.mode = mode;
+  if (c->graph_slot_dev) {
+    const int q = psi == c->graph_psi0 ? 0 : 1;
+    a.dslot = c->d_slot + q;
+    a.dslot_next = c->d_slot + (1 - q);
+  }
+  a.slot = c->ring_fill;
+  a.part = mode == 1 || mode == 2 ? c->d_norm_part : nullptr;
+  if (proj && mode == 2) {
+    a.slice = t.ncvj > 0 ? c->d_ring_slice : nullptr;
+    a.ir2abs = c->s.ir2abs;
+    a.upart = t.nflux > 0 || c->prod_on ? c->d_up_part : nullptr;
+    if (c->prod_on) {
+      a.tprod = c->d_tprod;
+      a.tp_cstride = c->pr_tstride;
     }
   }
-  c->slice_fresh = false;
-  c->cvj_joined = false;
-  timer_begin(c, K_ANG_FWD, sa);
+  return a;
+}
+
+static hipError_t run_update(Ctx* c, int mode, const double* psi, bool proj) {
+  const step::UpArgs a = update_args(c, mode, psi, proj);
+  if (c->precision == MW3_MIXED && !a.psi32) return hipErrorInvalidValue;
+  // one electronic state: V is diagonal (each Omega channel couples only to
+  // itself, through the one V slab); else listed partners where they fit
+  const int cpl = c->t.ne == 1 ? 0 : c->d_ch_cpl ? 1 : 2;
+  const int aux = (a.tprod ? 1 : 0) | (a.psi0 ? 2 : 0);
+  const int nk1 = c->opt_radial ? c->up_nk1 : 0;
+  return c->precision == MW3_MIXED ? step_update_f32(c, a, nk1, cpl, aux, mode)
+                                   : step_update_f64(c, a, nk1, cpl, aux, mode);
+}
+
+// the angular term of psi on stream s
+template <typename T>
+static hipError_t angular_impl(Ctx* c, const T* psi, hipStream_t s) {
+  const HostTables& t = c->t;
+  hipError_t e;
+  // kernel variants of this context's options (the autotuner's choices)
+  const bool use_fold = c->ang_fold && c->opt_angular == 0;
+  const bool use_one = c->ang_nt && c->opt_angular <= 1 && !use_fold;
+  // folded parts beside the Coriolis pass (mixed precision, FP16 products):
+  // the back part forms the coefficients and the Omega +- 1 terms itself
+  const bool use_cor = sizeof(T) == 4 && c->ang_fold_cor && c->opt_angular == 0 && c->opt_fp16 &&
+                       !use_fold && !use_one && !c->ang_fused;
+  timer_begin(c, K_ANG_FWD, s);
   if (use_fold) {
-    if ((e = launch_ang_fold<T>(c, psi, sa)) != hipSuccess) return e;
-    timer_end(c, K_ANG_FWD, sa);
+    if ((e = launch_ang_fold<T>(c, psi, s)) != hipSuccess) return e;
   } else if (use_one) {
-    if ((e = launch_ang_fused<T>(c, psi, sa)) != hipSuccess) return e;
-    timer_end(c, K_ANG_FWD, sa);
+    if ((e = launch_ang_fused<T>(c, psi, s)) != hipSuccess) return e;
   } else if (c->ang_fused) {
     KinParams ka{};
     ka.n1 = t.n1;
@@ -4330,37 +3643,32 @@ static hipError_t hpsi_impl(Ctx* c, const double* psi64) {
     ka.bcoef = (const double*)c->d_bcoef;
     ka.nJ = t.nJ;
     ka.n2 = t.n2;
-    e = run_gemm<G_ANG_FWD, T, T, T, T>(sa, (const T*)c->d_Dmat, psi, (T*)c->d_phi,
+    e = run_gemm<G_ANG_FWD, T, T, T, T>(s, (const T*)c->d_Dmat, psi, (T*)c->d_phi,
                                         c->p_angF, ka);
     if (e != hipSuccess) return e;
-    timer_end(c, K_ANG_FWD, sa);
+  } else if (use_cor) {
+    if constexpr (sizeof(T) == 4) {
+      if ((e = launch_ang_cor<1>(c, psi, s)) != hipSuccess) return e;
+    }
   } else {
-    if constexpr (sizeof(T) == 4) {
-      if (use_cor) {
-        if ((e = launch_ang_cor<1>(c, psi, sa)) != hipSuccess) return e;
-      }
-    }
-    if (!use_cor) {
-      e = run_gemm<G_ANG_FWD, T, T, T, T>(sa, (const T*)c->d_Dmat, psi, (T*)c->d_fbr,
-                                          c->p_angF);
-      if (e != hipSuccess) return e;
-    }
-    timer_end(c, K_ANG_FWD, sa);
+    e = run_gemm<G_ANG_FWD, T, T, T, T>(s, (const T*)c->d_Dmat, psi, (T*)c->d_fbr, c->p_angF);
+    if (e != hipSuccess) return e;
   }
-  if (use_cor3) {
+  timer_end(c, K_ANG_FWD, s);
+  if (use_cor) {
     if constexpr (sizeof(T) == 4) {
-      timer_begin(c, K_ANG_BWD, sa);
+      timer_begin(c, K_ANG_BWD, s);
       // (the psi argument is not read by part 3)
-      if ((e = launch_ang_cor<3>(c, (const float*)c->d_phi, sa)) != hipSuccess) return e;
-      timer_end(c, K_ANG_BWD, sa);
+      if ((e = launch_ang_cor<3>(c, (const float*)c->d_phi, s)) != hipSuccess) return e;
+      timer_end(c, K_ANG_BWD, s);
     }
   } else if (!use_fold && !use_one && !c->ang_fused) {
-    timer_begin(c, K_CORIOLIS, sa);
+    timer_begin(c, K_CORIOLIS, s);
     const unsigned nall = (unsigned)((int64_t)t.nJ * ((t.n1 + FBR_RB - 1) / FBR_RB));
     switch (c->fbr_all ? t.nc : 0) {
 #define MW3_FBR(NC)                                                                              \
   case NC:                                                                                       \
-    hipLaunchKernelGGL((k_fbr_coef_all<T, NC>), dim3(nall), dim3(FBR_THREADS), 0, sa,           \
+    hipLaunchKernelGGL((k_fbr_coef_all<T, NC>), dim3(nall), dim3(FBR_THREADS), 0, s,            \
                        (const T*)c->d_fbr, (T*)c->d_phi, (const double*)c->d_acoef,             \
                        (const double*)c->d_bcoef, c->d_nbr, t.nJ, t.n1, t.n2);                  \
     break;
@@ -4374,51 +3682,90 @@ static hipError_t hpsi_impl(Ctx* c, const double* psi64) {
 #undef MW3_FBR
       default:
         hipLaunchKernelGGL(k_fbr_coef<T>, dim3((unsigned)((int64_t)t.nc * t.nJ * t.n1)),
-                           dim3(256), 0, sa, (const T*)c->d_fbr, (T*)c->d_phi,
+                           dim3(256), 0, s, (const T*)c->d_fbr, (T*)c->d_phi,
                            (const double*)c->d_acoef, (const double*)c->d_bcoef, c->d_nbr, t.nc,
                            t.nJ, t.n1, t.n2);
     }
     if ((e = hipGetLastError()) != hipSuccess) return e;
-    timer_end(c, K_CORIOLIS, sa);
+    timer_end(c, K_CORIOLIS, s);
   }
-  if (!use_one && !use_fold && !use_cor3) {
-    timer_begin(c, K_ANG_BWD, sa);
-    e = run_gemm<G_ANG_BWD, T, T, T, T>(sa, (const T*)c->d_Dmat, (const T*)c->d_phi,
+  if (!use_one && !use_fold && !use_cor) {
+    timer_begin(c, K_ANG_BWD, s);
+    e = run_gemm<G_ANG_BWD, T, T, T, T>(s, (const T*)c->d_Dmat, (const T*)c->d_phi,
                                         (T*)c->d_ang, c->p_angB);
     if (e != hipSuccess) return e;
-    timer_end(c, K_ANG_BWD, sa);
+    timer_end(c, K_ANG_BWD, s);
   }
-  if (sa != s) {
-    // the second stream's sums of the last step end before ev_ang too, so
-    // that the next update, which rewrites what they read, waits once
-    if (c->cvj_pending) {
-      if ((e = hipStreamWaitEvent(sa, c->ev_cvj, 0)) != hipSuccess) return e;
-      c->cvj_joined = true;
-    }
-    if ((e = hipEventRecord(c->ev_ang, sa)) != hipSuccess) return e;
-  }
-  // radial kinetic correction on the low modes: folded DST over R, folded DST
-  // over r times (c - E)_+ divi, back over r, back over R into d_t2; the
-  // update forms T psi = radcut psi - d_t2 on rows r < nn1
-  KinParams kp{c->d_nn1, c->d_p2r1, c->d_p2r2, c->d_divi, t.radcut, t.n1};
-  timer_begin(c, K_DST_r);
-  if (use_mid) {
-    if ((e = launch_rad_mid<T>(c)) != hipSuccess) return e;
-  } else {
-    e = run_gemm<G_DST_r_KIN, T, T, T, T>(s, tab, t1, t2, c->p_dstr, kp);
-    if (e != hipSuccess) return e;
-    e = run_gemm<G_DST_r_INV, T, T, T, T>(s, tab, t2, t1, c->p_dstr2);
-    if (e != hipSuccess) return e;
-  }
-  timer_end(c, K_DST_r);
-  timer_begin(c, K_DST_RINV);
-  e = use_rad ? run_rad<T>(c, psi, t1, t2, 1)
-              : run_gemm<G_DST_R_INV, T, T, T, T>(s, t1, tab, t2, c->p_dstRi);
-  if (e != hipSuccess) return e;
-  timer_end(c, K_DST_RINV);
-  return sa != s ? hipStreamWaitEvent(s, c->ev_ang, 0) : hipSuccess;
+  return hipSuccess;
 }
 
+template <typename T>
+static hipError_t hpsi_impl(Ctx* c, const double* psi64) {
+  const T* psi = op_psi<T>(c, psi64);
+  if (!psi) return hipErrorInvalidValue;
+  const HostTables& t = c->t;
+  hipStream_t s = c->stream;
+  T* t1 = (T*)c->d_t1;
+  T* t2 = (T*)c->d_t2;
+  const T* tab = (const T*)c->d_dst_tables;
+  hipError_t e;
+  const bool use_rr = c->up_nk1 && c->opt_radial;
+  // the angular term beside the radial passes, on its own stream (option): it
+  // reads psi, written on the main stream, and writes only its own slabs
+  hipStream_t sa = c->opt_side ? c->side : s;
+  if (sa != s) {
+    if ((e = hipEventRecord(c->ev_psi, s)) != hipSuccess) return e;
+    if ((e = hipStreamWaitEvent(sa, c->ev_psi, 0)) != hipSuccess) return e;
+  }
+  if ((e = angular_impl<T>(c, psi, sa)) != hipSuccess) return e;
+  const bool use_rad = c->rad_nitems && c->opt_radial;
+  const bool use_mid = c->mid_nitems && c->opt_radial;
+  // radial kinetic correction on the low modes.  FP64: r products first, in
+  // the update (mw3_step.h); G of psi is left by the update that wrote it, or
+  // formed here; then its R products.  Else R products first, into the
+  // correction slab d_t2, by the low-mode kernels or as batched GEMMs
+  if (use_rr) {
+    if (!c->g_fresh) {
+      timer_begin(c, K_DST_R);
+      if ((e = run_update(c, 3, psi64, false)) != hipSuccess) return e;
+      timer_end(c, K_DST_R);
+    }
+    timer_begin(c, K_DST_r);
+    const step::RrArgs ra{c->d_g1, c->d_g2, c->d_rr_f, c->d_rr_b, c->d_rr_w, t.na, t.n1, t.n2,
+                          c->up_nk1, c->up_kst, c->rr_nb, c->d_up_sfirst, c->up_ns,
+                          c->up_nt == 2 ? 5 : 4, c->up_segmax};
+    if ((e = step_rad_rr_f64(c, ra)) != hipSuccess) return e;
+    timer_end(c, K_DST_r);
+  } else {
+    timer_begin(c, K_DST_R);
+    e = use_rad ? run_rad<T>(c, psi, t1, t2, 0)
+                : run_gemm<G_DST_R, T, T, T, T>(s, psi, tab, t1, c->p_dstR);
+    if (e != hipSuccess) return e;
+    timer_end(c, K_DST_R);
+    timer_begin(c, K_DST_r);
+    if (use_mid) {
+      if ((e = launch_rad_mid<T>(c)) != hipSuccess) return e;
+    } else {
+      KinParams kp{c->d_nn1, c->d_p2r1, c->d_p2r2, c->d_divi, t.radcut, t.n1};
+      e = run_gemm<G_DST_r_KIN, T, T, T, T>(s, tab, t1, t2, c->p_dstr, kp);
+      if (e != hipSuccess) return e;
+      e = run_gemm<G_DST_r_INV, T, T, T, T>(s, tab, t2, t1, c->p_dstr2);
+      if (e != hipSuccess) return e;
+    }
+    timer_end(c, K_DST_r);
+    timer_begin(c, K_DST_RINV);
+    e = use_rad ? run_rad<T>(c, psi, t1, t2, 1)
+                : run_gemm<G_DST_R_INV, T, T, T, T>(s, t1, tab, t2, c->p_dstRi);
+    if (e != hipSuccess) return e;
+    timer_end(c, K_DST_RINV);
+  }
+  c->g_fresh = false;
+  if (sa != s) {
+    if ((e = hipEventRecord(c->ev_ang, sa)) != hipSuccess) return e;
+    if ((e = hipStreamWaitEvent(s, c->ev_ang, 0)) != hipSuccess) return e;
+  }
+  return hipSuccess;
+}
 __global__ void k_to_f32(const double* __restrict__ src, float* __restrict__ dst, int64_t n) {
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
        i += (int64_t)gridDim.x * blockDim.x)
@@ -4445,134 +3792,44 @@ hipError_t launch_hpsi(Ctx* c, const double* psi) {
   return hpsi_impl<double>(c, psi);
 }
 
-template <typename T>
-static hipError_t update_impl(Ctx* c, int mode, int slot, const double* psi, bool proj) {
-  // psi_new rows that are never written (outside the compressed grid) keep
-  // zeros, so the reactant slice must start cleared only once (at create)
-  const HostTables& t = c->t;
-  const int nb = c->nnorm_blocks;  // work items
-  UpdArgs a{};
-  a.items = c->d_uw_item;
-  a.urow = c->d_uw_row;
-  a.uword = c->d_uw_word;
-  a.upart = c->d_uw_part;
-  a.nitems = nb;
-  a.nn1 = c->d_nn1;
-  a.absfr1 = c->d_absfr1;
-  a.absfr2 = c->d_absfr2;
-  a.ch_elec = c->d_ch_elec;
-  a.ch_omega = c->d_ch_omega;
-  a.ch_cpl = c->d_ch_cpl;
-  a.psi0 = (c->s.iphoto >= 1) ? c->d_psi0 : nullptr;
-  a.part = mode != 0 ? c->d_norm_part : nullptr;
-  a.nc = t.nc;
-  a.ne = t.ne;
-  a.na = t.na;
-  a.n1 = t.n1;
-  a.n2 = t.n2;
-  a.emindlt = c->s.emindlt;
-  a.rdelta2 = 1.0 / c->s.delta2;
-  a.radcut = t.radcut;
-  a.mode = mode;
-  a.pflux = (proj && t.nflux > 0 && c->d_fmap) ? 1 : 0;
-  a.fmap = c->d_fmap;
-  a.ir1flux = c->d_ir1flux;
-  a.zar = c->d_zar1flux;
-  a.zr = c->d_ring_zr + (int64_t)slot * t.nflux;
-  a.zdr = c->d_ring_zdr + (int64_t)2 * slot * t.nflux;
-  a.slice = (proj && t.ncvj > 0) ? c->d_slice : nullptr;
-  a.ir2abs = c->s.ir2abs;
-  a.rsah2 = 1.0 / std::sqrt(c->s.ah2);
-  a.out32 = mode != 0 ? psi_shadow(c, c->d_psim1) : nullptr;
-  a.psi32 = nullptr;
-  if (sizeof(T) == 4 && mode == 2) {
-    a.psi32 = psi_shadow(c, psi);  // current: H psi has just read it
-    if (!a.psi32) return hipErrorInvalidValue;
-  }
-  const bool prodp = mode == 2 && proj && c->prod_on;
-  a.tprod = prodp ? c->d_tprod : nullptr;
-  a.tp_cstride = c->pr_tstride;
-  a.ppart = c->d_ppart;
-  timer_begin(c, K_UPDATE);
-  double* out = mode == 0 ? c->d_hout : c->d_psim1;
-  const bool projk = a.pflux || a.slice;
-  const bool autoc = a.psi0 != nullptr;
-  const unsigned nblk4 = (unsigned)((nb + 3) / 4);  // one work item per wave
-  if (nblk4 > 0) {
-    // one electronic state: V is diagonal (each Omega channel couples only to
-    // itself, through the one V slab), whatever the channel count
-    if (t.ne == 1)
-      dispatch_update<T, true, false>(c, nblk4, psi, out, a, projk, autoc, prodp);
-    else if (c->d_ch_cpl)  // several states, at most 4 channels per Omega
-      dispatch_update<T, false, true>(c, nblk4, psi, out, a, projk, autoc, prodp);
-    else
-      dispatch_update<T, false, false>(c, nblk4, psi, out, a, projk, autoc, prodp);
-  }
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
-  // the step loop (mode 2) reduces the partials on the second stream, beside
-  // the next step's H psi (launch_projections)
-  if (mode == 1) e = launch_update_tail(c, mode, slot, proj, c->stream);
-  timer_end(c, K_UPDATE);
-  return e;
-}
-
-// flux columns and norm of the update's work-item partials, into ring slot
-hipError_t launch_update_tail(Ctx* c, int mode, int slot, bool proj, hipStream_t st) {
-  const HostTables& t = c->t;
-  if (mode == 2 && proj && t.nflux > 0 && c->d_fmap) {
-    const int ng = t.nc * t.na * ((t.n2 + 63) / 64);
-    hipLaunchKernelGGL(k_update_flux, dim3(ng), dim3(64), 0, st, c->d_uw_part, c->d_uw_gfirst,
-                       c->d_fmap, c->d_ring_zr, c->d_ring_zdr, t.n2, t.nflux,
-                       ring_slot(c, slot));
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-  }
-  if (mode != 0)
-    hipLaunchKernelGGL(k_reduce_parts, dim3(1), dim3(256), 0, st, c->d_norm_part,
-                       c->nnorm_blocks, c->d_ring_norm, ring_slot(c, slot));
-  return hipGetLastError();
-}
-
 hipError_t launch_update(Ctx* c, int mode, const double* psi, bool proj) {
-  int slot = c->ring_fill;
-  if (c->precision == MW3_MIXED) return update_impl<float>(c, mode, slot, psi, proj);
-  return update_impl<double>(c, mode, slot, psi, proj);
+  timer_begin(c, K_UPDATE);
+  const hipError_t e = run_update(c, mode, psi, proj);
+  if (e != hipSuccess) return e;
+  timer_end(c, K_UPDATE);
+  // the damped step leaves G of the psi it writes
+  if (mode == 2) c->g_fresh = c->up_nk1 && c->opt_radial;
+  return hipSuccess;
 }
 
-// the per-step sums of the update's partials and slice on stream st: flux
-// columns and norm, reactant-state and product-state sums, into ring slot
-hipError_t launch_tail_sums(Ctx* c, int slot, hipStream_t st) {
+// per-step sums of the ring's steps from what the updates left
+hipError_t launch_ring_sums(Ctx* c) {
   const HostTables& t = c->t;
+  const int ns = c->ring_fill;
   hipError_t e;
-  timer_begin(c, K_UPDATE_TAIL, st);
-  if ((e = launch_update_tail(c, 2, slot, true, st)) != hipSuccess) return e;
-  timer_end(c, K_UPDATE_TAIL, st);
-  if (t.ncvj > 0) {
-    timer_begin(c, K_PROJ, st);
-    int nj = c->s.jmax - c->s.jini + 1, nv = c->s.nvmax - c->s.nvini + 1;
-    hipLaunchKernelGGL(k_cvj, dim3(t.nc * nj), dim3(64 * CVJ_WAVES), sizeof(double) * t.n1, st,
-                       c->d_slice, c->d_dcvj, c->d_fdv, c->d_ring_cvj, nj, nv, t.na, t.n1,
-                       (int64_t)t.ncvj, ring_slot(c, slot));
+  if (ns == 0) return hipSuccess;
+  timer_begin(c, K_UPDATE_TAIL);
+  hipLaunchKernelGGL(k_norm_ring, dim3(ns), dim3(256), 0, c->stream, c->d_norm_part,
+                     c->up_nwaves, c->d_ring_norm);
+  if ((e = hipGetLastError()) != hipSuccess) return e;
+  if (t.nflux > 0) {
+    hipLaunchKernelGGL(k_flux_ring, dim3(nblk(t.nflux, 256), ns), dim3(256), 0, c->stream,
+                       c->d_up_part, c->d_up_sfirst, c->d_flux_col, c->d_ring_zr, c->d_ring_zdr,
+                       t.nflux, c->up_nseg, t.n2, t.nplane, c->up_ns, 16 * c->up_nt);
     if ((e = hipGetLastError()) != hipSuccess) return e;
-    timer_end(c, K_PROJ, st);
   }
-  if (c->prod_on && (e = launch_prod_step(c, slot, st)) != hipSuccess) return e;
-  return hipSuccess;
-}
-
-// reactant-state amplitudes of the slice the update wrote, into ring slot
-hipError_t launch_projections(Ctx* c, int slot) {
-  hipError_t e;
-  // on the second stream, after the update that wrote the slice and the
-  // partials: the flux columns and the norm of the step, then the
-  // reactant- and product-state sums
-  if ((e = hipEventRecord(c->ev_slice, c->stream)) != hipSuccess) return e;
-  if ((e = hipStreamWaitEvent(c->aux, c->ev_slice, 0)) != hipSuccess) return e;
-  if ((e = launch_tail_sums(c, slot, c->aux)) != hipSuccess) return e;
-  if ((e = hipEventRecord(c->ev_cvj, c->aux)) != hipSuccess) return e;
-  c->cvj_pending = true;
-  return hipSuccess;
+  timer_end(c, K_UPDATE_TAIL);
+  if (t.ncvj > 0) {
+    timer_begin(c, K_PROJ);
+    const int nj = c->s.jmax - c->s.jini + 1, nv = c->s.nvmax - c->s.nvini + 1;
+    const int jb = std::max(1, std::min(CVJ_J, 8192 / t.n1));  // within 64 KB of LDS
+    hipLaunchKernelGGL(k_cvj_ring, dim3(t.nc * ((nj + jb - 1) / jb), ns), dim3(256),
+                       sizeof(double) * jb * t.n1, c->stream, c->d_ring_slice, c->d_dcvj,
+                       c->d_fdv, c->d_ring_cvj, t.nc, nj, nv, t.na, t.n1, jb, (int64_t)t.ncvj);
+    if ((e = hipGetLastError()) != hipSuccess) return e;
+    timer_end(c, K_PROJ);
+  }
+  return c->prod_on ? launch_prod_sums(c) : hipSuccess;
 }
 
 hipError_t launch_energy_accum(Ctx* c) {
@@ -4627,44 +3884,31 @@ hipError_t launch_psie(Ctx* c, int k) {
 // ---------------------------------------------------------------------------
 // product-state projection (prodpaq / prodcvj, SRC/mod_coortrans01_02.f:694-822)
 // ---------------------------------------------------------------------------
-// funprod(c, ia, R) = sum over the update items of (c, ia, 64-R chunk) of their
-// partials (sum_r transRgjac psi_new), then for each product helicity o and
-// electronic state e the channel sum ring[o][e][l] = sum_{c: elec(c) = e}
-// dtrans[c][o][l] funprod(c, l), l = (ia - nangproj0) n2p + (R - n2prod0).
-// Block per (angle of the range, 64-R chunk of the range), lane = R.  Each
-// lane reads back only its own column of f, so no barrier is needed; f is
-// sized by the launch to the channel count (nc 64-lane rows), so that the
-// block holds only the LDS it uses beside the kernels of the other streams.
-__global__ __launch_bounds__(64) void k_prod_fun(const double* __restrict__ ppart,
-                                                 const int32_t* __restrict__ gfirst,
-                                                 const double* __restrict__ dtrans,
-                                                 const int32_t* __restrict__ ch_elec,
-                                                 double* __restrict__ ring_all, int nc, int ne,
-                                                 int na, int n2, int nap0, int n2p0, int n2p,
-                                                 int nomb, int rc0, int nrcp, int64_t L,
-                                                 RingSlot rs) {
-  double* __restrict__ ring = ring_all + (int64_t)rs.get() * nomb * ne * L;
-  extern __shared__ double f[];  // [nc][64]
-  const int lane = threadIdx.x;
-  const int a = blockIdx.x / nrcp, rc = rc0 + blockIdx.x % nrcp;
-  const int ia = nap0 + a;
-  const int R = rc * 64 + lane;
-  const int nrc = (n2 + 63) / 64;
-  for (int ch = 0; ch < nc; ch++) {
-    const int g = (ch * na + ia) * nrc + rc;
-    double s = 0.0;
-    for (int it = gfirst[g]; it < gfirst[g + 1]; it++) s += ppart[(int64_t)it * 64 + lane];
-    f[ch * 64 + lane] = s;
-  }
-  if (R < n2p0 || R >= n2p0 + n2p) return;
-  const int64_t l = (int64_t)a * n2p + (R - n2p0);
+// funprod(c, l) = sum_r transRgjac psi_new, l = (ia - nangproj0) n2p +
+// (R - n2prod0), is left by the update per segment for every step of the ring;
+// for each product helicity o and electronic state e the channel sum is
+// ring[s][o][e][l] = sum_{c: elec(c) = e} dtrans[c][o][l] funprod(c, l).
+__global__ __launch_bounds__(256) void k_prod_fun(const double* __restrict__ upart,
+                                                  const int32_t* __restrict__ sfirst,
+                                                  const double* __restrict__ dtrans,
+                                                  const int32_t* __restrict__ ch_elec,
+                                                  double* __restrict__ ring, int nc, int ne,
+                                                  int nomb, int64_t L, int na, int nap0, int n2p0,
+                                                  int n2p, int nseg, int ns, int sw) {
+  const int64_t l = (int64_t)blockIdx.x * blockDim.x + threadIdx.x, slot = blockIdx.y;
+  if (l >= L) return;
+  const int ia = nap0 + (int)(l / n2p), R = n2p0 + (int)(l % n2p), s = R / sw, x = R - s * sw;
   for (int o = 0; o < nomb; o++)
-    for (int e = 0; e < ne; e++) {
-      double acc = 0.0;
-      for (int ch = 0; ch < nc; ch++)
-        if (ch_elec[ch] == e) acc += f[ch * 64 + lane] * dtrans[((int64_t)ch * nomb + o) * L + l];
-      ring[((int64_t)o * ne + e) * L + l] = acc;
-    }
+    for (int e = 0; e < ne; e++) ring[((slot * nomb + o) * ne + e) * L + l] = 0.0;
+  for (int ch = 0; ch < nc; ch++) {
+    const int64_t q = (int64_t)(ch * na + ia) * ns + s;
+    double f = 0.0;
+    for (int k = sfirst[q]; k < sfirst[q + 1]; k++)
+      f += upart[((slot * nseg + k) * 4 + 3) * sw + x];
+    for (int o = 0; o < nomb; o++)
+      ring[((slot * nomb + o) * ne + ch_elec[ch]) * L + l] +=
+          f * dtrans[((int64_t)ch * nomb + o) * L + l];
+  }
 }
 
 // Cvjprod[s][o][vj] = sum over the K chunks of the flush GEMM's partials
@@ -4681,19 +3925,14 @@ __global__ void k_prod_sum(const double* __restrict__ part, double* __restrict__
   if (s == ns - 1) last[x] = acc;
 }
 
-hipError_t launch_prod_step(Ctx* c, int slot, hipStream_t s) {
-  const HostTables& t = c->t;
-  const int rc0 = c->pr_n2p0 / 64, rc1 = (c->pr_n2p0 + c->pr_n2p - 1) / 64;
-  const int nrcp = rc1 - rc0 + 1;
-  if (t.nc > kProdMaxCh) return hipErrorInvalidValue;  // mw3_prod_attach rejects it first
-  timer_begin(c, K_PROD, s);
-  hipLaunchKernelGGL(k_prod_fun, dim3((unsigned)(c->pr_nap * nrcp)), dim3(64),
-                     sizeof(double) * 64 * t.nc, s, c->d_ppart,
-                     c->d_uw_gfirst, c->d_dtrans, c->d_ch_elec, c->d_ring_prod, t.nc, t.ne,
-                     t.na, t.n2, c->pr_nap0, c->pr_n2p0, c->pr_n2p, c->pr_nomb, rc0, nrcp, c->pr_L,
-                     ring_slot(c, slot));
-  hipError_t e = hipGetLastError();
-  timer_end(c, K_PROD, s);
+hipError_t launch_prod_sums(Ctx* c) {
+  timer_begin(c, K_PROD);
+  hipLaunchKernelGGL(k_prod_fun, dim3(nblk(c->pr_L, 256), c->ring_fill), dim3(256), 0, c->stream,
+                     c->d_up_part, c->d_up_sfirst, c->d_dtrans, c->d_ch_elec, c->d_ring_prod,
+                     c->t.nc, c->t.ne, c->pr_nomb, c->pr_L, c->t.na, c->pr_nap0, c->pr_n2p0,
+                     c->pr_n2p, c->up_nseg, c->up_ns, 16 * c->up_nt);
+  const hipError_t e = hipGetLastError();
+  timer_end(c, K_PROD);
   return e;
 }
 
