@@ -125,7 +125,7 @@ static void free_all(Ctx* c) {
                   c->d_dst_tables, c->d_Dmat, c->d_acoef, c->d_bcoef, c->d_nbr,
                   c->d_flux_dense, c->d_flux_col, c->d_zar1flux, c->d_ring_zr, c->d_ring_zdr,
                   c->d_ring_cvj, c->d_zcr, c->d_zcdr, c->d_zs2, c->d_etot, c->d_fdv, c->d_dcvj,
-                  c->d_cvj_skip, c->d_norm_part, c->d_ring_norm, c->d_efe, c->d_zfe, c->d_phi,
+                  c->d_cvj_skip, c->d_norm_part, c->d_ring_norm, c->d_stats, c->d_efe, c->d_zfe, c->d_phi,
                   c->d_wmat, c->d_zero_skip, c->d_ch_elec, c->d_ch_omega, c->d_ch_cpl, c->d_potiflux,
                   c->d_flux_elec, c->d_scratch, c->d_fmap, c->d_ir1flux, c->d_ring_slice,
                   c->d_psi32, c->d_psim132, c->d_scr32, c->d_up_wave, c->d_up_seg,
@@ -350,6 +350,7 @@ int32_t mw3_create(const mw3_setup* setup, int32_t precision, mw3_ctx** out) {
          "mw3_create: slice");
   }
   CK(alloc_zero((void**)&c->d_ring_norm, sizeof(double) * 2 * kRing), "mw3_create: norms");
+  CK(alloc_zero((void**)&c->d_stats, sizeof(double) * stats_doubles()), "mw3_create: sums");
   if (setup->nofe > 0) {
     if (!setup->efe) {
       free_all(c);
@@ -439,21 +440,10 @@ int32_t mw3_cheby_begin(mw3_ctx* ctx, const double* psi0, double* stats3) {
   HIPCHK(c, launch_hpsi(c, c->d_psi), "mw3_cheby_begin: H psi0");
   if (stats3) {
     HIPCHK(c, launch_update(c, 0, c->d_psi), "mw3_cheby_begin: H psi0");
-    std::vector<double> h(n), p(psi0, psi0 + n);
-    HIPCHK(c, launch_gather_a0(c, c->d_hout, c->d_a0b), "mw3_cheby_begin: gather");
-    HIPCHK(c, hipMemcpyAsync(h.data(), c->d_a0b, n * sizeof(double), hipMemcpyDeviceToHost,
-                             c->stream),
-           "mw3_cheby_begin: download");
-    HIPCHK(c, hipStreamSynchronize(c->stream), "mw3_cheby_begin: sync");
-    double em = 0, x1 = 0, x2 = 0;
-    for (size_t i = 0; i < n; i++) {
-      em += p[i] * h[i];
-      x1 += p[i] * p[i];
-      x2 += h[i] * h[i];
-    }
-    stats3[0] = em;
-    stats3[1] = x1;
-    stats3[2] = x2;
+    HIPCHK(c, launch_stats(c, c->d_a0, c->d_hout), "mw3_cheby_begin: sums");
+    HIPCHK(c, hipMemcpyAsync(stats3, c->d_stats + stats_doubles() - 3, 3 * sizeof(double),
+                             hipMemcpyDeviceToHost, c->stream),
+           "mw3_cheby_begin: sums");
   }
   c->ring_fill = 0;
   c->rec_it.clear();

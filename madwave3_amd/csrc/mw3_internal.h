@@ -190,6 +190,7 @@ struct Ctx {
   double* d_dcvj = nullptr;
   uint8_t* d_cvj_skip = nullptr; // [ncvj] 1 if the reference state (kminelastic)
   double* d_norm_part = nullptr; // update wave sums [kRing][up_nwaves][2]
+  double* d_stats = nullptr;     // sums of mw3_cheby_begin (launch_stats)
   double* d_ring_norm = nullptr; // [kRing][2] (norm, autocorrelation)
   double* d_efe = nullptr;
   double* d_zfe = nullptr;       // [nofe][nc*nslab][2] dense
@@ -316,6 +317,8 @@ int build_tables(const mw3_setup* s, HostTables* t, std::string* err);
 
 // mw3_kernels.hip: launchers, return hipError_t
 hipError_t launch_scatter_a0(Ctx* c, const double* a0, double* dense);
+size_t stats_doubles();
+hipError_t launch_stats(Ctx* c, const double* a0, const double* h);
 hipError_t launch_gather_a0(Ctx* c, const double* dense, double* a0);
 hipError_t launch_hpsi(Ctx* c, const double* psi);
 float* psi_shadow(Ctx* c, const double* psi);  // FP32 copy of a psi slab (mixed), or null

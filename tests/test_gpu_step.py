@@ -83,3 +83,19 @@ def test_longest_r(n1, n2):
         g.begin(c.rpaq0)
         assert rel(g.steps(20)[0], n_o) < 10 * bar
         assert rel(g.state()[1], o.state()[1]) < 10 * bar
+
+
+@pytest.mark.parametrize("n1,n2,na", [(12, 12, 2), (32, 64, 16), (64, 128, 60)])
+def test_begin_sums(n1, n2, na):
+    """psi.H psi, psi.psi and H psi.H psi of the initial packet: fewer points than
+    a block, than the whole launch, and more (sums of n products: n 2^-53)."""
+    p = leps.config(1)
+    p.update(npun1=n1, npun2=n2, nangu=na, npun1min=8, jmax=min(5, na - 1), nvmax=2, netot=0,
+             iprod=0, kminelastic=4, width_bohr=0.6, absorb_bohr=4.5)
+    c = leps.build(p)
+    psi = np.random.default_rng(n1).standard_normal(c.ntot)
+    g = Propagator(c, MW3_FP64)
+    h = g.hphi(psi)
+    size = np.array([np.abs(psi * h).sum(), (psi * psi).sum(), (h * h).sum()])
+    want = np.array([(psi * h).sum(), (psi * psi).sum(), (h * h).sum()])
+    assert np.all(np.abs(g.begin(psi) - want) <= 2.0 * c.ntot * 2.0**-53 * size)
