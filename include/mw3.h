@@ -297,7 +297,8 @@ MW3_API int32_t mw3_cheby_spectrum(const double *autoc, int32_t kmax, double emi
 /* Execution options of a context (no counterpart in the reference; results
    do not depend on them beyond rounding order where stated).
    MW3_OPT_GRAPHS  1 (default): Chebyshev steps run as captured HIP graphs,
-                   one per step, whenever kernel timing is off and nofe = 0;
+                   of one step or of 16, whenever kernel timing is off and
+                   nofe = 0;
                    0: kernel by kernel.  Same kernels, same order of every
                    sum: results are bitwise identical.
    MW3_OPT_RADIAL  1 (default): the radial kinetic correction by the
@@ -314,8 +315,9 @@ MW3_API int32_t mw3_cheby_spectrum(const double *autoc, int32_t kmax, double emi
                    them.  A variant
                    not built for the context falls back to the next one.
    MW3_OPT_SIDE_STREAM  1: the angular term on its own stream beside the
-                   radial passes (default in MW3_MIXED); 0: one stream
-                   (default in MW3_FP64).
+                   radial passes (default in MW3_MIXED, where captured steps
+                   do so only beside batched GEMMs); 0: one stream (default
+                   in MW3_FP64).
    MW3_OPT_ANGULAR_GRID 1 (default) or 2: the folded angular kernel runs
                    its blocks per channel divided by this value.
    MW3_OPT_RADIAL_GRID  accepts 1 (default), 2 or 4 and has no effect: the

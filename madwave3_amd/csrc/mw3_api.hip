@@ -530,11 +530,27 @@ static hipError_t end_capture(hipStream_t s, hipError_t eb, hipGraphExec_t* out)
   return e;
 }
 
-// Captures one step of c as graph q (psi in buffer q).
-static hipError_t capture_step(Ctx* c, int q) {
+static void swap_psi(Ctx* c) {
+  std::swap(c->d_psi, c->d_psim1);
+  std::swap(c->d_psi32, c->d_psim132);
+}
+
+// Steps of one graph launch where that many are to come.  Between two graphs
+// the stream idles for 5 to 7 us: one launch per step cost the 32 x 64 x 16
+// grid a quarter of its step.
+constexpr int kRun = 16;
+
+// Captures one step of c as graph q (psi in buffer q), or kRun steps (an even
+// number, which leaves psi where it was) as graph 2.
+static hipError_t capture_steps(Ctx* c, int q) {
   hipError_t e = hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal);
   if (e != hipSuccess) return e;
-  return end_capture(c->stream, capture_body(c), &c->graph[q]);
+  for (int i = 0; i < (q == 2 ? kRun : 1); i++) {
+    if (i) swap_psi(c);
+    if (e == hipSuccess) e = capture_body(c);
+  }
+  if (q == 2) swap_psi(c);
+  return end_capture(c->stream, e, &c->graph[q]);
 }
 
 void drop_graphs(Ctx* c) {
@@ -554,17 +570,25 @@ static bool step_pre(Ctx* c) {
 }
 
 // Step of c, second part: the kernels, as a graph or one by one (a step whose
-// psi has no G yet runs one by one: it forms G first).
-static int step_body(Ctx* c, bool graphs) {
+// psi has no G yet runs one by one: it forms G first).  *run: the steps that
+// may be enqueued at once, then those that were.
+static int step_body(Ctx* c, bool graphs, int32_t* run) {
+  const bool many = *run >= kRun;
+  *run = 1;
   if (graphs && (c->g_fresh || !c->up_nk1 || !c->opt_radial)) {
-    const int q = c->d_psi == c->graph_psi0 ? 0 : 1;
+    int q = c->d_psi == c->graph_psi0 ? 0 : 1;
     if (c->dslot_host != c->ring_fill)
       HIPCHK(c, launch_slot_set(c, q, c->ring_fill), "mw3_cheby_steps: slot");
-    c->dslot_host = c->ring_fill + 1;
-    if (!c->graph[q]) HIPCHK(c, capture_step(c, q), "mw3_cheby_steps: step capture");
+    if (many && q == 0) {
+      q = 2;
+      *run = kRun;
+    }
+    c->dslot_host = c->ring_fill + *run;
+    if (!c->graph[q]) HIPCHK(c, capture_steps(c, q), "mw3_cheby_steps: step capture");
     HIPCHK(c, hipGraphLaunch(c->graph[q], c->stream), "mw3_cheby_steps: step graph");
     return MW3_OK;
   }
+  c->dslot_host = -1;
   HIPCHK(c, launch_hpsi(c, c->d_psi), "mw3_cheby_steps: H psi");
   HIPCHK(c, launch_update(c, 2, c->d_psi, true), "mw3_cheby_steps: update");
   return MW3_OK;
@@ -578,8 +602,7 @@ static int step_post(Ctx* c, int32_t* done, int32_t nsteps, double* norms,
   const int base = *done - c->ring_fill;  // output index of ring slot 0
   c->k += 1;
   if (!c->trial) HIPCHK(c, launch_psie(c, c->k), "mw3_cheby_steps: psi(E)");
-  std::swap(c->d_psi, c->d_psim1);
-  std::swap(c->d_psi32, c->d_psim132);
+  swap_psi(c);
   c->ring_fill += 1;
   *done += 1;
   if (c->trial && (c->ring_fill == kRing || *done == nsteps)) {
@@ -597,12 +620,18 @@ static int step_post(Ctx* c, int32_t* done, int32_t nsteps, double* norms,
 }
 
 // One Chebyshev step of c (H psi_k, update into psim1 = psi_{k+1},
-// projections, swap).
-static int step_enqueue(Ctx* c, int32_t* done, int32_t nsteps, double* norms, double* autocorr) {
+// projections, swap), or up to `most` of them at once (never past the end of
+// the ring or of the call; one at a time while kernels are timed).
+static int step_enqueue(Ctx* c, int32_t* done, int32_t nsteps, double* norms, double* autocorr,
+                        int32_t most = 1) {
   const bool graphs = step_pre(c);
-  int rc = step_body(c, graphs);
-  if (rc) return rc;
-  return step_post(c, done, nsteps, norms, autocorr);
+  int32_t run = c->timing ? 1 : std::min(most, std::min(nsteps - *done, kRing - c->ring_fill));
+  int rc = step_body(c, graphs, &run);
+  for (int32_t i = 0; i < run && rc == MW3_OK; i++) {
+    if (i) step_pre(c);
+    rc = step_post(c, done, nsteps, norms, autocorr);
+  }
+  return rc;
 }
 
 int32_t mw3_cheby_steps(mw3_ctx* ctx, int32_t nsteps, double* norms, double* autocorr) {
@@ -612,7 +641,8 @@ int32_t mw3_cheby_steps(mw3_ctx* ctx, int32_t nsteps, double* norms, double* aut
   if (nsteps < 0) return seterr(c, MW3_EINVAL, "mw3_cheby_steps: nsteps < 0");
   int32_t done = 0;
   int rc = MW3_OK;
-  while (done < nsteps && rc == MW3_OK) rc = step_enqueue(c, &done, nsteps, norms, autocorr);
+  while (done < nsteps && rc == MW3_OK)
+    rc = step_enqueue(c, &done, nsteps, norms, autocorr, kRun);
   return rc;
 }
 
@@ -630,16 +660,21 @@ int32_t mw3_cheby_steps_batch(mw3_ctx** ctxs, int32_t n, int32_t nsteps, double*
       return seterr(c, MW3_EINVAL, "mw3_cheby_steps_batch: contexts on different devices");
   }
   std::vector<int32_t> done(n, 0);
-  // step-major order: every context's step s is enqueued before any step s+1,
-  // so the streams of all contexts hold work at the same time (each member
-  // runs its steps as its own captured graphs where it can)
+  // in turns of a run of steps, so that the streams of all contexts hold work
+  // at the same time (each member runs its steps as its own captured graphs
+  // where it can)
   int rc = MW3_OK;
-  for (int32_t st = 0; st < nsteps && rc == MW3_OK; st++)
+  bool more = nsteps > 0;
+  while (more && rc == MW3_OK) {
+    more = false;
     for (int i = 0; i < n && rc == MW3_OK; i++) {
       Ctx* c = reinterpret_cast<Ctx*>(ctxs[i]);
-      rc = step_enqueue(c, &done[i], nsteps, norms ? norms + (size_t)i * nsteps : nullptr,
-                        nullptr);
+      if (done[i] < nsteps)
+        rc = step_enqueue(c, &done[i], nsteps, norms ? norms + (size_t)i * nsteps : nullptr,
+                          nullptr, kRun);
+      more = more || done[i] < nsteps;
     }
+  }
   return rc;
 }
 
@@ -1087,18 +1122,19 @@ int32_t mw3_get_option(const mw3_ctx* ctx, int32_t option, int32_t* value) {
   return MW3_OK;
 }
 
-// One autotuner trial: the context's current options over 2 + n steps from
-// the current state, timed over the last n with events on the main stream
+// One autotuner trial: the context's current options over n steps after those
+// that capture the graphs these n need, from the current state, timed with events on the main stream
 // once every stream has joined it.  No ring flush, no psi(E) sum.
 static int trial_ms(Ctx* c, int n, hipEvent_t e0, hipEvent_t e1, double* ms) {
   int32_t done = 0;
   c->trial = true;
   int rc = MW3_OK;
-  while (done < 2 && rc == MW3_OK) rc = step_enqueue(c, &done, 2, nullptr, nullptr);
+  const int warm = n >= kRun ? kRun + 2 : 2;
+  while (done < warm && rc == MW3_OK) rc = step_enqueue(c, &done, warm, nullptr, nullptr, kRun);
   if (rc == MW3_OK) {
     HIPCHK(c, hipEventRecord(e0, c->stream), "mw3_autotune: event");
     done = 0;
-    while (done < n && rc == MW3_OK) rc = step_enqueue(c, &done, n, nullptr, nullptr);
+    while (done < n && rc == MW3_OK) rc = step_enqueue(c, &done, n, nullptr, nullptr, kRun);
   }
   c->trial = false;
   if (rc) return rc;

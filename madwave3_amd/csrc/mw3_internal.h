@@ -297,7 +297,8 @@ struct Ctx {
   int flux_etest = 1;             // E > V(flux point) test when the flux sums are read
   bool trial = false;             // autotuner trial steps: no ring flush, no psi(E)
   bool graph_slot_dev = false;    // kernels being enqueued read their slot from d_slot
-  hipGraphExec_t graph[2] = {nullptr, nullptr};
+  // graph[2]: kRun steps from buffer 0, and back to it
+  hipGraphExec_t graph[3] = {nullptr, nullptr, nullptr};
   double* graph_psi0 = nullptr;   // d_psi at creation (buffer 0)
   int32_t* d_slot = nullptr;
   int dslot_host = -2;

@@ -3790,8 +3790,15 @@ static hipError_t hpsi_impl(Ctx* c, const double* psi64) {
   hipError_t e;
   const bool use_rr = c->up_nk1 && c->opt_radial;
   // the angular term beside the radial passes, on its own stream (option): it
-  // reads psi, written on the main stream, and writes only its own slabs
-  hipStream_t sa = c->opt_side ? c->side : s;
+  // reads psi, written on the main stream, and writes only its own slabs.
+  // Captured steps in mixed precision with the low-mode kernels keep one
+  // stream: a fork and a join inside a graph cost more than the overlap gives
+  // (128 x 256 x 60: 44 us a step against 50; 256 x 512 x 120: 125 against
+  // 128; three states 171 x 256 x 64: 92 against 97).  Beside the GEMMs of a
+  // coarse grid (256 x 256 x 140) the side stream gives 222 against 241, and
+  // outside graphs 122 against 125 at 256 x 512 x 120.
+  const bool one = c->graph_slot_dev && sizeof(T) == 4 && c->opt_radial && c->rad_nitems;
+  hipStream_t sa = c->opt_side && !one ? c->side : s;
   if (sa != s) {
     if ((e = hipEventRecord(c->ev_psi, s)) != hipSuccess) return e;
     if ((e = hipStreamWaitEvent(sa, c->ev_psi, 0)) != hipSuccess) return e;
