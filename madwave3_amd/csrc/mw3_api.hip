@@ -125,7 +125,7 @@ static void free_all(Ctx* c) {
                   c->d_dst_tables, c->d_Dmat, c->d_acoef, c->d_bcoef, c->d_nbr,
                   c->d_flux_dense, c->d_flux_col, c->d_zar1flux, c->d_ring_zr, c->d_ring_zdr,
                   c->d_ring_cvj, c->d_zcr, c->d_zcdr, c->d_zs2, c->d_etot, c->d_fdv, c->d_dcvj,
-                  c->d_cvj_skip, c->d_norm_part, c->d_ring_norm, c->d_stats, c->d_efe, c->d_zfe, c->d_phi,
+                  c->d_cvj_skip, c->d_norm_part, c->d_ring_norm, c->d_stats, c->d_fbr_rng, c->d_efe, c->d_zfe, c->d_phi,
                   c->d_wmat, c->d_zero_skip, c->d_ch_elec, c->d_ch_omega, c->d_ch_cpl, c->d_potiflux,
                   c->d_flux_elec, c->d_scratch, c->d_fmap, c->d_ir1flux, c->d_ring_slice,
                   c->d_psi32, c->d_psim132, c->d_scr32, c->d_up_wave, c->d_up_seg,
@@ -839,10 +839,7 @@ static void free_prod(Ctx* c) {
       (void)hipFree(*p);
       *p = nullptr;
     }
-  if (c->p_prod.d_descs) {
-    (void)hipFree(c->p_prod.d_descs);
-    c->p_prod.d_descs = nullptr;
-  }
+  free_plan(&c->p_prod);
   c->prod_on = false;
 }
 

@@ -95,13 +95,20 @@ struct GemmStrides {
   int64_t ldc_m, ldc_n;
 };
 
-// one pass of the step as a batch of GEMMs; vec: the operands meet the
-// alignment rules of the vectorised kernel; group / share_b: block order
-// (consecutive descriptors sharing the A panel / blocks sharing the B panel
-// kept on one XCD)
+// one 64 x 64 block of a pass: its descriptor, first row and column, and the
+// k from k0 up to k1 for which an operand may be other than zero
+struct GemmBlk {
+  int32_t z, m0, n0, k0, k1;
+};
+
+// one pass of the step as a batch of GEMMs, by the list of its blocks; vec:
+// the operands meet the alignment rules of the vectorised kernel; group /
+// share_b: order of the list (consecutive descriptors sharing the A panel /
+// blocks sharing the B panel kept on one XCD)
 struct GemmPlan {
   GemmDesc* d_descs = nullptr;
-  int nb = 0, maxM = 0, maxN = 0, vec = 0, group = 1, share_b = 0;
+  GemmBlk* d_blks = nullptr;
+  int nblk = 0, vec = 0, group = 1, share_b = 0;
   GemmStrides st{};
 };
 
@@ -204,6 +211,7 @@ struct Ctx {
   std::vector<double> rec_cvjp;  // [nrec][nomb * nvj] (product projection attached)
 
   // GEMM passes: R rows, r columns, angular forward, angular back
+  int32_t* d_fbr_rng = nullptr;  // [n1][2] first and last + 1 kept R of a row, any angle
   GemmPlan p_dstR, p_dstr, p_dstr2, p_dstRi, p_angF, p_angB;
   int32_t* d_rad_items = nullptr;  // R-pass work items {channel-angle, 16-row tile, nn1, k2lo}
   int rad_nitems = 0;              // 0: the R passes run as GEMMs
@@ -335,6 +343,7 @@ hipError_t launch_psie(Ctx* c, int k);
 hipError_t launch_zero(Ctx* c, void* p, size_t bytes);
 hipError_t build_plans(Ctx* c);
 void free_plans(Ctx* c);
+void free_plan(GemmPlan* p);
 hipError_t launch_flux_result(Ctx* c, double* d_out /* [(1+ne)][netot] */);
 // product projection: plan of the flush GEMM, per-step reduction into the ring
 hipError_t build_prod_plan(Ctx* c);

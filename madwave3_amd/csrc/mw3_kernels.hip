@@ -21,6 +21,7 @@
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
+#include <functional>
 
 #include "mw3_step.h"
 
@@ -128,6 +129,15 @@ __device__ __forceinline__ void tile_pos(int e, bool rowfast, int& rc, int& kk) 
   }
 }
 
+// Position in a plan's list of blocks.  Workgroups go to the 8 XCDs round
+// robin by linear id, each XCD with its own L2: each XCD takes one contiguous
+// run of the list, whose order (plan_blocks) puts the blocks that read the same
+// operand panel next to each other.
+__device__ __forceinline__ int gemm_block() {
+  const int hw = blockIdx.x, q = (int)(gridDim.x >> 3);
+  return hw < 8 * q ? (hw & 7) * q + (hw >> 3) : hw;
+}
+
 template <typename T, int TM, int TN, typename TA, typename TB>
 __device__ __forceinline__ void mfma_load_tiles(const GemmDesc& d, const GemmStrides& st,
                                                 const TA* Ab, const TB* Bb, int m0, int n0, int k0,
@@ -165,12 +175,13 @@ template <int ROLE, typename T, int TM, int TN, typename TA, typename TB, typena
 __global__ __launch_bounds__(256) void k_gemm_mfma(const TA* __restrict__ A, const TB* __restrict__ B,
                                                    TC* __restrict__ C,
                                                    const GemmDesc* __restrict__ descs,
+                                                   const GemmBlk* __restrict__ blks,
                                                    GemmStrides st, KinParams kp) {
   typedef MfmaAcc<T> M;
   constexpr int BMt = 32 * TM, BNt = 32 * TN;
-  const GemmDesc d = descs[blockIdx.z];
-  const int m0 = blockIdx.y * BMt, n0 = blockIdx.x * BNt;
-  if (m0 >= d.M || n0 >= d.N) return;
+  const GemmBlk bk = blks[gemm_block()];
+  const GemmDesc d = descs[bk.z];
+  const int m0 = bk.m0, n0 = bk.n0;
   __shared__ T As[BK][BMt + 4];
   __shared__ T Bs[BK][BNt + 4];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -184,8 +195,8 @@ __global__ __launch_bounds__(256) void k_gemm_mfma(const TA* __restrict__ A, con
   const TA* Ab = A + d.a_off;
   const TB* Bb = B + d.b_off;
   T ra[2 * TM], rb[2 * TN];
-  mfma_load_tiles<T, TM, TN>(d, st, Ab, Bb, m0, n0, 0, amf, bnf, ra, rb);
-  for (int k0 = 0; k0 < d.K; k0 += BK) {
+  mfma_load_tiles<T, TM, TN>(d, st, Ab, Bb, m0, n0, bk.k0, amf, bnf, ra, rb);
+  for (int k0 = bk.k0; k0 < bk.k1; k0 += BK) {
 #pragma unroll
     for (int l = 0; l < 2 * TM; l++) {
       int mm, kk;
@@ -199,7 +210,7 @@ __global__ __launch_bounds__(256) void k_gemm_mfma(const TA* __restrict__ A, con
       Bs[kk][nn] = rb[l];
     }
     __syncthreads();
-    if (k0 + BK < d.K) mfma_load_tiles<T, TM, TN>(d, st, Ab, Bb, m0, n0, k0 + BK, amf, bnf, ra, rb);
+    if (k0 + BK < bk.k1) mfma_load_tiles<T, TM, TN>(d, st, Ab, Bb, m0, n0, k0 + BK, amf, bnf, ra, rb);
 #pragma unroll
     for (int kk = 0; kk < BK; kk += 4) {
       const int kr = kk + (lane >> 4), c16 = lane & 15;
@@ -319,51 +330,20 @@ struct RoleAKC {
   static constexpr bool value = ROLE == G_DST_R || ROLE == G_DST_R_INV || ROLE == G_ANG_BWD;
 };
 
-// Block -> tile order.  Workgroups go to the 8 XCDs round robin by linear
-// id, each XCD with its own L2; hardware id hw is mapped to a logical id so
-// that each XCD runs one contiguous run of logical ids, and the logical order
-// puts the blocks that read the same operand panel next to each other:
-//   share_b = 0 (A panel shared: same descriptor group, same M tile)
-//           order [z / group][y][z % group][x];
-//   share_b = 1 (B panel shared: same descriptor, same N tile)
-//           order [z][x][y].
-struct GemmGrid {
-  int gx, gy, group, share_b;
-};
-
-__device__ __forceinline__ void gemm_block(const GemmGrid& g, int& x, int& y, int& z) {
-  const int hw = blockIdx.x, q = (int)(gridDim.x >> 3);
-  const int l = hw < 8 * q ? (hw & 7) * q + (hw >> 3) : hw;
-  if (g.share_b) {
-    y = l % g.gy;
-    const int t = l / g.gy;
-    x = t % g.gx;
-    z = t / g.gx;
-  } else {
-    x = l % g.gx;
-    int t = l / g.gx;
-    const int zg = t % g.group;
-    t /= g.group;
-    y = t % g.gy;
-    z = (t / g.gy) * g.group + zg;
-  }
-}
-
 template <int ROLE, typename T, int TM, int TN, typename TA, typename TB, typename TC>
 __global__ __launch_bounds__(256) void k_gemm_vec(const TA* __restrict__ A, const TB* __restrict__ B,
                                                   TC* __restrict__ C,
                                                   const GemmDesc* __restrict__ descs,
-                                                  GemmStrides st, KinParams kp, GemmGrid gg) {
+                                                  const GemmBlk* __restrict__ blks,
+                                                  GemmStrides st, KinParams kp) {
   typedef MfmaAcc<T> M;
   constexpr bool AKC = RoleAKC<ROLE>::value;
   constexpr int BMt = 32 * TM, BNt = 32 * TN;
   constexpr int LA = AKC ? BK + 4 : BMt + 4;  // LDS row length of A (K-major or M-major)
   constexpr int LB = BNt + 4;
-  int bx, by, bz;
-  gemm_block(gg, bx, by, bz);
-  const GemmDesc d = descs[bz];
-  const int m0 = by * BMt, n0 = bx * BNt;
-  if (m0 >= d.M || n0 >= d.N) return;
+  const GemmBlk bk = blks[gemm_block()];
+  const GemmDesc d = descs[bk.z];
+  const int m0 = bk.m0, n0 = bk.n0;
   __shared__ __align__(16) T As[AKC ? BMt * LA : BK * LA];
   __shared__ __align__(16) T Bs[BK * LB];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -395,8 +375,8 @@ __global__ __launch_bounds__(256) void k_gemm_vec(const TA* __restrict__ A, cons
                d.fold_sgn, rb[l]);
     }
   };
-  load(0);
-  for (int k0 = 0; k0 < d.K; k0 += BK) {
+  load(bk.k0);
+  for (int k0 = bk.k0; k0 < bk.k1; k0 += BK) {
 #pragma unroll
     for (int l = 0; l < TM / 2; l++) {
       const int v = threadIdx.x + 256 * l;
@@ -411,7 +391,7 @@ __global__ __launch_bounds__(256) void k_gemm_vec(const TA* __restrict__ A, cons
       st4(&Bs[(v / (8 * TN)) * LB + 4 * (v % (8 * TN))], rb[l]);
     }
     __syncthreads();
-    if (k0 + BK < d.K) load(k0 + BK);
+    if (k0 + BK < bk.k1) load(k0 + BK);
     T av[TM][4], bv[TN][4];
 #pragma unroll
     for (int a = 0; a < TM; a++) {
@@ -478,27 +458,16 @@ __global__ __launch_bounds__(256) void k_gemm_vec(const TA* __restrict__ A, cons
       }
 }
 
-template <int ROLE, int TM, int TN, typename TACC, typename TA, typename TB, typename TC>
-static void launch_gemm_vec(hipStream_t s, const TA* A, const TB* B, TC* C, const GemmPlan& p,
-                            KinParams kp) {
-  GemmGrid gg{(p.maxN + 32 * TN - 1) / (32 * TN), (p.maxM + 32 * TM - 1) / (32 * TM), p.group,
-              p.share_b};
-  const unsigned nblk = (unsigned)gg.gx * (unsigned)gg.gy * (unsigned)p.nb;
-  hipLaunchKernelGGL((k_gemm_vec<ROLE, TACC, TM, TN, TA, TB, TC>), dim3(nblk), dim3(256), 0, s, A,
-                     B, C, p.d_descs, p.st, kp, gg);
-}
-
 template <int ROLE, typename TA, typename TB, typename TC, typename TACC>
 static hipError_t run_gemm(hipStream_t s, const TA* A, const TB* B, TC* C, const GemmPlan& p,
                            KinParams kp = KinParams{}) {
-  if (p.nb == 0 || p.maxM == 0 || p.maxN == 0) return hipSuccess;  // nothing to write
-  if (!p.vec) {
-    dim3 grid((p.maxN + 63) / 64, (p.maxM + 63) / 64, p.nb);
-    hipLaunchKernelGGL((k_gemm_mfma<ROLE, TACC, 2, 2, TA, TB, TC>), grid, dim3(256), 0, s, A, B, C,
-                       p.d_descs, p.st, kp);
-    return hipGetLastError();
-  }
-  launch_gemm_vec<ROLE, 2, 2, TACC>(s, A, B, C, p, kp);
+  if (p.nblk == 0) return hipSuccess;  // nothing to write
+  if (p.vec)
+    hipLaunchKernelGGL((k_gemm_vec<ROLE, TACC, 2, 2, TA, TB, TC>), dim3(p.nblk), dim3(256), 0, s, A,
+                       B, C, p.d_descs, p.d_blks, p.st, kp);
+  else
+    hipLaunchKernelGGL((k_gemm_mfma<ROLE, TACC, 2, 2, TA, TB, TC>), dim3(p.nblk), dim3(256), 0, s, A,
+                       B, C, p.d_descs, p.d_blks, p.st, kp);
   return hipGetLastError();
 }
 
@@ -603,7 +572,8 @@ __global__ __launch_bounds__(FBR_THREADS) void k_fbr_coef_all(const T* __restric
                                                       T* __restrict__ phi,
                                                       const double* __restrict__ acoef,
                                                       const double* __restrict__ bcoef,
-                                                      const int32_t* __restrict__ nbr, int nJ,
+                                                      const int32_t* __restrict__ nbr,
+                                                      const int32_t* __restrict__ rng, int nJ,
                                                       int n1, int n2) {
   const int nrc = (n1 + FBR_RB - 1) / FBR_RB;
   const int jj = blockIdx.x / nrc, rc = blockIdx.x - jj * nrc;
@@ -621,6 +591,7 @@ __global__ __launch_bounds__(FBR_THREADS) void k_fbr_coef_all(const T* __restric
     const T* fb = fbr + (int64_t)jj * plane + R;
     T* ob = phi + (int64_t)jj * plane + R;
     for (int r = r0; r < r1; r++) {
+      if (R < rng[2 * r] || R >= rng[2 * r + 1]) continue;  // not read further on
       double f[NC];
 #pragma unroll
       for (int t = 0; t < NC; t++) {
@@ -1019,17 +990,73 @@ hipError_t launch_gather_a0(Ctx* c, const double* dense, double* a0) {
 // ---------------------------------------------------------------------------
 static bool plan_vec_ok(const std::vector<GemmDesc>& ds, const GemmStrides& st, bool akc);
 
-static hipError_t upload_plan(GemmPlan* p, const std::vector<GemmDesc>& d, bool akc) {
-  p->vec = plan_vec_ok(d, p->st, akc) ? 1 : 0;
-  p->nb = (int)d.size();
-  p->maxM = p->maxN = 0;
-  for (auto& x : d) {
-    p->maxM = std::max(p->maxM, x.M);
-    p->maxN = std::max(p->maxN, x.N);
+// what a block needs: false if nothing reads its results, else its range of k
+// (*k0, *k1 are the whole range on entry)
+typedef std::function<bool(int z, int m0, int n0, int* k0, int* k1)> GemmNeed;
+
+// The list of a plan's 64 x 64 blocks, in the order
+//   share_b = 0 (A panel shared: same descriptor group, same M tile)
+//           [z / group][m][z % group][n];
+//   share_b = 1 (B panel shared: same descriptor, same N tile)
+//           [z][n][m].
+// psi is zero off the kept points and only kept points are read of a term, so
+// blocks with no kept result are left out, and products start and end at the
+// first and last k whose operand may differ from zero (whole steps of BK, so
+// that the remaining terms add up in the same order).  A mixed step, all of it
+// GEMMs, on the 256 x 256 x 140 grid of a 20 angstrom box (7.8% of the points
+// kept): 222 -> 126 us.  An FP64 step with seven helicity blocks, 192 x 384 x 96
+// (35% kept), its angular term as GEMMs: 1017 -> 740 us, the coefficient pass
+// between them limited to the kept R of each row likewise.
+static std::vector<GemmBlk> plan_blocks(const std::vector<GemmDesc>& d, int group, int share_b,
+                                        const GemmNeed& need) {
+  std::vector<GemmBlk> out;
+  auto add = [&](int z, int m, int n) {
+    const GemmDesc& g = d[z];
+    if (64 * m >= g.M || 64 * n >= g.N) return;
+    GemmBlk b{z, 64 * m, 64 * n, 0, g.K};
+    if (need && !need(z, b.m0, b.n0, &b.k0, &b.k1)) return;
+    b.k0 = std::max(b.k0, 0) / BK * BK;
+    b.k1 = std::min((b.k1 + BK - 1) / BK * BK, g.K);
+    if (b.k1 <= b.k0) b.k0 = b.k1 = 0;
+    out.push_back(b);
+  };
+  auto tiles = [](int x) { return (x + 63) / 64; };
+  if (share_b) {
+    for (int z = 0; z < (int)d.size(); z++)
+      for (int n = 0; n < tiles(d[z].N); n++)
+        for (int m = 0; m < tiles(d[z].M); m++) add(z, m, n);
+    return out;
   }
-  hipError_t e = hipMalloc(&p->d_descs, sizeof(GemmDesc) * d.size());
-  if (e != hipSuccess) return e;
-  return hipMemcpy(p->d_descs, d.data(), sizeof(GemmDesc) * d.size(), hipMemcpyHostToDevice);
+  for (int z0 = 0; z0 < (int)d.size(); z0 += group) {
+    const int z1 = std::min(z0 + group, (int)d.size());
+    int maxM = 0;
+    for (int z = z0; z < z1; z++) maxM = std::max(maxM, d[z].M);
+    for (int m = 0; m < tiles(maxM); m++)
+      for (int z = z0; z < z1; z++)
+        for (int n = 0; n < tiles(d[z].N); n++) add(z, m, n);
+  }
+  return out;
+}
+
+void free_plan(GemmPlan* p) {
+  if (p->d_descs) (void)hipFree(p->d_descs);
+  if (p->d_blks) (void)hipFree(p->d_blks);
+  p->d_descs = nullptr;
+  p->d_blks = nullptr;
+}
+
+static hipError_t upload_plan(GemmPlan* p, const std::vector<GemmDesc>& d, bool akc,
+                              const GemmNeed& need = nullptr) {
+  p->vec = plan_vec_ok(d, p->st, akc) ? 1 : 0;
+  const std::vector<GemmBlk> b = plan_blocks(d, p->group, p->share_b, need);
+  p->nblk = (int)b.size();
+  hipError_t e = hipMalloc(&p->d_descs, sizeof(GemmDesc) * std::max<size_t>(d.size(), 1));
+  if (e == hipSuccess)
+    e = hipMemcpy(p->d_descs, d.data(), sizeof(GemmDesc) * d.size(), hipMemcpyHostToDevice);
+  if (e == hipSuccess) e = hipMalloc(&p->d_blks, sizeof(GemmBlk) * std::max<size_t>(b.size(), 1));
+  if (e == hipSuccess)
+    e = hipMemcpy(p->d_blks, b.data(), sizeof(GemmBlk) * b.size(), hipMemcpyHostToDevice);
+  return e;
 }
 
 // whether every descriptor of a plan meets the vector kernel's alignment
@@ -3315,6 +3342,37 @@ hipError_t build_plans(Ctx* c) {
     while (t.dst_sizes[q] != n) q++;
     return q;
   };
+  plan_tiles(c);
+  // kept points: R range of each (angle, r row), and whether an angle has any in
+  // each run of 64 plane points
+  std::vector<int> rlo((size_t)t.na * t.n1, t.n2), rhi((size_t)t.na * t.n1, 0);
+  const int npt = (int)((plane + 63) / 64);
+  std::vector<uint8_t> pt((size_t)t.na * npt, 0);
+  std::vector<int32_t> rng(2 * (size_t)t.n1, 0);
+  for (int r = 0; r < t.n1; r++) rng[2 * r] = t.n2;
+  for (int ia = 0; ia < t.na; ia++)
+    for (int r = 0; r < t.n1; r++)
+      for (int R = 0; R < t.n2; R++)
+        if (t.mask[(size_t)ia * plane + (size_t)r * t.n2 + R]) {
+          int& lo = rlo[(size_t)ia * t.n1 + r];
+          lo = std::min(lo, R);
+          rhi[(size_t)ia * t.n1 + r] = R + 1;
+          rng[2 * r] = std::min(rng[2 * r], R);
+          rng[2 * r + 1] = std::max(rng[2 * r + 1], R + 1);
+          pt[(size_t)ia * npt + ((size_t)r * t.n2 + R) / 64] = 1;
+        }
+  if ((e = hipMalloc(&c->d_fbr_rng, sizeof(int32_t) * rng.size())) != hipSuccess) return e;
+  if ((e = hipMemcpy(c->d_fbr_rng, rng.data(), sizeof(int32_t) * rng.size(),
+                     hipMemcpyHostToDevice)) != hipSuccess)
+    return e;
+  // kept range [lo, hi) of a folded axis of n: x and n - 1 - x are one element
+  auto fold = [](int n, int lo, int hi, int* j0, int* j1) {
+    const int last = hi - 1, ke = n - n / 2;
+    *j0 = std::min(*j0, std::min(lo, n - 1 - last));
+    *j1 = std::max(*j1, lo < ke && last >= n / 2 ? ke
+                                                : std::max(std::min(lo, n - 1 - lo),
+                                                           std::min(last, n - 1 - last)) + 1);
+  };
   // Radial kinetic as c psi - S (c - E)_+ divi S psi on the low modes
   // k1 < k1lo(ia), k2 < k2lo(ia) (see the low-mode tables in mw3_setup.cpp).
   // (1) R rows, folded: t1[r][k2] = sum_R S(R, k2) psi[r][R], k2 < k2lo, r < nn1
@@ -3342,7 +3400,19 @@ hipError_t build_plans(Ctx* c) {
           d.push_back(g);
         }
     c->p_dstR.st = GemmStrides{kp, 1, n, 2};
-    if ((e = upload_plan(&c->p_dstR, d, true)) != hipSuccess) return e;
+    // (every row is written: pass 2 folds rows onto each other)
+    auto need = [&](int z, int m0, int, int* k0, int* k1) {
+      const int ia = z / 2 % t.na;
+      int j0 = ke, j1 = 0;
+      for (int r = m0; r < std::min(m0 + 64, t.nn1[ia]); r++) {
+        const size_t q = (size_t)ia * t.n1 + r;
+        if (rhi[q]) fold(n, rlo[q], rhi[q], &j0, &j1);
+      }
+      *k0 = j0;
+      *k1 = std::min(*k1, j1);
+      return true;
+    };
+    if ((e = upload_plan(&c->p_dstR, d, true, need)) != hipSuccess) return e;
   }
   // (2) r columns, folded, times (c - E)_+ divi:
   //     t2[k1][k2] = f(k1, k2) sum_r S(r, k1) t1[r][k2], k1 < k1lo
@@ -3376,7 +3446,16 @@ hipError_t build_plans(Ctx* c) {
         }
       }
     c->p_dstr.st = GemmStrides{t.n2, 1, 2 * (int64_t)t.n2, 1};
-    if ((e = upload_plan(&c->p_dstr, d, false)) != hipSuccess) return e;
+    auto need = [&](int z, int, int, int* k0, int* k1) {
+      const int ia = z / 2 % t.na, n = t.nn1[ia];
+      int j0 = n, j1 = 0;
+      for (int r = 0; r < n; r++)
+        if (rhi[(size_t)ia * t.n1 + r]) fold(n, r, r + 1, &j0, &j1);
+      *k0 = j0;
+      *k1 = std::min(*k1, j1);
+      return true;
+    };
+    if ((e = upload_plan(&c->p_dstr, d, false, need)) != hipSuccess) return e;
   }
   // (3) back over r: t1[r][k2] = sum_{k1 < k1lo} S(r, k1) t2[k1][k2], r < nn1
   {
@@ -3396,7 +3475,13 @@ hipError_t build_plans(Ctx* c) {
         d.push_back(g);
       }
     c->p_dstr2.st = GemmStrides{t.n2, 1, t.n2, 1};
-    if ((e = upload_plan(&c->p_dstr2, d, false)) != hipSuccess) return e;
+    auto need = [&](int z, int m0, int, int*, int*) {
+      const int ia = z % t.na;
+      for (int r = m0; r < std::min(m0 + 64, t.nn1[ia]); r++)
+        if (rhi[(size_t)ia * t.n1 + r]) return true;
+      return false;
+    };
+    if ((e = upload_plan(&c->p_dstr2, d, false, need)) != hipSuccess) return e;
   }
   // (4) back over R: t2[r][R] = sum_{k2 < k2lo} t1[r][k2] S(k2, R) (the
   //     correction subtracted from c psi by the update)
@@ -3417,7 +3502,15 @@ hipError_t build_plans(Ctx* c) {
         d.push_back(g);
       }
     c->p_dstRi.st = GemmStrides{t.low_ld[q], 1, t.n2, 1};
-    if ((e = upload_plan(&c->p_dstRi, d, true)) != hipSuccess) return e;
+    auto need = [&](int z, int m0, int n0, int*, int*) {
+      const int ia = z % t.na;
+      for (int r = m0; r < std::min(m0 + 64, t.nn1[ia]); r++) {
+        const size_t q = (size_t)ia * t.n1 + r;
+        if (rlo[q] < n0 + 64 && rhi[q] > n0) return true;
+      }
+      return false;
+    };
+    if ((e = upload_plan(&c->p_dstRi, d, true, need)) != hipSuccess) return e;
   }
   // angular forward: fbr[c][jj][p] = sum_ia D_c(ia, jj) psi[c][ia][p]; with no
   // Coriolis neighbour in any channel the coefficients go into its epilogue
@@ -3443,7 +3536,18 @@ hipError_t build_plans(Ctx* c) {
       d.push_back(g);
     }
     c->p_angF.st = GemmStrides{plane, 1, plane, 1};
-    if ((e = upload_plan(&c->p_angF, d, false)) != hipSuccess) return e;
+    auto need = [&](int, int, int n0, int* k0, int* k1) {
+      int j0 = t.na, j1 = 0;
+      for (int ia = 0; ia < t.na; ia++)
+        if (pt[(size_t)ia * npt + n0 / 64]) {
+          j0 = std::min(j0, ia);
+          j1 = ia + 1;
+        }
+      *k0 = j0;
+      *k1 = j1;
+      return j1 > 0;
+    };
+    if ((e = upload_plan(&c->p_angF, d, false, need)) != hipSuccess) return e;
   }
   // angular back: ang[c][ia][p] = sum_jj D_c(ia, jj) phi[c][jj][p]
   {
@@ -3461,9 +3565,13 @@ hipError_t build_plans(Ctx* c) {
       d.push_back(g);
     }
     c->p_angB.st = GemmStrides{plane, 1, plane, 1};
-    if ((e = upload_plan(&c->p_angB, d, true)) != hipSuccess) return e;
+    auto need = [&](int, int m0, int n0, int*, int*) {
+      for (int ia = m0; ia < std::min(m0 + 64, t.na); ia++)
+        if (pt[(size_t)ia * npt + n0 / 64]) return true;
+      return false;
+    };
+    if ((e = upload_plan(&c->p_angB, d, true, need)) != hipSuccess) return e;
   }
-  plan_tiles(c);
   // strips, tiles and (FP64) radial tables of the update
   e = c->precision == MW3_MIXED ? step_build_f32(c) : step_build_f64(c);
   if (e != hipSuccess) return e;
@@ -3605,14 +3713,9 @@ hipError_t build_plans(Ctx* c) {
 }
 
 void free_plans(Ctx* c) {
-
   GemmPlan* ps[7] = {&c->p_dstR, &c->p_dstr, &c->p_dstr2, &c->p_dstRi, &c->p_angF, &c->p_angB,
                      &c->p_prod};
-  for (auto* p : ps)
-    if (p->d_descs) {
-      (void)hipFree(p->d_descs);
-      p->d_descs = nullptr;
-    }
+  for (auto* p : ps) free_plan(p);
 }
 
 // H psi terms into work slabs: d_t2 = T psi (rows r < nn1), d_ang = angular
@@ -3749,7 +3852,7 @@ static hipError_t angular_impl(Ctx* c, const T* psi, hipStream_t s) {
   case NC:                                                                                       \
     hipLaunchKernelGGL((k_fbr_coef_all<T, NC>), dim3(nall), dim3(FBR_THREADS), 0, s,            \
                        (const T*)c->d_fbr, (T*)c->d_phi, (const double*)c->d_acoef,             \
-                       (const double*)c->d_bcoef, c->d_nbr, t.nJ, t.n1, t.n2);                  \
+                       (const double*)c->d_bcoef, c->d_nbr, c->d_fbr_rng, t.nJ, t.n1, t.n2);    \
     break;
       MW3_FBR(2)
       MW3_FBR(3)
