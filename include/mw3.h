@@ -309,8 +309,8 @@ MW3_API int32_t mw3_cheby_spectrum(const double *autoc, int32_t kmax, double emi
                    the two r passes); 0: as batched GEMMs.
    MW3_OPT_ANGULAR 0 (default): the angular term by the parity-folded
                    one-pass kernel (with Coriolis-coupled channels, in
-                   MW3_MIXED with FP16 products: its forward and back parts
-                   around the coefficient pass); 1: the unfolded one-pass
+                   MW3_FP64 or with FP16 products: its forward and back parts
+                   around the coefficients); 1: the unfolded one-pass
                    kernel; 2: two GEMMs with the FBR coefficients between
                    them.  A variant
                    not built for the context falls back to the next one.

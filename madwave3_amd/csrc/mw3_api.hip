@@ -1097,7 +1097,7 @@ static void effective_options(const Ctx* c, int32_t* out) {
   out[MW3_OPT_GRAPHS] = c->graph_mode;
   out[MW3_OPT_RADIAL] = c->opt_radial && (c->up_nk1 || c->rad_nitems || c->mid_nitems) ? 1 : 0;
   int a = c->opt_angular;
-  const bool cor_fold = c->ang_fold_cor && c->precision == MW3_MIXED && c->opt_fp16;
+  const bool cor_fold = c->ang_fold_cor && (c->precision == MW3_FP64 || c->opt_fp16);
   if (a == 0 && !c->ang_fold && !cor_fold) a = 1;
   if (a == 1 && !c->ang_nt && !c->ang_fold) a = 2;
   if (a == 1 && !c->ang_nt) a = 0;

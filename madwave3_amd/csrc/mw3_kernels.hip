@@ -21,6 +21,7 @@
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
+#include <cstring>
 #include <functional>
 
 #include "mw3_step.h"
@@ -1371,24 +1372,35 @@ __global__ __launch_bounds__(64 * ANG_WAVES) void k_ang_fused(
 // partial round go one per block before any block takes a second, and the
 // waves of one SIMD differ by at most one group.
 // ---------------------------------------------------------------------------
+// With Coriolis-coupled channels (FP64) the products run apart, the coefficient
+// pass between them: PART 1 writes F to the FBR slab's rows of its functions
+// (jmap: function at each class-order position, -1 for padding), PART 2 reads G
+// there.  Bound by those slabs (0.24 GB each at 7 channels of 192 x 384 x 96);
+// the 64 x 64 GEMM blocks they replace multiplied both classes and the padding
+// of rows 96 to 127: 250 steps there 217.9 -> 194.3 ms.
 // FP32: at most 128 VGPRs (4 waves per SIMD), so that two blocks share a CU
-template <typename T, int NT>
+template <typename T, int NT, int PART = 0>
 __global__ __launch_bounds__(64 * ANG_WAVES, sizeof(T) == 4 ? 4 : 1) void k_ang_fold(
     const T* __restrict__ psi, const T* __restrict__ Dfold, const T* __restrict__ afold,
     const T* __restrict__ bfold, T* __restrict__ ang, const int32_t* __restrict__ groups,
-    int ngroups, int nbc, int na, int n1, int n2) {
+    int ngroups, int nbc, int na, int n1, int n2, T* __restrict__ fbr,
+    const int32_t* __restrict__ jmap, int nJ) {
   typedef MfmaAcc<T> M;
   typedef typename M::V V;
   constexpr int NR = 16 * NT, NC2 = 2 * NR;    // rows (ia < h) and columns (both classes)
   constexpr int P = NC2 + AngPitch<T>::extra;  // LDS row pitch
   constexpr int XA = 2;                        // psi chunks loaded ahead of the MFMAs
   __shared__ __align__(16) T Ds[NR * P];
+  __shared__ int32_t jms[PART ? NC2 : 1];
   const int pl = n1 * n2, h = na >> 1;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int g = lane >> 4, i = lane & 15;
   const int ch = blockIdx.x / nbc, bl = blockIdx.x - ch * nbc;
   const int stride = nbc * ANG_WAVES;
   const char* pb = (const char*)(psi + (int64_t)ch * na * pl);
+  char* const fb = PART ? (char*)(fbr + (int64_t)ch * nJ * pl) : nullptr;
+  if constexpr (PART != 0)
+    for (int v = threadIdx.x; v < NC2; v += 64 * ANG_WAVES) jms[v] = jmap[ch * NC2 + v];
   // xl[4 c + s] = psi[16 c + 4 g + s][p], xh[..] = psi[na-1-(16 c + 4 g + s)][p];
   // angles past h read angle h-1 and its mirror (finite), against zero rows of D
   T xl[4 * NT], xh[4 * NT];
@@ -1409,7 +1421,7 @@ __global__ __launch_bounds__(64 * ANG_WAVES, sizeof(T) == 4 ? 4 : 1) void k_ang_
   // psi loads go out before the D image's, so that the two latencies overlap
   int gi = 2 * (bl + nbc * (wave >> 1)) + (wave & 1);
   const bool busy = gi < ngroups;
-  if (busy) {
+  if (PART != 2 && busy) {
 #pragma unroll
     for (int c = 0; c < XA && c < NT; c++) ldx(c, 16 * groups[gi]);
   }
@@ -1440,6 +1452,22 @@ __global__ __launch_bounds__(64 * ANG_WAVES, sizeof(T) == 4 ? 4 : 1) void k_ang_
   const char* ac = (const char*)(afold + (int64_t)ch * NC2 * n1);
   const char* bc = (const char*)(bfold + (int64_t)ch * NC2 * n2);
   char* ob = (char*)(ang + (int64_t)ch * na * pl);
+  // PART 2: a group's G, zero at the padding of the class order
+  T gv[2 * NT][4];
+  auto ldg = [&](int col0) {
+    int pp = col0 + lane_opaque(i);
+    pp = pp < pl ? pp : pl - 1;
+    const int ll = lane_opaque(lane);
+#pragma unroll
+    for (int t = 0; t < 2 * NT; t++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        const int j = jms[16 * t + M::row(ll, r)];
+        const T x = *(const T*)(fb + (uint32_t)((j >= 0 ? j : 0) * pl + pp) * (uint32_t)sizeof(T));
+        gv[t][r] = j >= 0 ? x : (T)0;
+      }
+  };
+  if constexpr (PART == 2) ldg(16 * groups[gi]);
   for (; gi < ngroups; gi += stride) {
     const int col = 16 * groups[gi];
     const int cnext = 16 * groups[gi + stride < ngroups ? gi + stride : gi];
@@ -1459,6 +1487,11 @@ __global__ __launch_bounds__(64 * ANG_WAVES, sizeof(T) == 4 ? 4 : 1) void k_ang_
     // forward products: f[t] (t < NT) the s = +1 rows from u, f[NT + t] the
     // s = -1 rows from v
     V f[2 * NT];
+    if constexpr (PART == 2) {
+#pragma unroll
+      for (int t = 0; t < 2 * NT; t++) f[t] = (V){gv[t][0], gv[t][1], gv[t][2], gv[t][3]};
+      ldg(cnext);  // in flight during this group
+    } else {
 #pragma unroll
     for (int t = 0; t < 2 * NT; t++) f[t] = (V){0, 0, 0, 0};
     T a1[2][2 * NT];
@@ -1472,8 +1505,8 @@ __global__ __launch_bounds__(64 * ANG_WAVES, sizeof(T) == 4 ? 4 : 1) void k_ang_
     for (int k = 0; k < 4 * NT; k++) {
       if (k + 1 < 4 * NT) rd1(k + 1, a1[(k + 1) & 1]);
       if ((k & 3) == 0 && (k >> 2) + XA < NT) ldx((k >> 2) + XA, col);
-      if (k == (NT > 1 ? 4 * NT - 8 : 0)) ldcoef(0, ca[0], cb[0]);
-      if (k == 4 * NT - 4) ldcoef(1, ca[1], cb[1]);
+      if (PART == 0 && k == (NT > 1 ? 4 * NT - 8 : 0)) ldcoef(0, ca[0], cb[0]);
+      if (PART == 0 && k == 4 * NT - 4) ldcoef(1, ca[1], cb[1]);
       __builtin_amdgcn_sched_barrier(0);
       const T u = xl[k] + xh[k], v = xl[k] - xh[k];
 #pragma unroll
@@ -1482,15 +1515,31 @@ __global__ __launch_bounds__(64 * ANG_WAVES, sizeof(T) == 4 ? 4 : 1) void k_ang_
       for (int t = NT; t < 2 * NT; t++) f[t] = M::mma(a1[k & 1][t], v, f[t]);
       __builtin_amdgcn_sched_barrier(0);
     }
+    }
+    if constexpr (PART == 1) {
+#pragma unroll
+      for (int c = 0; c < XA && c < NT; c++) ldx(c, cnext);
+      const int ll = lane_opaque(lane), pp = lane_opaque(p);
+#pragma unroll
+      for (int t = 0; t < 2 * NT; t++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+          const int j = jms[16 * t + M::row(ll, r)];
+          if (j >= 0 && pp < pl)
+            *(T*)(fb + (uint32_t)(j * pl + pp) * (uint32_t)sizeof(T)) = f[t][r];
+        }
+      continue;
+    }
     // back products: row tile t of F (class t / NT), scaled by its
     // coefficients, feeds the class's NT output tiles o[(t / NT) NT + u];
     // stage (t, u) reads a[r] = D(16 u + i, 16 t + row(lane, r)) two stages
     // ahead, and halfway through row tile t the VALU scales row tile t + 1
     constexpr int NQ = 2 * NT * NT;
     auto scale = [&](int t) {
+      if constexpr (PART == 0) {
 #pragma unroll
-      for (int r = 0; r < 4; r++)
-        f[t][r] = f[t][r] * (ca[t & 1][r] + cb[t & 1][r]);
+        for (int r = 0; r < 4; r++) f[t][r] = f[t][r] * (ca[t & 1][r] + cb[t & 1][r]);
+      }
     };
     V o[2 * NT];
 #pragma unroll
@@ -1521,8 +1570,8 @@ __global__ __launch_bounds__(64 * ANG_WAVES, sizeof(T) == 4 ? 4 : 1) void k_ang_
           const int q = t * NT + u;
           if (q + 2 < NQ) rd2(q + 2, a4[(q + 2) % 4]);
           if (q + 3 < NQ) rd2(q + 3, a4[(q + 3) % 4]);
-          if (u == 0 && t + 2 < 2 * NT) ldcoef(t + 2, ca[t & 1], cb[t & 1]);
-          if (u == 0 && t == NT) {
+          if (PART == 0 && u == 0 && t + 2 < 2 * NT) ldcoef(t + 2, ca[t & 1], cb[t & 1]);
+          if (PART == 0 && u == 0 && t == NT) {
 #pragma unroll
             for (int c = 0; c < XA && c < NT; c++) ldx(c, cnext);
           }
@@ -1547,8 +1596,8 @@ __global__ __launch_bounds__(64 * ANG_WAVES, sizeof(T) == 4 ? 4 : 1) void k_ang_
         for (int u = 0; u < NT; u++) {
           const int q = t * NT + u;
           if (q + 2 < NQ) rd2(q + 2, a2[(q + 2) % 3]);
-          if (u == 0 && t + 2 < 2 * NT) ldcoef(t + 2, ca[t & 1], cb[t & 1]);
-          if (u == 0 && t == NT) {
+          if (PART == 0 && u == 0 && t + 2 < 2 * NT) ldcoef(t + 2, ca[t & 1], cb[t & 1]);
+          if (PART == 0 && u == 0 && t == NT) {
 #pragma unroll
             for (int c = 0; c < XA && c < NT; c++) ldx(c, cnext);
           }
@@ -2029,7 +2078,7 @@ static void launch_ang_fold_nt(Ctx* c, const T* psi, hipStream_t st) {
   hipLaunchKernelGGL((k_ang_fold<T, NT>), dim3((unsigned)(nbc * t.nc)), dim3(64 * ANG_WAVES), 0,
                      st, psi, (const T*)c->d_fold_D, (const T*)c->d_fold_a,
                      (const T*)c->d_fold_b, (T*)c->d_ang, c->d_ang_groups, c->ang_ngroups, nbc,
-                     t.na, t.n1, t.n2);
+                     t.na, t.n1, t.n2, (T*)nullptr, (const int32_t*)nullptr, t.nJ);
 }
 
 template <typename T>
@@ -2065,14 +2114,48 @@ static hipError_t ang_cor_grid(Ctx* c) {
   return ang_fold_grid_k(k_ang_fold_h<NT, 3>, c->t.nc, c->ang_ngroups, &c->ang_cor_nbc[2]);
 }
 
+// FP64: parts 1 and 2, with the coefficient pass between them
+template <int NT>
+static hipError_t ang_cor64_grid(Ctx* c) {
+  hipError_t e =
+      ang_fold_grid_k(k_ang_fold<double, NT, 1>, c->t.nc, c->ang_ngroups, &c->ang_cor_nbc[0]);
+  if (e != hipSuccess) return e;
+  return ang_fold_grid_k(k_ang_fold<double, NT, 2>, c->t.nc, c->ang_ngroups, &c->ang_cor_nbc[1]);
+}
+
 static hipError_t ang_cor_setup(Ctx* c, int nt) {
+  const bool m = c->precision == MW3_MIXED;
   switch (nt) {
-    case 1: return ang_cor_grid<1>(c);
-    case 2: return ang_cor_grid<2>(c);
-    case 3: return ang_cor_grid<3>(c);
-    case 4: return ang_cor_grid<4>(c);
+    case 1: return m ? ang_cor_grid<1>(c) : ang_cor64_grid<1>(c);
+    case 2: return m ? ang_cor_grid<2>(c) : ang_cor64_grid<2>(c);
+    case 3: return m ? ang_cor_grid<3>(c) : ang_cor64_grid<3>(c);
+    case 4: return m ? ang_cor_grid<4>(c) : ang_cor64_grid<4>(c);
     default: return hipErrorInvalidValue;
   }
+}
+
+template <int NT, int PART>
+static void launch_ang_cor64_nt(Ctx* c, const double* psi, hipStream_t st) {
+  const HostTables& t = c->t;
+  const int gdiv = c->opt_ang_grid > 0 ? c->opt_ang_grid : 1;
+  const int nbc = std::max(1, c->ang_cor_nbc[PART - 1] / gdiv);
+  hipLaunchKernelGGL((k_ang_fold<double, NT, PART>), dim3((unsigned)(nbc * t.nc)),
+                     dim3(64 * ANG_WAVES), 0, st, psi, (const double*)c->d_fold_D,
+                     (const double*)c->d_fold_a, (const double*)c->d_fold_b, (double*)c->d_ang,
+                     c->d_ang_groups, c->ang_ngroups, nbc, t.na, t.n1, t.n2,
+                     (double*)(PART == 1 ? c->d_fbr : c->d_phi), c->d_fold_jmap, t.nJ);
+}
+
+template <int PART>
+static hipError_t launch_ang_cor64(Ctx* c, const double* psi, hipStream_t st) {
+  switch (c->ang_fold_cor) {
+    case 1: launch_ang_cor64_nt<1, PART>(c, psi, st); break;
+    case 2: launch_ang_cor64_nt<2, PART>(c, psi, st); break;
+    case 3: launch_ang_cor64_nt<3, PART>(c, psi, st); break;
+    case 4: launch_ang_cor64_nt<4, PART>(c, psi, st); break;
+    default: return hipErrorInvalidValue;
+  }
+  return hipGetLastError();
 }
 
 // part 1: psi -> F into the FBR slab (function order); part 3: the FBR slab
@@ -2130,10 +2213,12 @@ static hipError_t build_ang_fold(Ctx* c, int* nt_out) {
   const int nt = (std::max(h, std::max(nemax, nomax)) + 15) / 16;
   if (nt > 4) return hipSuccess;
   const int NR = 16 * nt, NC2 = 2 * NR;
-  std::vector<double> Df((size_t)nc * NR * NC2, 0.0), af((size_t)nc * NC2 * t.n1, 0.0),
-      bf((size_t)nc * NC2 * t.n2, 0.0);
+  // (the FP64 parts beside the Coriolis pass read no coefficients)
+  const bool coef = c->ang_fused || c->precision == MW3_MIXED;
+  const size_t ncf = coef ? (size_t)nc * NC2 : 0;
+  std::vector<double> Df((size_t)nc * NR * NC2, 0.0), af(ncf * t.n1, 0.0), bf(ncf * t.n2, 0.0);
   std::vector<int32_t> jmap((size_t)nc * NC2, -1);
-  std::vector<double> bmf((size_t)nc * NC2 * t.n2, 0.0), bpf((size_t)nc * NC2 * t.n2, 0.0);
+  std::vector<double> bmf(ncf * t.n2, 0.0), bpf(ncf * t.n2, 0.0);
   for (int ch = 0; ch < nc; ch++) {
     int slot[2] = {0, NR};
     for (int j = 0; j < nJ; j++) {
@@ -2141,6 +2226,7 @@ static hipError_t build_ang_fold(Ctx* c, int* nt_out) {
       jmap[(size_t)ch * NC2 + col] = j;
       for (int ia = 0; ia < h; ia++)
         Df[((size_t)ch * NR + ia) * NC2 + col] = t.Dmat[((size_t)ch * na + ia) * t.nJp + j];
+      if (!coef) continue;
       for (int r = 0; r < t.n1; r++)
         af[((size_t)ch * NC2 + col) * t.n1 + r] = t.acoef[((size_t)ch * nJ + j) * t.n1 + r];
       for (int R = 0; R < t.n2; R++) {
@@ -2176,10 +2262,12 @@ static hipError_t build_ang_fold(Ctx* c, int* nt_out) {
     if (err != hipSuccess) return err;
     return hipMemcpy(*dst, v.data(), v.size() * sizeof(double), hipMemcpyHostToDevice);
   };
-  if ((e = put_table(&c->d_fold_a, af)) != hipSuccess) return e;
-  if ((e = put_table(&c->d_fold_b, bf)) != hipSuccess) return e;
-  if ((e = put_table(&c->d_fold_bm, bmf)) != hipSuccess) return e;
-  if ((e = put_table(&c->d_fold_bp, bpf)) != hipSuccess) return e;
+  if (coef) {
+    if ((e = put_table(&c->d_fold_a, af)) != hipSuccess) return e;
+    if ((e = put_table(&c->d_fold_b, bf)) != hipSuccess) return e;
+    if ((e = put_table(&c->d_fold_bm, bmf)) != hipSuccess) return e;
+    if ((e = put_table(&c->d_fold_bp, bpf)) != hipSuccess) return e;
+  }
   if ((e = hipMalloc(&c->d_fold_jmap, jmap.size() * sizeof(int32_t))) != hipSuccess) return e;
   if ((e = hipMemcpy(c->d_fold_jmap, jmap.data(), jmap.size() * sizeof(int32_t),
                      hipMemcpyHostToDevice)) != hipSuccess)
@@ -3351,16 +3439,24 @@ hipError_t build_plans(Ctx* c) {
   std::vector<int32_t> rng(2 * (size_t)t.n1, 0);
   for (int r = 0; r < t.n1; r++) rng[2 * r] = t.n2;
   for (int ia = 0; ia < t.na; ia++)
-    for (int r = 0; r < t.n1; r++)
-      for (int R = 0; R < t.n2; R++)
-        if (t.mask[(size_t)ia * plane + (size_t)r * t.n2 + R]) {
-          int& lo = rlo[(size_t)ia * t.n1 + r];
-          lo = std::min(lo, R);
-          rhi[(size_t)ia * t.n1 + r] = R + 1;
-          rng[2 * r] = std::min(rng[2 * r], R);
-          rng[2 * r + 1] = std::max(rng[2 * r + 1], R + 1);
-          pt[(size_t)ia * npt + ((size_t)r * t.n2 + R) / 64] = 1;
-        }
+    for (int r = 0; r < t.n1; r++) {
+      const uint8_t* row = &t.mask[(size_t)ia * plane + (size_t)r * t.n2];
+      const void* first = memchr(row, 1, (size_t)t.n2);
+      if (!first) continue;
+      const int lo = (int)((const uint8_t*)first - row);
+      int hi = t.n2;
+      while (!row[hi - 1]) hi--;
+      rlo[(size_t)ia * t.n1 + r] = lo;
+      rhi[(size_t)ia * t.n1 + r] = hi;
+      rng[2 * r] = std::min(rng[2 * r], lo);
+      rng[2 * r + 1] = std::max(rng[2 * r + 1], hi);
+      for (int R = lo; R < hi;) {  // the parts of the row in runs of 64 points
+        const size_t q = (size_t)r * t.n2 + R;
+        const int end = std::min(hi, R + 64 - (int)(q % 64));
+        if (memchr(row + R, 1, (size_t)(end - R))) pt[(size_t)ia * npt + q / 64] = 1;
+        R = end;
+      }
+    }
   if ((e = hipMalloc(&c->d_fbr_rng, sizeof(int32_t) * rng.size())) != hipSuccess) return e;
   if ((e = hipMemcpy(c->d_fbr_rng, rng.data(), sizeof(int32_t) * rng.size(),
                      hipMemcpyHostToDevice)) != hipSuccess)
@@ -3647,8 +3743,9 @@ hipError_t build_plans(Ctx* c) {
   // some angle (the mask is the same for every channel)
   const bool tiles_fit = (plane + 16 * ANG_WAVES - 1) / (16 * ANG_WAVES) * t.nc < (1 << 24);
   if (!tiles_fit) c->ang_nt = 0;  // tile entries keep the index in 24 bits
-  // (also for the folded parts beside the Coriolis pass: mixed precision)
-  const bool cor_try = !c->ang_fused && c->precision == MW3_MIXED && offs32;
+  // (also for the folded parts beside the Coriolis pass)
+  const bool cor_try =
+      !c->ang_fused && offs32 && (c->precision == MW3_MIXED || t.nJ <= t.na);
   if (tiles_fit && (c->ang_nt || (c->ang_fused && offs32) || cor_try)) {
     const int64_t tw = 16 * ANG_WAVES, tpc = (plane + tw - 1) / tw;
     std::vector<uint8_t> act((size_t)tpc, 0);  // bit w: wave w's 16 columns
@@ -3697,9 +3794,9 @@ hipError_t build_plans(Ctx* c) {
       c->ang_fold = ntf;
     }
   }
-  // with Coriolis coupling (mixed precision): the folded forward part into
-  // the FBR slab and the folded back part from the coefficient pass's output,
-  // the coefficient pass between them as in the GEMM variant
+  // with Coriolis coupling: the folded forward part into the FBR slab and the
+  // folded back part, which in mixed precision forms the coefficients itself and
+  // in FP64 reads the coefficient pass's output
   c->ang_fold_cor = 0;
   if (cor_try && tiles_fit && c->ang_ngroups > 0) {
     int ntf = 0;
@@ -3811,8 +3908,11 @@ static hipError_t angular_impl(Ctx* c, const T* psi, hipStream_t s) {
   const bool use_one = c->ang_nt && c->opt_angular <= 1 && !use_fold;
   // folded parts beside the Coriolis pass (mixed precision, FP16 products):
   // the back part forms the coefficients and the Omega +- 1 terms itself
-  const bool use_cor = sizeof(T) == 4 && c->ang_fold_cor && c->opt_angular == 0 && c->opt_fp16 &&
-                       !use_fold && !use_one && !c->ang_fused;
+  // (FP64: the folded parts around the coefficient pass)
+  const bool fold_cor = c->ang_fold_cor && c->opt_angular == 0 && !use_fold && !use_one &&
+                        !c->ang_fused;
+  const bool use_cor = sizeof(T) == 4 && fold_cor && c->opt_fp16;
+  const bool use_cor64 = sizeof(T) == 8 && fold_cor;
   timer_begin(c, K_ANG_FWD, s);
   if (use_fold) {
     if ((e = launch_ang_fold<T>(c, psi, s)) != hipSuccess) return e;
@@ -3832,6 +3932,9 @@ static hipError_t angular_impl(Ctx* c, const T* psi, hipStream_t s) {
     if constexpr (sizeof(T) == 4) {
       if ((e = launch_ang_cor<1>(c, psi, s)) != hipSuccess) return e;
     }
+  } else if (use_cor64) {
+    if constexpr (sizeof(T) == 8)
+      if ((e = launch_ang_cor64<1>(c, psi, s)) != hipSuccess) return e;
   } else {
     e = run_gemm<G_ANG_FWD, T, T, T, T>(s, (const T*)c->d_Dmat, psi, (T*)c->d_fbr, c->p_angF);
     if (e != hipSuccess) return e;
@@ -3873,8 +3976,13 @@ static hipError_t angular_impl(Ctx* c, const T* psi, hipStream_t s) {
   }
   if (!use_one && !use_fold && !use_cor) {
     timer_begin(c, K_ANG_BWD, s);
-    e = run_gemm<G_ANG_BWD, T, T, T, T>(s, (const T*)c->d_Dmat, (const T*)c->d_phi,
-                                        (T*)c->d_ang, c->p_angB);
+    e = hipSuccess;
+    if (!use_cor64) {
+      e = run_gemm<G_ANG_BWD, T, T, T, T>(s, (const T*)c->d_Dmat, (const T*)c->d_phi,
+                                          (T*)c->d_ang, c->p_angB);
+    } else if constexpr (sizeof(T) == 8) {
+      e = launch_ang_cor64<2>(c, psi, s);
+    }
     if (e != hipSuccess) return e;
     timer_end(c, K_ANG_BWD, s);
   }
