@@ -38,25 +38,26 @@ def build_case(cfg):
     return leps.build(leps.config(cfg))
 
 
-# kernel launches per step in each group (mixed and FP64 alike)
-GROUP_LAUNCHES = {"radial_dst": 3, "angular": 1, "update_fused": 1, "update_tail": 2,
-                  "projections": 1, "energy_sums": 2, "coriolis": 1, "products": 1}
+# kernel launches per step in each group (mixed; in FP64 radial_dst is one), per
+# ring of steps for the last four
+GROUP_LAUNCHES = {"radial_dst": 3, "angular": 1, "update_fused": 1, "coriolis": 1,
+                  "update_tail": 2, "projections": 1, "energy_sums": 2, "products": 1}
+RING_GROUPS = ("update_tail", "projections", "energy_sums", "products")
 
 
 def kernel_groups(times, steps):
     """Per-step milliseconds of each kernel group from mw3_timing_get totals:
-    radial_dst (the radial correction passes: k_rad_fwd, k_rad_mid, k_rad_inv
-    at configuration 2), angular (the one-pass angular kernel; in mixed
-    precision on a third stream beside the radial passes), update_fused
-    (the update kernel), update_tail (flux columns and norm of the step,
-    second stream),
-    projections (reactant-state sums; second stream, overlapped with the next
-    step), products (the per-step product-state reduction, same stream as
-    projections), energy_sums (once per ring flush, with the product-state
-    GEMM of the ring: its total time over the timed region divided by the
-    `steps` timed steps, since every flush is timed) and coriolis (the FBR
-    coefficient pass with the Omega +- 1 stencil, run instead of the fused
-    forward epilogue when channels are Coriolis-coupled)."""
+    radial_dst (the radial correction passes: k_rad_fwd_lds, k_rad_mid_f,
+    k_rad_inv_h at configuration 2; in FP64 k_rad_rr, the r products being part
+    of the update), angular (the one-pass angular kernel; in mixed precision on
+    a stream of its own beside the radial passes), update_fused (the update
+    kernel), coriolis (the FBR coefficient pass with the Omega +- 1 stencil, run
+    instead of the fused forward epilogue when channels are Coriolis-coupled)
+    and, once per ring of steps, update_tail (norms and flux columns),
+    projections (reactant-state sums), products (the product-state reduction)
+    and energy_sums (with the product-state GEMM of the ring): the total time
+    over the timed region divided by the `steps` timed steps, since every flush
+    is timed."""
     acc = {}
     for name, (ms, cnt) in times.items():
         if name.startswith("dst"):
@@ -80,16 +81,16 @@ def kernel_groups(times, steps):
     per = {}
     for g, (ms, n) in acc.items():
         if n:
-            per[g] = ms / steps if g == "energy_sums" else ms / n
+            per[g] = ms / steps if g in RING_GROUPS else ms / n
     return per
 
 
 def per_kernel(times, steps):
     """Milliseconds per step of each timed kernel id: per timed launch,
-    except the energy accumulation (once per ring flush, every flush timed),
-    whose total is divided by the timed steps."""
-    return {k: (ms / steps if k == "energy_accum" else ms / max(cnt, 1))
-            for k, (ms, cnt) in times.items()}
+    except the sums over a ring of steps (every flush timed), whose total is
+    divided by the timed steps."""
+    ring = ("energy_accum", "update_tail", "projections", "prod_projection")
+    return {k: (ms / steps if k in ring else ms / max(cnt, 1)) for k, (ms, cnt) in times.items()}
 
 
 def angular_flops(case, variant, N):

@@ -708,7 +708,7 @@ __global__ __launch_bounds__(64 * kUpWaves, 2) void k_update(UpArgs a) {
 // first product's result layout is the second one's right operand as it
 // stands.  A wave runs each loop only a few times, so the time is that of a
 // chain of memory latencies: the next block's loads, and the second product's
-// first table rows, are in flight behind the products.  38 us at 256 x 512 x
+// first table rows, are in flight behind the products.  29 us at 256 x 512 x
 // 120 (38 k1 by 77 k2 modes of 120 angles).
 // ---------------------------------------------------------------------------
 struct RrArgs {
