@@ -4002,13 +4002,19 @@ static hipError_t hpsi_impl(Ctx* c, const double* psi64) {
   const bool use_rr = c->up_nk1 && c->opt_radial;
   // the angular term beside the radial passes, on its own stream (option): it
   // reads psi, written on the main stream, and writes only its own slabs.
-  // Captured steps in mixed precision with the low-mode kernels keep one
-  // stream: a fork and a join inside a graph cost more than the overlap gives
-  // (128 x 256 x 60: 44 us a step against 50; 256 x 512 x 120: 125 against
-  // 128; three states 171 x 256 x 64: 92 against 97).  Beside the GEMMs of a
-  // coarse grid (256 x 256 x 140) the side stream gives 222 against 241, and
-  // outside graphs 122 against 125 at 256 x 512 x 120.
-  const bool one = c->graph_slot_dev && sizeof(T) == 4 && c->opt_radial && c->rad_nitems;
+  // Captured steps in mixed precision keep one stream: a fork and a join inside
+  // a graph cost more than the overlap gives (128 x 256 x 60: 44 us a step
+  // against 50; 256 x 512 x 120: 125 against 128; three states 171 x 256 x 64: 92
+  // against 97; with radial GEMMs 32 x 64 x 16: 24 against 36, 256 x 480 x 120:
+  // 141 against 155).  The exception are radial GEMMs beside an angular term of
+  // several launches (GEMMs, or the parts around the Coriolis coefficients), from
+  // half a million points on: 128 forked against 139 (256 x 256 x 140, 713 000
+  // points), 70 against 82 (J = 1, 105 x 225 x 45, 757 000), 154 against 165 (J =
+  // 2, 160 x 300 x 80, 4.1 M).
+  const bool low = c->opt_radial && c->rad_nitems;
+  const bool one_pass = (c->ang_fold && c->opt_angular == 0) || (c->ang_nt && c->opt_angular <= 1);
+  const bool one =
+      c->graph_slot_dev && sizeof(T) == 4 && (low || one_pass || t.ntot < 500000);
   hipStream_t sa = c->opt_side && !one ? c->side : s;
   if (sa != s) {
     if ((e = hipEventRecord(c->ev_psi, s)) != hipSuccess) return e;
