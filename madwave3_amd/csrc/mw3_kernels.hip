@@ -2351,10 +2351,10 @@ static hipError_t ang_fused_setup(Ctx* c, int nt) {
 // ---------------------------------------------------------------------------
 
 // ---------------------------------------------------------------------------
-// The forward R pass in FP32 with the sine table in LDS: the same sums as
-// k_rad_fwd (t1[r][k2] = sum_{j<h} f_p(r, j) S(j, k2) with the fold f_0 =
-// psi[j] + psi[n2-1-j] for even k2, f_1 = psi[j] - psi[n2-1-j] for odd k2),
-// but each wave owns whole work items: it streams its 16-row tile from HBM,
+// The forward R pass in FP32 with the sine table in LDS: t1[r][k2] =
+// sum_{j<h} f_p(r, j) S(j, k2) with the fold f_0 = psi[j] + psi[n2-1-j] for even
+// k2, f_1 = psi[j] - psi[n2-1-j] for odd k2.
+// Each wave owns whole work items: it streams its 16-row tile from HBM,
 // folds it in registers and multiplies it by every low mode, reading the
 // table from LDS.  The block copies the table into LDS once (even modes,
 // then odd ones, rows padded by 4 floats) and its waves then run with no
@@ -2366,7 +2366,7 @@ static hipError_t ang_fused_setup(Ctx* c, int nt) {
 // the first item's go out before the table copy, and each next item's before
 // the stores of the one before.
 // Items are spread over the waves round robin by block first, so that every
-// SIMD gets about the same number.  Stores as k_rad_fwd: rows past nn1 of
+// SIMD gets about the same number.  Rows past nn1 of
 // the last row tile hold finite values no later pass reads (FULL), and the
 // two parities of a mode pair are one 8-byte store.
 // ---------------------------------------------------------------------------
@@ -2486,10 +2486,9 @@ __global__ __launch_bounds__(64 * kFwdLdsWaves) void k_rad_fwd_lds(
 }
 
 // ---------------------------------------------------------------------------
-// The inverse R pass in FP32 with the sine table in LDS: the sums of
-// k_rad_inv (corr[r][R] = E + O, corr[r][n2-1-R] = E - O for R < h, E / O
-// over the even / odd modes k2 < k2lo) with each wave owning whole work
-// items: it loads its 16 rows of t1 once (columns k2 >= k2lo read as zero),
+// The inverse R pass in FP32 with the sine table in LDS:
+// corr[r][R] = E + O, corr[r][n2-1-R] = E - O for R < h, E / O the sums over
+// the even / odd modes k2 < k2lo, with each wave owning whole work items: it loads its 16 rows of t1 once (columns k2 >= k2lo read as zero),
 // then walks the 16-wide R tiles of the first half, reading the table
 // S(R, k2) from LDS one tile ahead, and skips the tile pairs whose rows hold
 // no compressed-grid point in those columns or their mirrors (the update
