@@ -105,6 +105,16 @@ static __device__ __forceinline__ int opaque(int v) {
   return v;
 }
 
+// LDS values that a wave's lanes leave for each other: what was written before is
+// seen by the reads after, and what was read before is not overwritten by the
+// writes after (a wave's LDS operations execute in order, so this costs no
+// instruction; it keeps the compiler to that order)
+static __device__ __forceinline__ void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+}
+
 // four consecutive values
 template <typename T>
 static __device__ __forceinline__ void ldv4(const T* p, T (&v)[4]) {
@@ -248,7 +258,7 @@ __global__ __launch_bounds__(64 * kUpWaves, 2) void k_update(UpArgs a) {
   // sums of a first segment that belongs to a wave before
   constexpr int NH = FWD ? NKA * 4 * NT * 64 : 1;
   __shared__ __align__(16) T hacc[kUpWaves - 1][NH];
-  __shared__ double hsum[kUpWaves - 1][MODE == 2 ? 4 : 1][SW];
+  __shared__ __align__(16) double hsum[kUpWaves - 1][MODE == 2 ? 4 : 1][SW];
   extern __shared__ double rowl[];  // [n1][3]
   const int lane0 = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
@@ -314,12 +324,14 @@ __global__ __launch_bounds__(64 * kUpWaves, 2) void k_update(UpArgs a) {
         const int k1 = v / (SW / 4), x = 4 * (v - k1 * (SW / 4));
         ldv4(g2 + (k1 < a.kst ? k1 : a.kst - 1) * SW + x, y[l]);
       }
+      wave_lds_sync();  // the last segment's reads
 #pragma unroll
       for (int l = 0; l < NV; l++) {
         const int v = lane + 64 * l;
         const int k1 = v / (SW / 4), x = 4 * (v - k1 * (SW / 4));
         stvn<T, 4>(&gl[k1 * LG + x], y[l]);
       }
+      wave_lds_sync();
     }
   };
 
@@ -501,8 +513,10 @@ __global__ __launch_bounds__(64 * kUpWaves, 2) void k_update(UpArgs a) {
     double o[4][NT];
     T bv[4][NT];  // the new psi (MODE 3: psi) in operator precision, zero off the grid
     if constexpr (FWD) {  // the tile's table rows, for the forward product
+      wave_lds_sync();  // the last tile's reads
 #pragma unroll
       for (int j = 0; j < NK1; j++) stvn<T, 4>(stg + i * LS + 16 * j + 4 * g, av[j]);
+      wave_lds_sync();
     }
     if constexpr (MODE == 3) {
 #pragma unroll
