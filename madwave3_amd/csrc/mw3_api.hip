@@ -180,6 +180,31 @@ const char* mw3_kernel_name(int32_t id) {
   return names[id];
 }
 
+// The buffers for what the updates leave per step (norms, slices, segment sums:
+// of the flux line's three rows, and a fourth with product weights), in place of
+// those there; nothing changes on failure.
+static hipError_t alloc_ring(Ctx* c, bool prod) {
+  const HostTables& t = c->t;
+  const size_t nw = 2 * (size_t)std::max(1, c->up_nwaves);
+  const size_t ns = t.ncvj > 0 ? (size_t)t.nc * t.n1 * t.na : 0;
+  const size_t np = t.nflux > 0 || prod
+                        ? (size_t)std::max(1, c->up_nseg) * (prod ? 4 : 3) * 16 * c->up_nt
+                        : 0;
+  const int d = ring_depth(sizeof(double) * (nw + ns + np));
+  double* p[3] = {nullptr, nullptr, nullptr};
+  const size_t n[3] = {nw, ns, np};
+  hipError_t e = hipSuccess;
+  for (int i = 0; i < 3 && e == hipSuccess; i++)
+    if (n[i]) e = alloc_zero((void**)&p[i], sizeof(double) * d * n[i]);
+  double** const old[3] = {&c->d_norm_part, &c->d_ring_slice, &c->d_up_part};
+  if (e == hipSuccess)
+    for (int i = 0; i < 3; i++) std::swap(p[i], *old[i]);
+  for (double* q : p)
+    if (q) (void)hipFree(q);
+  if (e == hipSuccess) c->up_ring = d;
+  return e;
+}
+
 int32_t mw3_create(const mw3_setup* setup, int32_t precision, mw3_ctx** out) {
   if (!out) return seterr(nullptr, MW3_EINVAL, "mw3_create: out is NULL");
   *out = nullptr;
@@ -344,10 +369,6 @@ int32_t mw3_create(const mw3_setup* setup, int32_t precision, mw3_ctx** out) {
     std::vector<int32_t> i1f(t.ir1flux.begin(), t.ir1flux.end());
     if (i1f.empty()) i1f.assign(t.na, 1);
     CK(upload_raw(&c->d_ir1flux, i1f.data(), i1f.size()), "mw3_create: flux map");
-    if (t.ncvj > 0)
-      CK(alloc_zero((void**)&c->d_ring_slice,
-                    sizeof(double) * kRing * (size_t)t.nc * t.n1 * t.na),
-         "mw3_create: slice");
   }
   CK(alloc_zero((void**)&c->d_ring_norm, sizeof(double) * 2 * kRing), "mw3_create: norms");
   CK(alloc_zero((void**)&c->d_stats, sizeof(double) * stats_doubles()), "mw3_create: sums");
@@ -361,12 +382,7 @@ int32_t mw3_create(const mw3_setup* setup, int32_t precision, mw3_ctx** out) {
     CK(alloc_zero((void**)&c->d_zfe, sizeof(double) * 2 * setup->nofe * nd), "mw3_create: zfe");
   }
   CK(build_plans(c), "mw3_create: plans");
-  CK(alloc_zero((void**)&c->d_norm_part,
-                sizeof(double) * 2 * kRing * (size_t)std::max(1, c->up_nwaves)),
-     "mw3_create: norms");
-  CK(alloc_zero((void**)&c->d_up_part,
-                sizeof(double) * kRing * (size_t)std::max(1, c->up_nseg) * 64 * c->up_nt),
-     "mw3_create: segment sums");
+  CK(alloc_ring(c, false), "mw3_create: sums of the steps");
   CK(hipStreamSynchronize(c->stream), "mw3_create: sync");
 #undef CK
   *out = reinterpret_cast<mw3_ctx*>(c);
@@ -419,7 +435,7 @@ static int clear_accumulators(Ctx* c) {
     HIPCHK(c, launch_zero(c, c->d_zs2prod, sizeof(double) * 2 * nx * netot), "clear");
     HIPCHK(c, launch_zero(c, c->d_cvjp_last, sizeof(double) * nx), "clear");
   }
-  c->ring_fill = 0;
+  c->ring_fill = c->sum_from = 0;
   return MW3_OK;
 }
 
@@ -445,7 +461,7 @@ int32_t mw3_cheby_begin(mw3_ctx* ctx, const double* psi0, double* stats3) {
                              hipMemcpyDeviceToHost, c->stream),
            "mw3_cheby_begin: sums");
   }
-  c->ring_fill = 0;
+  c->ring_fill = c->sum_from = 0;
   c->rec_it.clear();
   c->rec_cvj.clear();
   c->rec_cvjp.clear();
@@ -496,7 +512,7 @@ static int flush_ring(Ctx* c, double* norms_dst, double* auto_dst) {
     if (auto_dst) auto_dst[i] = nb[2 * i + 1];
   }
   c->ring_k0 += c->ring_fill;
-  c->ring_fill = 0;
+  c->ring_fill = c->sum_from = 0;
   if (c->timing) timer_collect(c);
   return MW3_OK;
 }
@@ -535,11 +551,6 @@ static void swap_psi(Ctx* c) {
   std::swap(c->d_psi32, c->d_psim132);
 }
 
-// Steps of one graph launch where that many are to come.  Between two graphs
-// the stream idles for 5 to 7 us: one launch per step cost the 32 x 64 x 16
-// grid a quarter of its step.
-constexpr int kRun = 16;
-
 // Captures one step of c as graph q (psi in buffer q), or kRun steps (an even
 // number, which leaves psi where it was) as graph 2.
 static hipError_t capture_steps(Ctx* c, int q) {
@@ -569,6 +580,18 @@ static bool step_pre(Ctx* c) {
   return graphs_usable(c);
 }
 
+// The sums of the ring's steps so far, where the next `run` steps would take the
+// place of what they are formed from (none in a trial, whose ring is not read).
+static int ring_room(Ctx* c, int run) {
+  if (c->trial || c->ring_fill - c->sum_from + run <= c->up_ring) return MW3_OK;
+  const bool timed = c->timing_step;
+  c->timing_step = true;  // like the energy sums: every ring's are timed
+  const hipError_t e = launch_ring_sums(c);
+  c->timing_step = timed;
+  HIPCHK(c, e, "mw3_cheby_steps: ring sums");
+  return MW3_OK;
+}
+
 // Step of c, second part: the kernels, as a graph or one by one (a step whose
 // psi has no G yet runs one by one: it forms G first).  *run: the steps that
 // may be enqueued at once, then those that were.
@@ -583,12 +606,16 @@ static int step_body(Ctx* c, bool graphs, int32_t* run) {
       q = 2;
       *run = kRun;
     }
+    const int rc = ring_room(c, *run);
+    if (rc) return rc;
     c->dslot_host = c->ring_fill + *run;
     if (!c->graph[q]) HIPCHK(c, capture_steps(c, q), "mw3_cheby_steps: step capture");
     HIPCHK(c, hipGraphLaunch(c->graph[q], c->stream), "mw3_cheby_steps: step graph");
     return MW3_OK;
   }
   c->dslot_host = -1;
+  const int rc = ring_room(c, 1);
+  if (rc) return rc;
   HIPCHK(c, launch_hpsi(c, c->d_psi), "mw3_cheby_steps: H psi");
   HIPCHK(c, launch_update(c, 2, c->d_psi, true), "mw3_cheby_steps: update");
   return MW3_OK;
@@ -607,7 +634,7 @@ static int step_post(Ctx* c, int32_t* done, int32_t nsteps, double* norms,
   *done += 1;
   if (c->trial && (c->ring_fill == kRing || *done == nsteps)) {
     // autotuner trial: the ring is discarded unread
-    c->ring_fill = 0;
+    c->ring_fill = c->sum_from = 0;
     return MW3_OK;
   }
   if (c->ring_fill == kRing || *done == nsteps) {
@@ -949,6 +976,7 @@ int32_t mw3_prod_attach(mw3_ctx* ctx, const mw3_prod_setup* ps) {
   if (e == hipSuccess) e = alloc_zero((void**)&c->d_cvjp_last, sizeof(double) * nx);
   if (e == hipSuccess) e = alloc_zero((void**)&c->d_zs2prod, sizeof(double) * 2 * nx * netot);
   if (e == hipSuccess) e = build_prod_plan(c);
+  if (e == hipSuccess) e = alloc_ring(c, true);
   if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
   if (e != hipSuccess) {
     free_prod(c);
@@ -1227,7 +1255,7 @@ int32_t mw3_autotune(mw3_ctx* ctx, int32_t trial_steps, int32_t* chosen, double*
   c->d_psim1 = pm0;
   c->k = k0;
   c->ring_k0 = rk0;
-  c->ring_fill = 0;
+  c->ring_fill = c->sum_from = 0;
   c->g_fresh = false;
   HIPCHK(c, hipMemcpyAsync(c->d_psi, c->d_hout, bytes, hipMemcpyDeviceToDevice, c->stream),
          "mw3_autotune: restore");

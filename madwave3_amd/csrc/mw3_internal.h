@@ -23,6 +23,11 @@ namespace mw3 {
 // ring, so a longer ring moves fewer accumulator bytes per step
 constexpr int kRing = 256;
 
+// Steps of one graph launch where that many are to come.  Between two graphs
+// the stream idles for 5 to 7 us: one launch per step cost the 32 x 64 x 16
+// grid a quarter of its step.
+constexpr int kRun = 16;
+
 // Host-side operator tables built from mw3_setup (mw3_setup.cpp).
 struct HostTables {
   // sizes
@@ -138,7 +143,14 @@ struct Ctx {
   void* d_up_seg = nullptr;         // [up_nseg] step::UpSeg
   uint32_t* d_up_tile = nullptr;    // [up_nwaves][up_tmax][64]
   int32_t* d_up_sfirst = nullptr;   // [nc na up_ns + 1] first segment of each strip
-  double* d_up_part = nullptr;      // [kRing][up_nseg][4][16 up_nt] sums over r
+  // What the updates leave for the sums of the ring (norms, flux columns,
+  // product weights, slices), for the last up_ring steps: the sums of steps
+  // sum_from .. ring_fill - 1 of the ring are formed before a step takes the
+  // place of one of them.  4 / n1 of a psi slab per step, so as many steps as
+  // fit 64 MB, from one graph launch to a whole ring (ring_depth).
+  double* d_up_part = nullptr;      // [up_ring][up_nseg][3, 4 with products][16 up_nt] sums over r
+  int up_ring = kRun;
+  int sum_from = 0;
   int up_nwaves = 0, up_nseg = 0, up_tmax = 0, up_nt = 1, up_ns = 0, up_segmax = 0;
   int up_nk1 = 0;                 // 16-mode tiles of the low r modes (0: radial GEMMs only)
   int up_kst = 0;                 // low r modes kept of G, G2
@@ -196,7 +208,7 @@ struct Ctx {
   double* d_fdv = nullptr;
   double* d_dcvj = nullptr;
   uint8_t* d_cvj_skip = nullptr; // [ncvj] 1 if the reference state (kminelastic)
-  double* d_norm_part = nullptr; // update wave sums [kRing][up_nwaves][2]
+  double* d_norm_part = nullptr; // update wave sums [up_ring][up_nwaves][2]
   double* d_stats = nullptr;     // sums of mw3_cheby_begin (launch_stats)
   double* d_ring_norm = nullptr; // [kRing][2] (norm, autocorrelation)
   double* d_efe = nullptr;
@@ -259,14 +271,14 @@ struct Ctx {
 
   int32_t* d_fmap = nullptr;     // [nc][na][n2] flux point index or -1
   int32_t* d_ir1flux = nullptr;  // [na]
-  double* d_ring_slice = nullptr; // [kRing][nc][na][n1] psi at R = ir2abs / sqrt(ah2)
+  double* d_ring_slice = nullptr; // [up_ring][nc][na][n1] psi at R = ir2abs / sqrt(ah2)
 
   // product-state projection (iprod = 2, mw3_prod_attach).  Per step, the
   // update leaves funprod(c, l) = sum_r T psi_new (T = transRgjac on the dense
-  // grid), l = (angle, R) of the projection range, in its segment sums.  At
-  // each ring flush dtrans rotates it and the channels of each electronic
-  // state are summed into d_ring_prod[slot][Omega'][e][l], one split-K GEMM
-  // per Omega' projects that on prodwf: Cvjprod[s][Omega'][j'v'] (partials
+  // grid), l = (angle, R) of the projection range, in its segment sums.  With
+  // the ring's other sums dtrans rotates it and the channels of each electronic
+  // state are summed into d_ring_prod[slot][Omega'][e][l]; at each ring flush
+  // one split-K GEMM per Omega' projects that on prodwf: Cvjprod[s][Omega'][j'v'] (partials
   // [Omega'][chunk][kRing][nvj]), and the energy accumulation adds
   // C_k(E) Cvjprod to zS2prod.
   bool prod_on = false;
@@ -337,6 +349,7 @@ hipError_t launch_spectrum(hipStream_t s, const double* d_auto, double* d_a, int
                            double delta2, double* d_spec);  // T, V and angular terms into work slabs
 // 0: H psi into d_hout, 1: first step, 2: damped step (psi_new into d_psim1)
 hipError_t launch_update(Ctx* c, int mode, const double* psi, bool proj = false);
+int ring_depth(size_t bytes);
 hipError_t launch_ring_sums(Ctx* c);
 hipError_t launch_energy_accum(Ctx* c);
 hipError_t launch_psie(Ctx* c, int k);

@@ -628,16 +628,20 @@ hipError_t launch_slot_set(Ctx* c, int q, int v) {
 }
 
 // ---------------------------------------------------------------------------
-// sums over a ring of steps that the update leaves per block, per reactant
-// slice and per channel.  They run once per ring, one block (or grid row) per
-// step, instead of as small kernels after every update.
+// sums over a run of the ring's steps that the update leaves per block, per
+// reactant slice and per channel.  They run once per up_ring steps, one block
+// (or grid row) per step, instead of as small kernels after every update: step
+// from + blockIdx.x (y) of the ring, at its place modulo up_ring in what the
+// updates left.
 // ---------------------------------------------------------------------------
-// (norm, autocorrelation) of step blockIdx.x from the update's block sums
+// (norm, autocorrelation) of a step from the update's block sums
 __global__ __launch_bounds__(256) void k_norm_ring(const double* __restrict__ part_ring, int nb,
-                                                   double* __restrict__ out_ring) {
+                                                   double* __restrict__ out_ring, int from,
+                                                   int ring) {
   typedef double d2 __attribute__((ext_vector_type(2)));
-  const d2* p2 = (const d2*)part_ring + (int64_t)blockIdx.x * nb;
-  double* __restrict__ out = out_ring + 2 * (int64_t)blockIdx.x;
+  const int slot = from + blockIdx.x;
+  const d2* p2 = (const d2*)part_ring + (int64_t)(slot & (ring - 1)) * nb;
+  double* __restrict__ out = out_ring + 2 * (int64_t)slot;
   __shared__ double sh[2][256];
   d2 s0 = {0, 0}, s1 = {0, 0};
   int i = threadIdx.x;
@@ -663,22 +667,23 @@ __global__ __launch_bounds__(256) void k_norm_ring(const double* __restrict__ pa
   }
 }
 
-// flux samples of step blockIdx.y: the sums over r that the update left per
-// segment, added over the segments of the point's strip
+// flux samples of a step: the sums over r that the update left per segment,
+// added over the segments of the point's strip
 __global__ __launch_bounds__(256) void k_flux_ring(const double* __restrict__ upart,
                                                    const int32_t* __restrict__ sfirst,
                                                    const uint32_t* __restrict__ col,
                                                    double* __restrict__ zr,
                                                    double* __restrict__ zdr, int64_t nflux,
                                                    int nseg, int n2, int64_t plane, int ns,
-                                                   int sw) {
-  const int64_t f = (int64_t)blockIdx.x * blockDim.x + threadIdx.x, slot = blockIdx.y;
+                                                   int sw, int nrow, int from, int ring) {
+  const int64_t f = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (f >= nflux) return;
+  const int64_t slot = from + blockIdx.y, place = slot & (ring - 1);
   const int64_t cia = col[f] / plane;
   const int R = col[f] % n2, s = R / sw, x = R - s * sw;
   double re = 0.0, im = 0.0, zv = 0.0;
   for (int k = sfirst[cia * ns + s]; k < sfirst[cia * ns + s + 1]; k++) {
-    const double* up = upart + ((slot * nseg + k) * 4) * sw + x;
+    const double* up = upart + ((place * nseg + k) * nrow) * sw + x;
     re += up[0];
     im += up[sw];
     zv += up[2 * sw];
@@ -688,8 +693,8 @@ __global__ __launch_bounds__(256) void k_flux_ring(const double* __restrict__ up
   zr[slot * nflux + f] = zv;
 }
 
-// Cvj(c, j, v) = sum_r fd(r, v, j) sum_ia slice(c, ia, r) D(ia, j) of step
-// blockIdx.y (Cvjflux_k, SRC/mod_flux_01y2.f:672-702; slice = psi at
+// Cvj(c, j, v) = sum_r fd(r, v, j) sum_ia slice(c, ia, r) D(ia, j) of a step
+// (Cvjflux_k, SRC/mod_flux_01y2.f:672-702; slice = psi at
 // R = ir2abs / sqrt(ah2)).  Block = (channel, jb <= CVJ_J values of j), a
 // thread per r: each slice value is read once for the jb angular sums.
 constexpr int CVJ_J = 8;
@@ -697,11 +702,12 @@ __global__ __launch_bounds__(256) void k_cvj_ring(const double* __restrict__ sli
                                                   const double* __restrict__ dcvj,
                                                   const double* __restrict__ fdv,
                                                   double* __restrict__ cvj_ring, int nc, int nj,
-                                                  int nv, int na, int n1, int jb, int64_t ncvj) {
+                                                  int nv, int na, int n1, int jb, int64_t ncvj,
+                                                  int from, int ring) {
   const int njb = (nj + jb - 1) / jb;
   const int c = blockIdx.x / njb, j0 = (blockIdx.x - c * njb) * jb;
-  const int64_t slot = blockIdx.y;
-  const double* __restrict__ sl = slice_ring + (slot * nc + c) * (int64_t)na * n1;
+  const int64_t slot = from + blockIdx.y, place = slot & (ring - 1);
+  const double* __restrict__ sl = slice_ring + (place * nc + c) * (int64_t)na * n1;
   double* __restrict__ cvj = cvj_ring + slot * ncvj + ((int64_t)c * nj + j0) * nv;
   extern __shared__ double xj[];  // [jb][n1]
   const double* dj[CVJ_J];
@@ -3872,6 +3878,7 @@ static step::UpArgs update_args(Ctx* c, int mode, const double* psi, bool proj) 
     a.dslot_next = c->d_slot + (1 - q);
   }
   a.slot = c->ring_fill;
+  a.ring = c->up_ring;
   a.part = mode == 1 || mode == 2 ? c->d_norm_part : nullptr;
   if (proj && mode == 2) {
     a.slice = t.ncvj > 0 ? c->d_ring_slice : nullptr;
@@ -4104,20 +4111,33 @@ hipError_t launch_update(Ctx* c, int mode, const double* psi, bool proj) {
   return hipSuccess;
 }
 
-// per-step sums of the ring's steps from what the updates left
+// Steps kept for the ring's sums, at `bytes` per step: as many as fit 64 MB,
+// from kRun to kRing.  A whole ring would take 2.4 GB at seven blocks of 192 x
+// 384 x 96 (psi slab 0.4 GB), 16 steps take 0.13.  The sums' three launches per
+// 16 steps are under a hundredth of the step there; grids whose steps are short
+// keep the whole ring.
+int ring_depth(size_t bytes) {
+  int d = kRing;
+  while (d > kRun && d * bytes > ((size_t)64 << 20)) d /= 2;
+  return d;
+}
+
+// per-step sums of the ring's steps from what the updates left, as far as they
+// are not formed yet
 hipError_t launch_ring_sums(Ctx* c) {
   const HostTables& t = c->t;
-  const int ns = c->ring_fill;
+  const int from = c->sum_from, ns = c->ring_fill - from, ring = c->up_ring;
   hipError_t e;
-  if (ns == 0) return hipSuccess;
+  if (ns <= 0) return hipSuccess;
   timer_begin(c, K_UPDATE_TAIL);
   hipLaunchKernelGGL(k_norm_ring, dim3(ns), dim3(256), 0, c->stream, c->d_norm_part,
-                     c->up_nwaves, c->d_ring_norm);
+                     c->up_nwaves, c->d_ring_norm, from, ring);
   if ((e = hipGetLastError()) != hipSuccess) return e;
   if (t.nflux > 0) {
     hipLaunchKernelGGL(k_flux_ring, dim3(nblk(t.nflux, 256), ns), dim3(256), 0, c->stream,
                        c->d_up_part, c->d_up_sfirst, c->d_flux_col, c->d_ring_zr, c->d_ring_zdr,
-                       t.nflux, c->up_nseg, t.n2, t.nplane, c->up_ns, 16 * c->up_nt);
+                       t.nflux, c->up_nseg, t.n2, t.nplane, c->up_ns, 16 * c->up_nt,
+                       c->prod_on ? 4 : 3, from, ring);
     if ((e = hipGetLastError()) != hipSuccess) return e;
   }
   timer_end(c, K_UPDATE_TAIL);
@@ -4127,11 +4147,14 @@ hipError_t launch_ring_sums(Ctx* c) {
     const int jb = std::max(1, std::min(CVJ_J, 8192 / t.n1));  // within 64 KB of LDS
     hipLaunchKernelGGL(k_cvj_ring, dim3(t.nc * ((nj + jb - 1) / jb), ns), dim3(256),
                        sizeof(double) * jb * t.n1, c->stream, c->d_ring_slice, c->d_dcvj,
-                       c->d_fdv, c->d_ring_cvj, t.nc, nj, nv, t.na, t.n1, jb, (int64_t)t.ncvj);
+                       c->d_fdv, c->d_ring_cvj, t.nc, nj, nv, t.na, t.n1, jb, (int64_t)t.ncvj,
+                       from, ring);
     if ((e = hipGetLastError()) != hipSuccess) return e;
     timer_end(c, K_PROJ);
   }
-  return c->prod_on ? launch_prod_sums(c) : hipSuccess;
+  if (c->prod_on && (e = launch_prod_sums(c)) != hipSuccess) return e;
+  c->sum_from = c->ring_fill;
+  return hipSuccess;
 }
 
 hipError_t launch_energy_accum(Ctx* c) {
@@ -4196,9 +4219,11 @@ __global__ __launch_bounds__(256) void k_prod_fun(const double* __restrict__ upa
                                                   const int32_t* __restrict__ ch_elec,
                                                   double* __restrict__ ring, int nc, int ne,
                                                   int nomb, int64_t L, int na, int nap0, int n2p0,
-                                                  int n2p, int nseg, int ns, int sw) {
-  const int64_t l = (int64_t)blockIdx.x * blockDim.x + threadIdx.x, slot = blockIdx.y;
+                                                  int n2p, int nseg, int ns, int sw, int from,
+                                                  int nring) {
+  const int64_t l = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (l >= L) return;
+  const int64_t slot = from + blockIdx.y, place = slot & (nring - 1);
   const int ia = nap0 + (int)(l / n2p), R = n2p0 + (int)(l % n2p), s = R / sw, x = R - s * sw;
   for (int o = 0; o < nomb; o++)
     for (int e = 0; e < ne; e++) ring[((slot * nomb + o) * ne + e) * L + l] = 0.0;
@@ -4206,7 +4231,7 @@ __global__ __launch_bounds__(256) void k_prod_fun(const double* __restrict__ upa
     const int64_t q = (int64_t)(ch * na + ia) * ns + s;
     double f = 0.0;
     for (int k = sfirst[q]; k < sfirst[q + 1]; k++)
-      f += upart[((slot * nseg + k) * 4 + 3) * sw + x];
+      f += upart[((place * nseg + k) * 4 + 3) * sw + x];
     for (int o = 0; o < nomb; o++)
       ring[((slot * nomb + o) * ne + ch_elec[ch]) * L + l] +=
           f * dtrans[((int64_t)ch * nomb + o) * L + l];
@@ -4229,10 +4254,11 @@ __global__ void k_prod_sum(const double* __restrict__ part, double* __restrict__
 
 hipError_t launch_prod_sums(Ctx* c) {
   timer_begin(c, K_PROD);
-  hipLaunchKernelGGL(k_prod_fun, dim3(nblk(c->pr_L, 256), c->ring_fill), dim3(256), 0, c->stream,
+  hipLaunchKernelGGL(k_prod_fun, dim3(nblk(c->pr_L, 256), c->ring_fill - c->sum_from), dim3(256),
+                     0, c->stream,
                      c->d_up_part, c->d_up_sfirst, c->d_dtrans, c->d_ch_elec, c->d_ring_prod,
                      c->t.nc, c->t.ne, c->pr_nomb, c->pr_L, c->t.na, c->pr_nap0, c->pr_n2p0,
-                     c->pr_n2p, c->up_nseg, c->up_ns, 16 * c->up_nt);
+                     c->pr_n2p, c->up_nseg, c->up_ns, 16 * c->up_nt, c->sum_from, c->up_ring);
   const hipError_t e = hipGetLastError();
   timer_end(c, K_PROD);
   return e;

@@ -228,10 +228,14 @@ struct UpArgs {
   const int32_t* dslot;
   int32_t* dslot_next;
   int slot;
-  double* part;          // [kRing][nwaves][2] (norm, autocorrelation)
-  double* upart;         // [kRing][nseg][4][16 NT]: sum_r of Re and Im zAR1flux
-                         // psi, psi at the flux row, product weights psi; or null
-  double* slice;         // [kRing][nc na][n1] or null
+  // what the step leaves for the ring's sums, at place slot mod ring (a power
+  // of two)
+  int ring;
+  double* part;          // [ring][nwaves][2] (norm, autocorrelation)
+  double* upart;         // [ring][nseg][3 or 4][16 NT]: sum_r of Re and Im zAR1flux
+                         // psi, psi at the flux row, with product weights those
+                         // times psi; or null
+  double* slice;         // [ring][nc na][n1] or null
   int ir2abs;
 };
 
@@ -276,8 +280,9 @@ __global__ __launch_bounds__(64 * kUpWaves, 2) void k_update(UpArgs a) {
   const uint32_t rb = (uint32_t)n2 * 16u;  // values of a row tile
   T* const gl = lds + wave * (NG + NSTG);
   T* const stg = gl + NG;
-  const int64_t slot = a.dslot ? (int64_t)*a.dslot : (int64_t)a.slot;
-  if (a.dslot_next && blockIdx.x == 0 && threadIdx.x == 0) *a.dslot_next = (int32_t)slot + 1;
+  const int islot = a.dslot ? *a.dslot : a.slot;
+  if (a.dslot_next && blockIdx.x == 0 && threadIdx.x == 0) *a.dslot_next = islot + 1;
+  const int64_t slot = islot & (a.ring - 1);
   if constexpr (MODE != 3)
     for (int k = threadIdx.x; k < 3 * n1; k += 64 * kUpWaves) {
       const int r = k / 3;
@@ -471,7 +476,7 @@ __global__ __launch_bounds__(64 * kUpWaves, 2) void k_update(UpArgs a) {
     }
     if constexpr (MODE == 2) {
       if (a.upart) {
-        double* up = a.upart + (slot * a.nseg + s.seg) * (4 * SW) + NT * i;
+        double* up = a.upart + (slot * a.nseg + s.seg) * ((PRODP ? 4 : 3) * SW) + NT * i;
 #pragma unroll
         for (int k = 0; k < (PRODP ? 4 : 3); k++) {
           double x[NT];

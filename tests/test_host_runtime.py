@@ -1,0 +1,88 @@
+"""What libmw3 asks of the HIP runtime, on a runtime without a device
+(tests/fakehip.c, loaded in a process of its own): device memory of a context."""
+import json
+import os
+import subprocess
+import sys
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+PRELUDE = """
+import ctypes as ct, json, sys
+fake = ct.CDLL(sys.argv[1], mode=ct.RTLD_GLOBAL)
+fake.fake_log.restype = ct.c_char_p
+fake.fake_bytes.restype = ct.c_size_t
+sys.path.insert(0, sys.argv[2])
+from madwave3_amd import leps, lib as L
+def log():
+    s = fake.fake_log().decode()
+    fake.fake_log_clear()
+    return s
+def case(n1, n2, na, J=0, **kw):
+    p = leps.config(4, J=J) if J else leps.config(1)
+    p.update(npun1=n1, npun2=n2, nangu=na, npun1min=min(16, n1 // 2), jmax=min(5, na - 1),
+             nvmax=2, netot=100, iprod=0, kminelastic=4, width_bohr=0.6, absorb_bohr=4.5)
+    if J:
+        p.update(Jtot=J, iommin=J % 2 if J > 1 else 0, iommax=min(J, 6), iomref=-1)
+    p.update(kw)
+    return leps.build(p)
+out = {}
+"""
+
+
+@pytest.fixture(scope="module")
+def fake(tmp_path_factory):
+    so = str(tmp_path_factory.mktemp("fake") / "fakehip.so")
+    subprocess.run(["gcc", "-O1", "-w", "-shared", "-fPIC", "-o", so,
+                    os.path.join(HERE, "fakehip.c")], check=True)
+
+    def run(script):
+        r = subprocess.run([sys.executable, "-c", PRELUDE + script + "\nprint(json.dumps(out))",
+                            so, os.path.dirname(HERE)], capture_output=True, text=True,
+                           timeout=300)
+        assert r.returncode == 0, r.stderr
+        return json.loads(r.stdout.splitlines()[-1])
+    return run
+
+
+MEMORY = """
+for i, (n1, n2, na, J, prec, prod) in enumerate([(64, 256, 64, 12, 0, 0), (64, 256, 64, 12, 1, 0),
+                                                 (64, 256, 64, 0, 1, 1), (32, 64, 16, 0, 0, 0)]):
+    c = case(n1, n2, na, J, **(dict(iprod=2, nvmaxprod=2, jmaxprod=5) if prod else {}))
+    g = L.Propagator(c, prec, prod=False)
+    b0 = fake.fake_bytes()
+    if prod:
+        g.prod_attach()
+    b = fake.fake_bytes()
+    out[i] = dict(bytes=b, attach=b - b0, nc=c.ncan, n1=n1, n2=n2, na=na, prec=prec, ntot=c.ntot,
+                  nflux=g.nflux, netot=c.netot, ncvj=c.ncan * (c.jmax - c.jini + 1) * 3)
+    if prod:
+        L_ = (c.nangproj1 - c.nangproj0 + 1) * (c.n2prod1 - c.n2prod0 + 1)
+        nvj = L.prod_shape(c)[1] * L.prod_shape(c)[2]
+        out[i]["prod"] = 8 * (L_ * (1 + nvj + 256) + 256 * nvj * 600)
+    g.close()
+out["left"] = fake.fake_bytes()
+"""
+
+
+def test_device_memory_of_a_context(fake):
+    """Within the slabs, accumulators and tables a propagation needs; what the
+    updates leave for the ring's sums takes at most 64 MB, or 16 steps'."""
+    out = fake(MEMORY)
+    assert out.pop("left") == 0
+    for r in out.values():
+        s = 4 if r["prec"] else 8
+        grid = r["nc"] * r["na"] * r["n1"] * r["n2"]
+        cols = r["nc"] * r["na"] * (r["n2"] + 32)
+        state = 5 * 8 * grid + (3 * 4 * grid if r["prec"] else 0)  # psi, psi_{k-1}, psi0, H psi, input
+        work = 5 * s * grid + s * grid / r["nc"] + 2 * 8 * r["ntot"]
+        accum = r["nflux"] * (32 * r["netot"] + 24 * 256) + r["ncvj"] * (16 * r["netot"] + 8 * 256)
+        step = cols * 4 * 8 * 1.25 + 8 * r["nc"] * r["na"] * r["n1"]  # (strips cut in segments: 1.25)
+        rings = max(64 << 20, 16 * step)
+        low = 0 if r["prec"] else 2.5 * 8 * 48 * cols  # G, G2
+        tables = 0.5 * 8 * grid + (4 << 20)
+        limit = state + work + accum + rings + low + tables + r.get("prod", 0) + (
+            s * grid if "prod" in r else 0)
+        print(r, "limit %.1f MB" % (limit / 1e6))
+        assert r["bytes"] <= limit, (r, limit)
