@@ -944,6 +944,32 @@ static hipError_t zalloc(void** p, size_t n) {
   return e == hipSuccess ? hipMemset(*p, 0, std::max<size_t>(n, 16)) : e;
 }
 
+// blocks of the step's update that a CU holds, of the two that its registers
+// allow: 160 KB of LDS over what the kernel takes (its sums and tables, and 24
+// bytes per r row)
+template <typename T, int NK1, int NT>
+static hipError_t resident(int n1, int* blocks) {
+  hipFuncAttributes f{};
+  const hipError_t e = hipFuncGetAttributes(&f, (const void*)k_update<T, NK1, NT, 0, 0, 2>);
+  *blocks = f.sharedSizeBytes + sizeof(double) * 3 * (size_t)n1 > 80 * 1024 ? 1 : 2;
+  return e;
+}
+
+template <typename T>
+static hipError_t resident(const Ctx* c, int* blocks) {
+  const int n1 = c->t.n1;
+  if constexpr (sizeof(T) == 4) {
+    return c->up_nt == 2 ? resident<T, 0, 2>(n1, blocks) : resident<T, 0, 1>(n1, blocks);
+  } else {
+    switch (c->up_nk1) {
+      case 1: return resident<T, 1, 1>(n1, blocks);
+      case 3: return resident<T, 3, 1>(n1, blocks);
+      case 4: return resident<T, 4, 1>(n1, blocks);
+      default: return resident<T, 0, 1>(n1, blocks);
+    }
+  }
+}
+
 // strips, tiles and (where the low modes fit the kernels) tables of the step
 template <typename T>
 static hipError_t build(Ctx* c) {
@@ -1019,8 +1045,15 @@ static hipError_t build(Ctx* c) {
   if ((e = upload_t<T>(&c->d_up_tab, tab)) != hipSuccess) return e;
   // Waves.  Few strips (every strip's block resident at once): a block per
   // strip, its waves an equal part each, so that a strip is one segment.  Else
-  // runs of equal length over all channels' tiles, for two waves per SIMD, so
-  // that the one resident set of waves ends together.
+  // runs of equal length over all channels' tiles, for as many waves as are
+  // resident at once, so that the one resident set ends together.  Runs too
+  // where a strip's quarter is more than twice their length, which leaves most
+  // of the chip idle: few strips of many rows (us a step, a block per strip ->
+  // runs: 64 x 64 x 8 FP64 18.4 either way, 256 x 64 x 8 26.7 -> 20.8, mixed
+  // 1500 x 64 x 16 98 -> 71, 3000 x 64 x 16 170 -> 117).  Runs for two blocks per
+  // CU where one fits took longer than those for one (4096 x 64 x 16 mixed 165
+  // against 150, FP64 210 against 195, four mode tiles at 160 x 256 x 60 53
+  // against 47).
   int64_t total = 0, nstrip = 0;
   for (int x : cnt) {
     total += x;
@@ -1032,12 +1065,14 @@ static hipError_t build(Ctx* c) {
   if ((e = hipGetDevice(&dev)) != hipSuccess) return e;
   if ((e = hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev)) != hipSuccess)
     return e;
-  const bool aligned = nstrip <= 2 * ncu;
-  int tmax = (int)std::max<int64_t>(1, (total + 8 * ncu - 1) / (8 * ncu));
-  if (aligned) {
-    tmax = 1;
-    for (int x : cnt) tmax = std::max(tmax, (x + kUpWaves - 1) / kUpWaves);
-  }
+  int res = 0;
+  if ((e = resident<T>(c, &res)) != hipSuccess) return e;
+  const int nw = res * kUpWaves * ncu;  // resident waves
+  int tmax = (int)std::max<int64_t>(1, (total + nw - 1) / nw);
+  int per = 1;  // tiles of a wave, a block to each strip
+  for (int x : cnt) per = std::max(per, (x + kUpWaves - 1) / kUpWaves);
+  const bool aligned = nstrip <= res * ncu && per <= 2 * tmax;
+  if (aligned) tmax = per;
   std::vector<UpWave> waves;
   std::vector<UpSeg> segs;
   std::vector<uint32_t> lists;

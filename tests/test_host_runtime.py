@@ -1,5 +1,6 @@
 """What libmw3 asks of the HIP runtime, on a runtime without a device
-(tests/fakehip.c, loaded in a process of its own): device memory of a context."""
+(tests/fakehip.c, loaded in a process of its own): device memory of a context, blocks
+of the update."""
 import json
 import os
 import subprocess
@@ -86,3 +87,25 @@ def test_device_memory_of_a_context(fake):
             s * grid if "prod" in r else 0)
         print(r, "limit %.1f MB" % (limit / 1e6))
         assert r["bytes"] <= limit, (r, limit)
+
+
+BLOCKS = """
+for i, (n1, n2, na) in enumerate([(16, 32, 4), (128, 64, 8), (1200, 64, 16), (3500, 64, 16),
+                                  (256, 256, 60)]):
+    c = case(n1, n2, na, jmax=0, nvmax=0)
+    for prec in (0, 1):
+        g = L.Propagator(c, prec)
+        g.begin(c.rpaq0)
+        out["%d %d" % (i, prec)] = [n1, fake.fake_grid(b"k_update")]
+        g.close()
+"""
+
+
+def test_update_fills_the_chip(fake):
+    """The update's blocks (256 CUs, two blocks on each, one with more than 80 KB of
+    LDS): long strips are shared out, and no more blocks run than are resident."""
+    out = fake(BLOCKS)
+    for k, (n1, blocks) in out.items():
+        print(k, n1, blocks)
+        assert 0 < blocks <= (256 if 24 * n1 > 80 * 1024 else 512)
+        assert n1 < 1000 or blocks > 200
