@@ -879,16 +879,25 @@ __global__ void k_psie(double* __restrict__ zfe, const double* __restrict__ psi,
 // 71-90): spec(E) = [a_0 + sum_k a_k cos(-k acos Es)] / (sqrt(1 - Es^2) delta2)
 // with a_0 = auto_0 hbr, a_k = 2 hbr e^{-k xkgam} auto_k; NaN -> 0.
 //
-// A block sums four energies: thread j takes k = 1 + j + 512 m and gets
-// cos(k th) from that of the term before by a rotation through 512 th, which
-// is exact in binary, so its angle carries no rounding that grows with k
-// (k th itself, rounded, would).  Four products per term in place of a cosine
-// with its argument reduction, and ne / 4 blocks instead of ne / 256: bound by
-// the loads of a_k, once per four energies, from the L2.
-// 30 000 terms at 2 000 energies: the call 5.92 -> 0.12 ms, mostly allocation
-// and copies now.  Error of the sum against extended precision at those sizes:
-// 3.5e-13 (4.1e-13 by cosines), of which 1.4e-14 (2.2e-13) beyond that of
-// the rounded angle th itself.
+// k_spectrum: a block sums four energies; thread j takes k = 1 + j + 512 m and
+// gets cos(k th) from that of the term before by a rotation through 512 th.  The
+// rotation's factors are rounded once and its products once a turn, so the error
+// of a term grows by about an ulp per 512 k, where a rounded k th alone is off
+// by half an ulp of itself: 30 000 terms at 2 000 energies, against extended
+// precision, 3.5e-13 (4.1e-13 by cosines), of which 1.4e-14 (2.2e-13) beyond
+// that of the rounded angle th itself.  Four products per term in place of a
+// cosine with its argument reduction, and ne / 4 blocks instead of ne / 256:
+// bound by the loads of a_k, once per four energies, from the L2.  That call
+// 5.92 -> 0.12 ms, mostly allocation and copies now.  Up to 512 terms a thread
+// has one term at most, and only as many threads run.
+//
+// k_spec_direct: one energy per thread and a cosine per term, for so many
+// energies that they fill the chip by themselves and so few terms that two sines
+// and cosines per thread of the other form cost more than they save.  Both
+// kernels, us (direct / blocks): 100 000 energies with 10 terms 8 / 26, 256 terms
+// 76 / 84, 700 terms 197 / 262, 1024 terms 289 / 265; 32 000 energies with 10
+// terms 9 / 12, 31 terms 10.5 / 12.1, 513 terms 95 / 87; 64 000 with 400 terms
+// 76 / 119.
 // ---------------------------------------------------------------------------
 __global__ void k_spec_coef(const double* __restrict__ autoc, double* __restrict__ a, int kmax,
                             double hbr, double xkgam) {
@@ -896,7 +905,29 @@ __global__ void k_spec_coef(const double* __restrict__ autoc, double* __restrict
     a[k] = k == 0 ? autoc[0] * hbr : 2.0 * hbr * exp(-(double)k * xkgam) * autoc[k];
 }
 
-constexpr int SPEC_T = 512, SPEC_E = 4;
+constexpr int SPEC_T = 512, SPEC_E = 4, SPEC_DIRECT = 896;
+
+// a sum over the spectrum's norm sqrt(1 - Es^2) delta2, rounded once where Es is
+// near 1 (by a product of its own it is 4e-12 off at Es = 0.99999)
+static __device__ __forceinline__ double spec_value(double x, double Es, double delta2) {
+  x = x / (sqrt(fma(-Es, Es, 1.0)) * delta2);
+  return isnan(x) ? 0.0 : x;
+}
+
+__global__ __launch_bounds__(256) void k_spec_direct(const double* __restrict__ a, int kmax,
+                                                     const double* __restrict__ e, int ne,
+                                                     double emindlt, double delta2,
+                                                     double* __restrict__ spec) {
+  __shared__ double sa[SPEC_DIRECT + 1];
+  for (int k = threadIdx.x; k <= kmax; k += 256) sa[k] = a[k];
+  __syncthreads();
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i >= ne) return;
+  const double Es = (e[i] - emindlt) / delta2, th = acos(Es);
+  double x = sa[0];
+  for (int k = 1; k <= kmax; k++) x += sa[k] * cos((double)k * th);
+  spec[i] = spec_value(x, Es, delta2);
+}
 
 __global__ __launch_bounds__(SPEC_T) void k_spectrum(const double* __restrict__ a, int kmax,
                                                      const double* __restrict__ e, int ne,
@@ -904,25 +935,39 @@ __global__ __launch_bounds__(SPEC_T) void k_spectrum(const double* __restrict__ 
                                                      double* __restrict__ spec) {
   __shared__ double red[SPEC_T / 64][SPEC_E];
   const int i0 = blockIdx.x * SPEC_E;
-  const int k0 = 1 + threadIdx.x;
-  double co[SPEC_E], si[SPEC_E], cr[SPEC_E], sr[SPEC_E], sp[SPEC_E];
-#pragma unroll
-  for (int q = 0; q < SPEC_E; q++) {
-    const int i = i0 + q < ne ? i0 + q : ne - 1;
-    const double th = acos((e[i] - emindlt) / delta2);
-    sincos((double)k0 * th, &si[q], &co[q]);
-    sincos((double)SPEC_T * th, &sr[q], &cr[q]);
-    sp[q] = 0.0;
+  const int k0 = 1 + threadIdx.x, nw = blockDim.x >> 6;
+  double th[SPEC_E], sp[SPEC_E] = {};
+  if (threadIdx.x < SPEC_E) {
+    const int i = i0 + threadIdx.x;
+    red[0][threadIdx.x] = acos((e[i < ne ? i : ne - 1] - emindlt) / delta2);
   }
-#pragma unroll 4
-  for (int k = k0; k <= kmax; k += SPEC_T) {
-    const double ak = a[k];
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < SPEC_E; q++) th[q] = red[0][q];
+  __syncthreads();
+  if (kmax <= SPEC_T) {  // a term per thread at most
+    if (k0 <= kmax) {
+      const double ak = a[k0];
+#pragma unroll
+      for (int q = 0; q < SPEC_E; q++) sp[q] = ak * cos((double)k0 * th[q]);
+    }
+  } else {
+    double co[SPEC_E], si[SPEC_E], cr[SPEC_E], sr[SPEC_E];
 #pragma unroll
     for (int q = 0; q < SPEC_E; q++) {
-      sp[q] += ak * co[q];
-      const double c = co[q] * cr[q] - si[q] * sr[q];
-      si[q] = si[q] * cr[q] + co[q] * sr[q];
-      co[q] = c;
+      sincos((double)k0 * th[q], &si[q], &co[q]);
+      sincos((double)SPEC_T * th[q], &sr[q], &cr[q]);
+    }
+#pragma unroll 4
+    for (int k = k0; k <= kmax; k += SPEC_T) {
+      const double ak = a[k];
+#pragma unroll
+      for (int q = 0; q < SPEC_E; q++) {
+        sp[q] += ak * co[q];
+        const double c = co[q] * cr[q] - si[q] * sr[q];
+        si[q] = si[q] * cr[q] + co[q] * sr[q];
+        co[q] = c;
+      }
     }
   }
 #pragma unroll
@@ -935,9 +980,8 @@ __global__ __launch_bounds__(SPEC_T) void k_spectrum(const double* __restrict__ 
   if (threadIdx.x < SPEC_E && i < ne) {
     const double Es = (e[i] - emindlt) / delta2;
     double x = a[0];
-    for (int w = 0; w < SPEC_T / 64; w++) x += red[w][threadIdx.x];
-    x = x / (sqrt(1.0 - Es * Es) * delta2);
-    spec[i] = isnan(x) ? 0.0 : x;
+    for (int w = 0; w < nw; w++) x += red[w][threadIdx.x];
+    spec[i] = spec_value(x, Es, delta2);
   }
 }
 
@@ -948,7 +992,13 @@ hipError_t launch_spectrum(hipStream_t s, const double* d_auto, double* d_a, int
                      0, s, d_auto, d_a, kmax, hbr, xkgam);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(k_spectrum, dim3((unsigned)((ne + SPEC_E - 1) / SPEC_E)), dim3(SPEC_T), 0, s,
+  if (kmax <= SPEC_DIRECT && ne >= (kmax < 32 ? 16384 : 40960)) {
+    hipLaunchKernelGGL(k_spec_direct, dim3((unsigned)((ne + 255) / 256)), dim3(256), 0, s, d_a,
+                       kmax, d_e, ne, emindlt, delta2, d_spec);
+    return hipGetLastError();
+  }
+  const int nt = std::max(64, std::min(SPEC_T, (kmax + 63) / 64 * 64));
+  hipLaunchKernelGGL(k_spectrum, dim3((unsigned)((ne + SPEC_E - 1) / SPEC_E)), dim3(nt), 0, s,
                      d_a, kmax, d_e, ne, emindlt, delta2, d_spec);
   return hipGetLastError();
 }
