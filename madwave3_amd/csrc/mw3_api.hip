@@ -194,8 +194,12 @@ static hipError_t alloc_ring(Ctx* c, bool prod) {
   double* p[3] = {nullptr, nullptr, nullptr};
   const size_t n[3] = {nw, ns, np};
   hipError_t e = hipSuccess;
-  for (int i = 0; i < 3 && e == hipSuccess; i++)
-    if (n[i]) e = alloc_zero((void**)&p[i], sizeof(double) * d * n[i]);
+  for (int i = 0; i < 3 && e == hipSuccess; i++) {
+    if (!n[i]) continue;
+    // (rows of a slice without kept points stay zero; a step writes all of the others)
+    e = i == 1 ? alloc_zero((void**)&p[i], sizeof(double) * d * n[i])
+               : hipMalloc((void**)&p[i], sizeof(double) * d * n[i]);
+  }
   double** const old[3] = {&c->d_norm_part, &c->d_ring_slice, &c->d_up_part};
   if (e == hipSuccess)
     for (int i = 0; i < 3; i++) std::swap(p[i], *old[i]);

@@ -1096,8 +1096,7 @@ static std::vector<GemmBlk> plan_blocks(const std::vector<GemmDesc>& d, int grou
 }
 
 void free_plan(GemmPlan* p) {
-  if (p->d_descs) (void)hipFree(p->d_descs);
-  if (p->d_blks) (void)hipFree(p->d_blks);
+  if (p->d_descs) (void)hipFree(p->d_descs);  // d_blks lies in it
   p->d_descs = nullptr;
   p->d_blks = nullptr;
 }
@@ -1107,13 +1106,14 @@ static hipError_t upload_plan(GemmPlan* p, const std::vector<GemmDesc>& d, bool 
   p->vec = plan_vec_ok(d, p->st, akc) ? 1 : 0;
   const std::vector<GemmBlk> b = plan_blocks(d, p->group, p->share_b, need);
   p->nblk = (int)b.size();
-  hipError_t e = hipMalloc(&p->d_descs, sizeof(GemmDesc) * std::max<size_t>(d.size(), 1));
-  if (e == hipSuccess)
-    e = hipMemcpy(p->d_descs, d.data(), sizeof(GemmDesc) * d.size(), hipMemcpyHostToDevice);
-  if (e == hipSuccess) e = hipMalloc(&p->d_blks, sizeof(GemmBlk) * std::max<size_t>(b.size(), 1));
-  if (e == hipSuccess)
-    e = hipMemcpy(p->d_blks, b.data(), sizeof(GemmBlk) * b.size(), hipMemcpyHostToDevice);
-  return e;
+  const size_t nd = sizeof(GemmDesc) * d.size(), nb = sizeof(GemmBlk) * b.size();
+  std::vector<char> both(nd + nb + 1);
+  if (nd) memcpy(both.data(), d.data(), nd);
+  if (nb) memcpy(both.data() + nd, b.data(), nb);
+  hipError_t e = hipMalloc((void**)&p->d_descs, both.size());
+  if (e != hipSuccess) return e;
+  p->d_blks = (GemmBlk*)((char*)p->d_descs + nd);
+  return hipMemcpy(p->d_descs, both.data(), both.size(), hipMemcpyHostToDevice);
 }
 
 // whether every descriptor of a plan meets the vector kernel's alignment
@@ -3804,10 +3804,19 @@ hipError_t build_plans(Ctx* c) {
   if (tiles_fit && (c->ang_nt || (c->ang_fused && offs32) || cor_try)) {
     const int64_t tw = 16 * ANG_WAVES, tpc = (plane + tw - 1) / tw;
     std::vector<uint8_t> act((size_t)tpc, 0);  // bit w: wave w's 16 columns
-    for (int ia = 0; ia < t.na; ia++)
-      for (int64_t q = 0; q < plane; q++)
-        if (t.mask[(size_t)ia * plane + q])
+    for (int64_t q = 0; q < plane; q += 16) {
+      const size_t n = (size_t)std::min<int64_t>(16, plane - q);
+      for (int ia = 0; ia < t.na; ia++) {
+        uint64_t v[2] = {0, 0};
+        const uint8_t* m = &t.mask[(size_t)ia * plane + q];
+        if (n == 16) memcpy(v, m, 16);
+        else memcpy(v, m, n);
+        if (v[0] | v[1]) {
           act[(size_t)(q / tw)] |= (uint8_t)(1u << ((q % tw) / 16));
+          break;
+        }
+      }
+    }
     std::vector<int32_t> tl, gl;
     for (int ch = 0; ch < t.nc; ch++)
       for (int64_t k = 0; k < tpc; k++)

@@ -19,6 +19,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <cstring>
 #include <type_traits>
 #include <vector>
 
@@ -923,15 +924,6 @@ __global__ __launch_bounds__(512, 4) void k_rad_rr(RrArgs a) {
 // ---------------------------------------------------------------------------
 // host side
 // ---------------------------------------------------------------------------
-template <typename T>
-static hipError_t upload_t(void** dst, const std::vector<double>& v) {
-  std::vector<T> x(v.begin(), v.end());
-  const size_t n = sizeof(T) * std::max<size_t>(x.size(), 1);
-  hipError_t e = hipMalloc(dst, n);
-  if (e != hipSuccess || x.empty()) return e;
-  return hipMemcpy(*dst, x.data(), sizeof(T) * x.size(), hipMemcpyHostToDevice);
-}
-
 template <typename U>
 static hipError_t upload_v(U** dst, const std::vector<U>& v) {
   hipError_t e = hipMalloc((void**)dst, sizeof(U) * std::max<size_t>(v.size(), 1));
@@ -995,33 +987,45 @@ static hipError_t build(Ctx* c) {
   const int NT = c->up_nt, SW = 16 * NT, ns = (n2 + SW - 1) / SW;
   const int nrt = (n1 + 15) / 16;
   std::vector<uint32_t> tiles;
+  tiles.reserve((size_t)na * ns * nrt * 16);
   std::vector<int32_t> first((size_t)na * ns), cnt((size_t)na * ns);
+  // bit x: kept point R + x of a row (x < 16 NT), eight mask bytes (0 or 1) to a
+  // product whose top byte gathers them
+  auto row_bits = [&](const uint8_t* row, int R) {
+    uint32_t b = 0;
+    for (int x = 0; x < SW && R + x < n2; x += 8) {
+      uint64_t v = 0;
+      if (R + x + 8 <= n2) std::memcpy(&v, row + R + x, 8);
+      else std::memcpy(&v, row + R + x, (size_t)(n2 - R - x));
+      b |= (uint32_t)((v * 0x0102040810204080ull) >> 56) << x;
+    }
+    return b;
+  };
   for (int ia = 0; ia < na; ia++)
     for (int s = 0; s < ns; s++) {
       const size_t q0 = (size_t)ia * ns + s;
       first[q0] = (int32_t)(tiles.size() / 64);
       for (int rt = 0; rt < nrt; rt++) {
-        uint32_t w[64];
-        uint32_t any = 0;
-        for (int lane = 0; lane < 64; lane++) {
-          w[lane] = 0;
-          for (int q = 0; q < 4; q++)
-            for (int k = 0; k < NT; k++) {
-              const int r = 16 * rt + Mma<T>::row(lane >> 4, q);
-              const int R = s * SW + NT * (lane & 15) + k;
-              if (r < n1 && R < n2 && t.mask[(size_t)ia * t.nplane + (size_t)r * n2 + R])
-                w[lane] |= 1u << (q * NT + k);
-            }
-          any |= w[lane];
+        uint32_t b[16], any = 0;
+        for (int i = 0; i < 16; i++) {
+          const int r = 16 * rt + i;
+          b[i] = r < n1 ? row_bits(&t.mask[(size_t)ia * t.nplane + (size_t)r * n2], s * SW) : 0u;
+          any |= b[i];
         }
         if (!any) continue;
-        for (int lane = 0; lane < 64; lane++) tiles.push_back((uint32_t)rt << 8 | w[lane]);
+        for (int lane = 0; lane < 64; lane++) {
+          uint32_t w = (uint32_t)rt << 8;
+          for (int q = 0; q < 4; q++)
+            w |= ((b[Mma<T>::row(lane >> 4, q)] >> (NT * (lane & 15))) & ((1u << NT) - 1u))
+                 << (q * NT);
+          tiles.push_back(w);
+        }
       }
       cnt[q0] = (int32_t)(tiles.size() / 64) - first[q0];
     }
   // S(r, k1) per r size, zero at r >= nn1 and past the size's low modes
   const int kp = 16 * c->up_nk1;
-  std::vector<double> tab;
+  std::vector<T> tab;
   std::vector<int> off((size_t)na, 0), qoff(t.dst_sizes.size(), -1);
   for (int ia = 0; ia < na && kp; ia++) {
     int q = 0;
@@ -1036,13 +1040,13 @@ static hipError_t build(Ctx* c) {
           for (int l = 0; l < 256; l++) {
             const int r = 16 * rt + (l >> 2) % 16, k = 16 * j + 4 * (l >> 6) + l % 4;
             tab.push_back(r < t.nn1[ia] && k < kcap
-                              ? t.dst_tables[(size_t)t.low_off[q] + (size_t)k * t.low_ld[q] + r]
-                              : 0.0);
+                              ? (T)t.dst_tables[(size_t)t.low_off[q] + (size_t)k * t.low_ld[q] + r]
+                              : (T)0);
           }
     }
     off[ia] = qoff[q];
   }
-  if ((e = upload_t<T>(&c->d_up_tab, tab)) != hipSuccess) return e;
+  if ((e = upload_v((T**)&c->d_up_tab, tab)) != hipSuccess) return e;
   // Waves.  Few strips (every strip's block resident at once): a block per
   // strip, its waves an equal part each, so that a strip is one segment.  Else
   // runs of equal length over all channels' tiles, for as many waves as are
@@ -1077,6 +1081,7 @@ static hipError_t build(Ctx* c) {
   std::vector<UpSeg> segs;
   std::vector<uint32_t> lists;
   std::vector<int32_t> sfirst;
+  lists.reserve((size_t)(aligned ? kUpWaves * nstrip : (total + tmax - 1) / tmax) * tmax * 64);
   int segmax = 1;
   for (int ch = 0; ch < t.nc; ch++)
     for (int ia = 0; ia < na; ia++)
@@ -1132,10 +1137,11 @@ static hipError_t build(Ctx* c) {
   int q2 = 0;
   while (t.dst_sizes[q2] != n2) q2++;
   auto S = [&](int j, int k) {
-    return j < ke && k < k2max ? t.dst_tables[(size_t)t.low_off[q2] + (size_t)k * t.low_ld[q2] + j]
-                               : 0.0;
+    return j < ke && k < k2max ? (T)t.dst_tables[(size_t)t.low_off[q2] + (size_t)k * t.low_ld[q2] + j]
+                               : (T)0;
   };
-  std::vector<double> tf, tb;
+  std::vector<T> tf((size_t)nb * 2 * NP * 256), tb(tf.size());
+  size_t o = 0;
   // back: row i of a table tile gives D's row i, which is to be R offset
   // 4 g + r where i = row(g, r); its columns are the modes that result
   // register r of lane group g holds
@@ -1145,27 +1151,28 @@ static hipError_t build(Ctx* c) {
   for (int b = 0; b < nb; b++)
     for (int p = 0; p < 2; p++)
       for (int u = 0; u < NP; u++)
-        for (int l = 0; l < 256; l++) {
+        for (int l = 0; l < 256; l++, o++) {
           const int lg = l >> 6, li = (l >> 2) % 16, x = l % 4;
-          tf.push_back(S(16 * b + 4 * lg + x, 2 * (16 * u + li) + p));
-          tb.push_back(S(16 * b + inv[li], 2 * (16 * u + Mma<T>::row(lg, x)) + p));
+          tf[o] = S(16 * b + 4 * lg + x, 2 * (16 * u + li) + p);
+          tb[o] = S(16 * b + inv[li], 2 * (16 * u + Mma<T>::row(lg, x)) + p);
         }
-  std::vector<double> wt;
+  std::vector<T> wt((size_t)na * c->up_nk1 * 2 * NP * 256);
+  o = 0;
   for (int ia = 0; ia < na; ia++)
     for (int mt = 0; mt < c->up_nk1; mt++)
       for (int p = 0; p < 2; p++)
         for (int u = 0; u < NP; u++)
-          for (int l = 0; l < 256; l++) {
+          for (int l = 0; l < 256; l++, o++) {
             const int k1 = 16 * mt + (l >> 2) % 16;
             const int k2 = 2 * (16 * u + Mma<T>::row(l >> 6, l % 4)) + p;
             double w = 0.0;
             if (k1 < t.k1lo[ia] && k2 < t.k2lo[ia])
               w = t.radcut - (t.p2r1[(size_t)ia * n1 + k1] + t.p2r2[k2]);
-            wt.push_back(w > 0.0 ? w * t.divi[ia] : 0.0);
+            wt[o] = (T)(w > 0.0 ? w * t.divi[ia] : 0.0);
           }
-  if ((e = upload_t<T>(&c->d_rr_w, wt)) != hipSuccess) return e;
-  if ((e = upload_t<T>(&c->d_rr_f, tf)) != hipSuccess) return e;
-  if ((e = upload_t<T>(&c->d_rr_b, tb)) != hipSuccess) return e;
+  if ((e = upload_v((T**)&c->d_rr_w, wt)) != hipSuccess) return e;
+  if ((e = upload_v((T**)&c->d_rr_f, tf)) != hipSuccess) return e;
+  if ((e = upload_v((T**)&c->d_rr_b, tb)) != hipSuccess) return e;
   if ((e = zalloc(&c->d_g1, sizeof(T) * (size_t)segs.size() * k1max * SW)) != hipSuccess) return e;
   return zalloc(&c->d_g2, sizeof(T) * (size_t)t.nc * na * k1max * ns * SW);
 }
