@@ -346,7 +346,8 @@ MW3_API int32_t mw3_set_option(mw3_ctx *ctx, int32_t option, int32_t value);
 MW3_API int32_t mw3_get_option(const mw3_ctx *ctx, int32_t option, int32_t *value);
 
 /* The autotuner (no counterpart in the reference): times trial_steps
-   (2..254, rounded down to even) Chebyshev steps of the context under every
+   (2..254, rounded down to even, from 16 on to runs of 16, which long calls
+   are made of) Chebyshev steps of the context under every
    combination of the options above that the context can run, from its
    current state, and keeps the fastest.  The state, k and every accumulator
    are as before the call (the trial steps are discarded: no ring flush, no

@@ -1151,21 +1151,26 @@ int32_t mw3_get_option(const mw3_ctx* ctx, int32_t option, int32_t* value) {
   return MW3_OK;
 }
 
-// One autotuner trial: the context's current options over n steps after those
-// that capture the graphs these n need, from the current state, timed with events on the main stream
-// once every stream has joined it.  No ring flush, no psi(E) sum.
+// One autotuner trial: the context's current options over n steps from the
+// current state, timed with events on the main stream once every stream has
+// joined it.  No ring flush, no psi(E) sum.  The steps before them capture every
+// graph: whether or not the first runs by itself to form G, and from either
+// buffer, four more steps than the longest run go through that run and both
+// single steps.  The timed steps start from buffer 0, where runs of kRun start.
 static int trial_ms(Ctx* c, int n, hipEvent_t e0, hipEvent_t e1, double* ms) {
-  int32_t done = 0;
   c->trial = true;
-  int rc = MW3_OK;
-  const int warm = n >= kRun ? kRun + 2 : 2;
-  while (done < warm && rc == MW3_OK) rc = step_enqueue(c, &done, warm, nullptr, nullptr, kRun);
-  if (rc == MW3_OK) {
-    HIPCHK(c, hipEventRecord(e0, c->stream), "mw3_autotune: event");
-    done = 0;
-    while (done < n && rc == MW3_OK) rc = step_enqueue(c, &done, n, nullptr, nullptr, kRun);
-  }
+  auto steps = [&](int m) {
+    int rc = MW3_OK;
+    for (int32_t done = 0; done < m && rc == MW3_OK;)
+      rc = step_enqueue(c, &done, m, nullptr, nullptr, kRun);
+    return rc;
+  };
+  int rc = steps(n >= kRun ? kRun + 4 : 4);
+  if (rc == MW3_OK && c->d_psi != c->graph_psi0) rc = steps(1);
+  hipError_t e = hipSuccess;
+  if (rc == MW3_OK && (e = hipEventRecord(e0, c->stream)) == hipSuccess) rc = steps(n);
   c->trial = false;
+  HIPCHK(c, e, "mw3_autotune: event");
   if (rc) return rc;
   HIPCHK(c, hipEventRecord(e1, c->stream), "mw3_autotune: event");
   HIPCHK(c, hipEventSynchronize(e1), "mw3_autotune: sync");
@@ -1180,7 +1185,8 @@ int32_t mw3_autotune(mw3_ctx* ctx, int32_t trial_steps, int32_t* chosen, double*
   if (!c) return MW3_EINVAL;
   if (trial_steps < 2 || trial_steps > kRing - 2)
     return seterr(c, MW3_EINVAL, "mw3_autotune: trial_steps must be in 2..254");
-  const int n = trial_steps & ~1;  // even: the psi buffers end where they began
+  // whole runs of steps, as a long call enqueues them, where there is one
+  const int n = trial_steps >= kRun ? trial_steps / kRun * kRun : trial_steps & ~1;
   int rc = flush_ring(c, nullptr, nullptr);
   if (rc) return rc;
   HIPCHK(c, hipStreamSynchronize(c->stream), "mw3_autotune: sync");
@@ -1190,6 +1196,8 @@ int32_t mw3_autotune(mw3_ctx* ctx, int32_t trial_steps, int32_t* chosen, double*
   const size_t bytes = sizeof(double) * (size_t)c->t.nc * c->t.nslab;
   double* const p0 = c->d_psi;
   double* const pm0 = c->d_psim1;
+  float* const q0 = c->d_psi32;
+  float* const qm0 = c->d_psim132;
   HIPCHK(c, hipMemcpyAsync(c->d_hout, c->d_psi, bytes, hipMemcpyDeviceToDevice, c->stream),
          "mw3_autotune: save");
   HIPCHK(c, hipMemcpyAsync(c->d_scratch, c->d_psim1, bytes, hipMemcpyDeviceToDevice, c->stream),
@@ -1254,9 +1262,11 @@ int32_t mw3_autotune(mw3_ctx* ctx, int32_t trial_steps, int32_t* chosen, double*
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
   c->timing = timing;
-  // restore the state (an even number of trial steps leaves the buffers in place)
+  // restore the state
   c->d_psi = p0;
   c->d_psim1 = pm0;
+  c->d_psi32 = q0;
+  c->d_psim132 = qm0;
   c->k = k0;
   c->ring_k0 = rk0;
   c->ring_fill = c->sum_from = 0;

@@ -1,6 +1,6 @@
 """What libmw3 asks of the HIP runtime, on a runtime without a device
 (tests/fakehip.c, loaded in a process of its own): device memory of a context, blocks
-of the update."""
+of the update, what the autotuner times."""
 import json
 import os
 import subprocess
@@ -109,3 +109,31 @@ def test_update_fills_the_chip(fake):
         print(k, n1, blocks)
         assert 0 < blocks <= (256 if 24 * n1 > 80 * 1024 else 512)
         assert n1 < 1000 or blocks > 200
+
+
+TUNE = """
+for prec in (0, 1):
+    for first in (0, 1):
+        for n in (2, 4, 16, 20, 48):
+            g = L.Propagator(case(32, 64, 16), prec)
+            g.begin(g.case.rpaq0)
+            if first:
+                g.steps(1)
+            log()
+            g.autotune(n)
+            out["%d %d %d" % (prec, first, n)] = log()
+            g.close()
+"""
+
+
+def test_autotuner_times_steps_only(fake):
+    """No capture between a trial's events, and the graph trials of 16 steps and
+    more time the runs of 16 that a long call is made of."""
+    for key, s in fake(TUNE).items():
+        n = int(key.split()[-1])
+        parts = s.split("T")
+        assert len(parts) % 2 == 1 and len(parts) > 8
+        timed = parts[1::2]
+        assert not any(c in t for t in timed for c in "CIk"), (key, timed)
+        graphs = "K" + "G" * (n // 16 if n >= 16 else n)  # (K: the ring slot of the first)
+        assert graphs in timed and all(t == graphs or "G" not in t for t in timed), (key, timed)
