@@ -1077,7 +1077,6 @@ int32_t mw3_set_option(mw3_ctx* ctx, int32_t option, int32_t value) {
   if (!c) return MW3_EINVAL;
   int rc = flush_ring(c, nullptr, nullptr);  // no step of the old setting left pending
   if (rc) return rc;
-  c->g_fresh = false;
   switch (option) {
     case MW3_OPT_GRAPHS:
       if (value != 0 && value != 1) return seterr(c, MW3_EINVAL, "mw3_set_option: graphs 0 or 1");
@@ -1085,7 +1084,10 @@ int32_t mw3_set_option(mw3_ctx* ctx, int32_t option, int32_t value) {
       return MW3_OK;
     case MW3_OPT_RADIAL:
       if (value != 0 && value != 1) return seterr(c, MW3_EINVAL, "mw3_set_option: radial 0 or 1");
-      if (value != c->opt_radial) drop_graphs(c);
+      if (value != c->opt_radial) {
+        drop_graphs(c);
+        c->g_fresh = false;  // only the low-mode steps leave G
+      }
       c->opt_radial = value;
       return MW3_OK;
     case MW3_OPT_ANGULAR:
@@ -1108,9 +1110,7 @@ int32_t mw3_set_option(mw3_ctx* ctx, int32_t option, int32_t value) {
     case MW3_OPT_RADIAL_GRID:
       if (value != 1 && value != 2 && value != 4)
         return seterr(c, MW3_EINVAL, "mw3_set_option: radial grid divisor 1, 2 or 4");
-      if (value != c->opt_rad_grid) drop_graphs(c);
-      c->opt_rad_grid = value;
-      return MW3_OK;
+      return MW3_OK;  // no radial kernel has a grid to divide
     case MW3_OPT_FP16_PRODUCTS:
       if (value != 0 && value != 1)
         return seterr(c, MW3_EINVAL, "mw3_set_option: fp16 products 0 or 1");
@@ -1218,7 +1218,6 @@ int32_t mw3_autotune(mw3_ctx* ctx, int32_t trial_steps, int32_t* chosen, double*
     c->opt_radial = k[MW3_OPT_RADIAL];
     c->opt_angular = k[MW3_OPT_ANGULAR];
     c->opt_side = k[MW3_OPT_SIDE_STREAM];
-    c->opt_rad_grid = k[MW3_OPT_RADIAL_GRID];
     c->opt_ang_grid = k[MW3_OPT_ANGULAR_GRID];
     c->opt_fp16 = k[MW3_OPT_FP16_PRODUCTS];
   };
@@ -1229,21 +1228,20 @@ int32_t mw3_autotune(mw3_ctx* ctx, int32_t trial_steps, int32_t* chosen, double*
     for (int r = 0; r <= 1; r++)
       for (int a = 0; a <= 2; a++)
         for (int sd = 0; sd <= 1; sd++)
-          for (int gd = 1; gd <= 4; gd *= 2)
-            for (int ag = 1; ag <= 2; ag++) {
-              Key k;
-              k[MW3_OPT_GRAPHS] = g;
-              k[MW3_OPT_RADIAL] = r;
-              k[MW3_OPT_ANGULAR] = a;
-              k[MW3_OPT_SIDE_STREAM] = sd;
-              k[MW3_OPT_RADIAL_GRID] = gd;
-              k[MW3_OPT_ANGULAR_GRID] = ag;
-              k[MW3_OPT_FP16_PRODUCTS] = best_key[MW3_OPT_FP16_PRODUCTS];  // kept as set
-              apply(k);
-              Key eff;
-              effective_options(c, eff.data());
-              if (std::find(cands.begin(), cands.end(), eff) == cands.end()) cands.push_back(eff);
-            }
+          for (int ag = 1; ag <= 2; ag++) {
+            Key k;
+            k[MW3_OPT_GRAPHS] = g;
+            k[MW3_OPT_RADIAL] = r;
+            k[MW3_OPT_ANGULAR] = a;
+            k[MW3_OPT_SIDE_STREAM] = sd;
+            k[MW3_OPT_RADIAL_GRID] = 1;
+            k[MW3_OPT_ANGULAR_GRID] = ag;
+            k[MW3_OPT_FP16_PRODUCTS] = best_key[MW3_OPT_FP16_PRODUCTS];  // kept as set
+            apply(k);
+            Key eff;
+            effective_options(c, eff.data());
+            if (std::find(cands.begin(), cands.end(), eff) == cands.end()) cands.push_back(eff);
+          }
   double best = 1e30;
   for (const auto& key : cands) {
     drop_graphs(c);

@@ -312,7 +312,6 @@ struct Ctx {
   // GEMMs (2), each falling back to the next where not built; the angular
   // term on the third stream (1) or the main one (0)
   int opt_radial = 1, opt_angular = 0, opt_side = 0;
-  int opt_rad_grid = 1;           // accepted; no kernel has a radial grid to divide
   int opt_ang_grid = 1;           // folded angular kernel: blocks per channel / this
   int flux_etest = 1;             // E > V(flux point) test when the flux sums are read
   bool trial = false;             // autotuner trial steps: no ring flush, no psi(E)

@@ -1,6 +1,6 @@
 """What libmw3 asks of the HIP runtime, on a runtime without a device
 (tests/fakehip.c, loaded in a process of its own): device memory of a context, blocks
-of the update, what the autotuner times."""
+of the update, what the autotuner times, what an option without effect costs."""
 import json
 import os
 import subprocess
@@ -137,3 +137,33 @@ def test_autotuner_times_steps_only(fake):
         assert not any(c in t for t in timed for c in "CIk"), (key, timed)
         graphs = "K" + "G" * (n // 16 if n >= 16 else n)  # (K: the ring slot of the first)
         assert graphs in timed and all(t == graphs or "G" not in t for t in timed), (key, timed)
+
+
+OPTION = """
+for prec in (0, 1):
+    g = L.Propagator(case(32, 64, 16), prec)
+    g.begin(g.case.rpaq0)
+    g.steps(40)
+    log()
+    for v in (2, 4, 1):
+        g.set_option(L.MW3_OPT_RADIAL_GRID, v)
+    g.steps(32)
+    s = log()
+    out[prec] = s
+    bad = 0
+    try:
+        g.set_option(L.MW3_OPT_RADIAL_GRID, 3)
+    except L.Mw3Error:
+        bad = 1
+    out["%d bad" % prec] = bad
+    g.close()
+"""
+
+
+def test_option_without_effect_keeps_graphs(fake):
+    """MW3_OPT_RADIAL_GRID takes 1, 2 and 4 (and refuses others), and the steps after
+    it run as the graphs captured before it."""
+    out = fake(OPTION)
+    for prec in "01":
+        assert "C" not in out[prec] and "I" not in out[prec] and "G" in out[prec], out[prec]
+        assert out[prec + " bad"] == 1
