@@ -152,16 +152,16 @@ struct Ctx {
   int up_ring = kRun;
   int sum_from = 0;
   int up_nwaves = 0, up_nseg = 0, up_tmax = 0, up_nt = 1, up_ns = 0, up_segmax = 0;
-  int up_nk1 = 0;                 // 16-mode tiles of the low r modes (0: radial GEMMs only)
+  int up_nk1 = 0;                 // 16-mode tiles of the low r modes (0: no r products here)
   int up_kst = 0;                 // low r modes kept of G, G2
   int rr_np = 0, rr_nb = 0;       // k2 tiles per parity, 16-R blocks of a half row
   double* d_up_row = nullptr;     // [16 ceil(n1/16)][4] absfr1, zAR1flux
-  void* d_up_tab = nullptr;       // S(r, k1) per r size
-  void* d_rr_f = nullptr;         // S(R, k2) by parity, forward and back order
-  void* d_rr_b = nullptr;
-  void* d_rr_w = nullptr;         // weights (radcut - E)_+ divi
-  void* d_g1 = nullptr;           // G of psi_k, segment sums [up_nseg][up_kst][16 up_nt]
-  void* d_g2 = nullptr;           // [nc na][up_ns][up_kst][16 up_nt]
+  double* d_up_tab = nullptr;     // FP64: S(r, k1) per r size
+  double* d_rr_f = nullptr;       // S(R, k2) by parity, forward and back order
+  double* d_rr_b = nullptr;
+  double* d_rr_w = nullptr;       // weights (radcut - E)_+ divi
+  double* d_g1 = nullptr;         // G of psi_k, segment sums [up_nseg][up_kst][16]
+  double* d_g2 = nullptr;         // [nc na][up_ns][up_kst][16]
   bool g_fresh = false;           // d_g1 is G of d_psi
   void* d_v = nullptr;  // double or float dense V
   double* d_absfr1 = nullptr;
@@ -401,7 +401,7 @@ hipError_t step_build_f32(Ctx* c);
 hipError_t step_build_f64(Ctx* c);
 hipError_t step_update_f32(Ctx* c, const step::UpArgs& a, int nk1, int cpl, int aux, int mode);
 hipError_t step_update_f64(Ctx* c, const step::UpArgs& a, int nk1, int cpl, int aux, int mode);
-hipError_t step_rad_rr_f64(Ctx* c, const step::RrArgs& a);
+hipError_t step_rad_rr(Ctx* c, const step::RrArgs& a);
 void timer_begin(Ctx* c, int id, hipStream_t s = nullptr);
 void timer_end(Ctx* c, int id, hipStream_t s = nullptr);
 

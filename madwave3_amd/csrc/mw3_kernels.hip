@@ -4100,9 +4100,9 @@ static hipError_t hpsi_impl(Ctx* c, const double* psi64) {
     }
     timer_begin(c, K_DST_r);
     const step::RrArgs ra{c->d_g1, c->d_g2, c->d_rr_f, c->d_rr_b, c->d_rr_w, t.na, t.n1, t.n2,
-                          c->up_nk1, c->up_kst, c->rr_nb, c->d_up_sfirst, c->up_ns,
-                          c->up_nt == 2 ? 5 : 4, c->up_segmax};
-    if ((e = step_rad_rr_f64(c, ra)) != hipSuccess) return e;
+                          c->up_nk1, c->up_kst, c->rr_nb, c->d_up_sfirst, c->up_ns, 4,
+                          c->up_segmax};
+    if ((e = step_rad_rr(c, ra)) != hipSuccess) return e;
     timer_end(c, K_DST_r);
   } else {
     timer_begin(c, K_DST_R);

@@ -3,8 +3,8 @@
 // mw3_step_f32.hip and mw3_step_f64.hip).
 //
 // The radial term is T psi = c psi - S (c - E)_+ divi S psi on the low modes
-// k1 < k1lo, k2 < k2lo (mw3_setup.cpp).  The products over r come first and
-// last, so that both ride in the update, which has every r row of its columns
+// k1 < k1lo, k2 < k2lo (mw3_setup.cpp).  In FP64 the products over r come first
+// and last, so that both ride in the update, which has every r row of its columns
 // in hand:
 //   update of the step before:  G[k1][R]  = sum_r S(r, k1) psi(r, R)
 //   k_rad_rr:                   G2[k1][R] = sum_k2 S(R, k2) (c - E(k1, k2))_+ divi
@@ -12,7 +12,10 @@
 //   update:                     corr[r][R] = sum_k1 S(r, k1) G2[k1][R]
 // psi is then read once for the radial term (as the update's own psi), and
 // neither the transformed rows nor the correction pass through a dense slab:
-// G and G2 hold k1lo rows instead of n1 (38 of 256 at 256 x 512 x 120).
+// G and G2 hold k1lo rows instead of n1 (38 of 256 at 256 x 512 x 120).  Mixed
+// precision forms the correction before the update, with the products over R
+// first (the order of its FP32 sums is part of its results), and its update reads
+// it.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -20,7 +23,6 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
-#include <type_traits>
 #include <vector>
 
 #include "mw3_internal.h"
@@ -40,11 +42,8 @@ struct Mma<double> {
   static __host__ __device__ constexpr int row(int g, int r) { return 4 * r + g; }
 };
 template <>
-struct Mma<float> {
+struct Mma<float> {  // (no r products: the rows alone)
   typedef float V __attribute__((ext_vector_type(4)));
-  static __device__ __forceinline__ V mma(float a, float b, V c) {
-    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-  }
   static __host__ __device__ constexpr int row(int g, int r) { return 4 * g + r; }
 };
 
@@ -167,13 +166,14 @@ static __device__ __forceinline__ void stvn(T* p, const T (&v)[N]) {
 // and nothing moves between lanes.  FP32 takes two R per lane (whole 128-byte
 // lines per row), FP64 one.
 //
-// Bound by memory: at 256 x 512 x 120 (6.0 M kept points) a step moves 32
+// Bound by memory: at 256 x 512 x 120 (5.55 M kept points) a step moves 40
 // bytes per point in mixed precision (psi32 4, psi_{k-1} 8, angular and radial
-// slabs and V 12, stores 12, plus the projections), 48 us, 45 measured (with
-// the angular kernel beside it 51); the row-item form before it, one wave per
-// 64 R, took 54 and a second stream's sums.  In FP64 the two r products are
-// 2 x 16.5 GFLOP of matrix work under the loads: 75 us, in place of 54 us plus
-// an R-first radial term of 82 us (R passes 62, r passes 20).  Equal runs:
+// slabs and V 12, product weights 4, stores 12), 43 us at the rate of a large copy
+// (5.2 TB/s), 45 measured (with the angular kernel beside it 51); the row-item
+// form before it, one wave per 64 R, took 54 and a second stream's sums.  In FP64
+// it moves 48 (51 us), and the two r products are 2 x 0.66 GFLOP of matrix work
+// under the loads (18 us at the rate of a large product): 75 us, in place of 76 us
+// plus an R-first radial term of 98 us (R passes 72, r passes 26).  Equal runs:
 // a block per strip left the last blocks alone at 74 (mixed) and 104 us.
 // ---------------------------------------------------------------------------
 constexpr int kUpWaves = 4;  // waves per block
@@ -203,10 +203,10 @@ struct UpArgs {
   const double* rowtab;  // [n1][4]: absfr1, Re and Im zAR1flux, 0
   // tables are stored in the order the lanes read them (one contiguous load
   // per wave: rows at a stride of a power of two meet on the same cache sets)
-  const void* tab;       // S(r, k1) [size][row tile][NK1][lane (g, i)][4]: row i,
+  const double* tab;     // S(r, k1) [size][row tile][NK1][lane (g, i)][4]: row i,
                          // k1 = 16 j + 4 g + q
-  const void* g2;        // [nc na][strip][kst][16 NT]
-  void* g1;              // [nseg][kst][16 NT]
+  const double* g2;      // [nc na][strip][kst][16]
+  double* g1;            // [nseg][kst][16]
   int ns, kst;           // strips of a row, rows of G2
   const double* psi;     // psi_k
   const void* psi32;     // its FP32 copy (mixed precision)
@@ -248,16 +248,17 @@ template <typename T, int NK1, int NT, int CPL, int AUX, int MODE>
 __global__ __launch_bounds__(64 * kUpWaves, 2) void k_update(UpArgs a) {
   typedef typename Mma<T>::V V;
   constexpr bool M32 = sizeof(T) == 4;
-  constexpr bool P32 = M32 && MODE >= 2;  // psi_k from its FP32 copy
+  static_assert(NK1 == 0 ? MODE != 3 : !M32, "the r products are FP64's");
+  constexpr bool P32 = M32 && MODE == 2;  // psi_k from its FP32 copy
   constexpr int SW = 16 * NT, KP = 16 * NK1, NKA = NK1 > 0 ? NK1 : 1;
   constexpr bool FWD = NK1 > 0 && MODE >= 2, BACK = NK1 > 0 && MODE != 3;
   constexpr bool PRODP = (AUX & 1) && MODE == 2, AUTO = (AUX & 2) && MODE != 3;
   constexpr int NCPL = CPL == 1 ? 3 : 1;
   constexpr uint32_t ES = sizeof(T);
-  // LDS, per wave: G2 of the strip (rows padded so that the lane groups of a
-  // read fall on different banks) and a tile's table rows; for all: the r rows'
+  // LDS, per wave: G2 of the strip and a tile's table rows (padded so that the
+  // lane groups of a read fall on different banks); for all: the r rows'
   // absorption factors and flux weights
-  constexpr int LG = SW + (M32 ? 8 : 0), LS = KP + (M32 ? 4 : NK1 % 4 ? 0 : 4);
+  constexpr int LG = SW, LS = KP + (NK1 % 4 ? 0 : 4);
   constexpr int NG = BACK ? KP * LG : 0, NSTG = FWD ? 16 * LS : 0;
   __shared__ __align__(16) T lds[kUpWaves * (NG + NSTG) > 0 ? kUpWaves * (NG + NSTG) : 4];
   // sums of a first segment that belongs to a wave before
@@ -321,7 +322,7 @@ __global__ __launch_bounds__(64 * kUpWaves, 2) void k_update(UpArgs a) {
       }
     }
     if constexpr (BACK) {
-      const T* g2 = (const T*)a.g2 + ((int64_t)s.cia * a.ns + s.strip) * a.kst * SW;
+      const T* g2 = a.g2 + ((int64_t)s.cia * a.ns + s.strip) * a.kst * SW;
       constexpr int NV = KP * SW / 256;  // 4-value vectors per lane
       T y[NV][4];
 #pragma unroll
@@ -367,7 +368,7 @@ __global__ __launch_bounds__(64 * kUpWaves, 2) void k_update(UpArgs a) {
     const int64_t vb = (int64_t)s.ia * plane + ro, base = (int64_t)s.c * slab + vb;
     const int R0 = s.strip * SW + NT * i;
     if constexpr (NK1 > 0) {
-      const T* tr = (const T*)a.tab + s.taboff + (int64_t)rt * (16 * KP) + 4 * lane;
+      const T* tr = a.tab + s.taboff + (int64_t)rt * (16 * KP) + 4 * lane;
 #pragma unroll
       for (int j = 0; j < NK1; j++) ldv4(tr + 256 * j, av[j]);
     }
@@ -463,7 +464,7 @@ __global__ __launch_bounds__(64 * kUpWaves, 2) void k_update(UpArgs a) {
 #pragma unroll
             for (int t = 0; t < NT; t++)
               acc[m][t][r] += hacc[wave + k][(m * 4 * NT + r * NT + t) * 64 + lane];
-      T* g1 = (T*)a.g1 + (int64_t)s.seg * a.kst * SW + NT * i;
+      T* g1 = a.g1 + (int64_t)s.seg * a.kst * SW + NT * i;
 #pragma unroll
       for (int m = 0; m < NK1; m++)
 #pragma unroll
@@ -528,10 +529,7 @@ __global__ __launch_bounds__(64 * kUpWaves, 2) void k_update(UpArgs a) {
 #pragma unroll
       for (int q = 0; q < 4; q++)
 #pragma unroll
-        for (int t = 0; t < NT; t++) {
-          const T x = M32 ? (T)pf[q][t] : (T)pd[q][t];
-          bv[q][t] = ((keep >> (q * NT + t)) & 1u) ? x : (T)0;
-        }
+        for (int t = 0; t < NT; t++) bv[q][t] = ((keep >> (q * NT + t)) & 1u) ? (T)pd[q][t] : (T)0;
     } else {
       // the coupled channels' V and psi, in flight during the back product
       T cv[NCPL][4][NT];
@@ -717,7 +715,7 @@ __global__ __launch_bounds__(64 * kUpWaves, 2) void k_update(UpArgs a) {
 }
 
 // ---------------------------------------------------------------------------
-// k_rad_rr: G -> G2 of one (channel, angle) and 16 modes k1: fold over R,
+// k_rad_rr (FP64): G -> G2 of one (channel, angle) and 16 modes k1: fold over R,
 // sum over R to the low k2 modes of both parities, weights, and back to R.
 // S(n2-1-R, k2) = (-1)^k2 S(R, k2), so with u = G[R] + G[n2-1-R] and
 // v = G[R] - G[n2-1-R] the even modes see u and the odd ones v, and back
@@ -727,26 +725,31 @@ __global__ __launch_bounds__(64 * kUpWaves, 2) void k_update(UpArgs a) {
 // the quarters' partial tiles), in the second an eighth of the R tiles.  The
 // first product's result layout is the second one's right operand as it
 // stands.  A wave runs each loop only a few times, so the time is that of a
-// chain of memory latencies: the next block's loads, and the second product's
-// first table rows, are in flight behind the products.  29 us at 256 x 512 x
-// 120 (38 k1 by 77 k2 modes of 120 angles).
+// chain of memory latencies: the next block's G is in flight behind the products.
+// The tables are read where they are used; their registers would push the
+// block's second copy off the CU.  29 us at 256 x 512 x 120 (38 k1 by 77 k2 modes
+// of 120 angles).
 // ---------------------------------------------------------------------------
 struct RrArgs {
-  const void* g1;
-  void* g2;
-  const void* tf;  // [nb][parity][NP][lane (g, i)][4]: S(j, 2 k + parity), k = 16 t + i,
-                   // j = 16 jb + 4 g + e
-  const void* tb;  // [nb][parity][NP][lane][4]: the back product's, in MFMA order
-  const void* wt;  // weights (c - E(k1, k2))_+ divi [na][k1 tile][parity][NP][lane][4] of
-                   // the first product's results
+  const double* g1;
+  double* g2;
+  const double* tf;  // [nb][parity][NP][lane (g, i)][4]: S(j, 2 k + parity), k = 16 t + i,
+                     // j = 16 jb + 4 g + e
+  const double* tb;  // [nb][parity][NP][lane][4]: the back product's, in MFMA order
+  const double* wt;  // weights (c - E(k1, k2))_+ divi [na][k1 tile][parity][NP][lane][4] of
+                     // the first product's results
   int na, n1, n2, nk1, kst, nb;
   const int32_t* sfirst;  // [nc na ns + 1] first segment of each strip
-  int ns, swl, segmax;    // strips per row, log2 of their width, most segments of one
+  // strips per row, log2 of their width (4; as a constant the addresses built on it
+  // are all formed ahead, which spills: 28.9 us against 28.6), most segments of one
+  int ns, swl, segmax;
 };
 
-template <typename T, int NP, bool VEC>
+template <int NP, bool VEC>
 __global__ __launch_bounds__(512, 4) void k_rad_rr(RrArgs a) {
-  typedef typename Mma<T>::V V;
+  typedef double T;
+  typedef Mma<T> M;
+  typedef M::V V;
   constexpr uint32_t ES = sizeof(T);
   __shared__ V red[4][2][NP][64];
   const int lane = threadIdx.x & 63;
@@ -758,8 +761,8 @@ __global__ __launch_bounds__(512, 4) void k_rad_rr(RrArgs a) {
   const int n2 = a.n2, nb = a.nb, h = n2 / 2, ke = n2 - h, kst = a.kst, swl = a.swl, sw = 1 << swl;
   const int k1 = 16 * mt + i, k1c = k1 < kst ? k1 : kst - 1;
   if (mt * 16 >= kst) return;  // no row of this tile is kept
-  const T* tf = (const T*)a.tf + par * NP * 256 + 4 * lane;
-  const T* tb = (const T*)a.tb;
+  const T* tf = a.tf + par * NP * 256 + 4 * lane;
+  const T* tb = a.tb;
   const int32_t* sf = a.sfirst + (int64_t)cia * a.ns;
   const int64_t segw = (int64_t)kst * sw;  // values of a segment
   // segments 0 and 1 of the strip that holds the 16-column block b, 4 columns
@@ -767,44 +770,32 @@ __global__ __launch_bounds__(512, 4) void k_rad_rr(RrArgs a) {
   // reads zero, without a memory access
   auto gload = [&](int b, int c, T (&y)[2][4]) {
     const int s = (16 * b) >> swl, s0 = sf[s], n = sf[s + 1] - s0;
-    const Rsrc r = rsrc((const T*)a.g1 + s0 * segw, (uint32_t)((n < 2 ? n : 2) * segw) * ES);
+    const Rsrc r = rsrc(a.g1 + s0 * segw, (uint32_t)((n < 2 ? n : 2) * segw) * ES);
     const uint32_t o = (uint32_t)(k1c * sw + 16 * b - s * sw + c) * ES;
 #pragma unroll
     for (int q = 0; q < 2; q++) {
       const uint32_t oq = o + q * (uint32_t)segw * ES;
-      if constexpr (ES == 8) {
-        T z0[2], z1[2];
-        bld<T, 2>(r, oq, z0);
-        bld<T, 2>(r, oq + 16u, z1);
-        y[q][0] = z0[0], y[q][1] = z0[1], y[q][2] = z1[0], y[q][3] = z1[1];
-      } else {
-        bld<T, 4>(r, oq, y[q]);
-      }
+      T z0[2], z1[2];
+      bld<T, 2>(r, oq, z0);
+      bld<T, 2>(r, oq + 16u, z1);
+      y[q][0] = z0[0], y[q][1] = z0[1], y[q][2] = z1[0], y[q][3] = z1[1];
     }
   };
   // the same columns of the segments from k on
   auto gmore = [&](int o, int k, T (&y)[4]) {
     const int s = o >> swl, s1 = sf[s + 1];
     for (int q = sf[s] + k; q < s1; q++) {
-      const T* G = (const T*)a.g1 + q * segw + k1c * sw + (o - s * sw);
+      const T* G = a.g1 + q * segw + k1c * sw + (o - s * sw);
 #pragma unroll
       for (int e = 0; e < 4; e++) y[e] += G[e];
     }
   };
-  // FP64: the tables are read where they are used (their registers would push
-  // the block's second copy off the CU)
-  constexpr bool PF = ES == 4;
-  T an[NP][4], xn[2][4], mn[2][4];
-  auto ftab = [&](int jb) {
-#pragma unroll
-    for (int t = 0; t < NP; t++) ldv4(tf + (int64_t)(jb * 2 * NP + t) * 256, an[t]);
-  };
+  T xn[2][4], mn[2][4];
   auto prefetch = [&](int jb) {
     if constexpr (VEC) {
       gload(jb, 4 * g, xn);
       gload(n2 / 16 - 1 - jb, 12 - 4 * g, mn);
     }
-    if constexpr (PF) ftab(jb);
   };
   V acc[NP];
 #pragma unroll
@@ -814,11 +805,8 @@ __global__ __launch_bounds__(512, 4) void k_rad_rr(RrArgs a) {
   for (int jb = jw; jb < nb; jb += 4) {
     T at[NP][4], xs[4] = {0, 0, 0, 0}, ms[4] = {0, 0, 0, 0}, u[4];
     const int j0 = 16 * jb + 4 * g;
-    if constexpr (!PF) ftab(jb);
 #pragma unroll
-    for (int e = 0; e < 4; e++)
-#pragma unroll
-      for (int t = 0; t < NP; t++) at[t][e] = an[t][e];
+    for (int t = 0; t < NP; t++) ldv4(tf + (int64_t)(jb * 2 * NP + t) * 256, at[t]);
     if constexpr (VEC) {
       T mm[4] = {0, 0, 0, 0};
 #pragma unroll
@@ -838,7 +826,7 @@ __global__ __launch_bounds__(512, 4) void k_rad_rr(RrArgs a) {
       for (int e = 0; e < 4; e++) {
         const int o1 = n2 - 1 - j0 - e, o = o1 > 0 ? o1 : 0, s = o >> swl;
         for (int q = sf[s]; q < sf[s + 1]; q++)
-          ms[e] += ((const T*)a.g1)[q * segw + k1c * sw + (o - s * sw)];
+          ms[e] += a.g1[q * segw + k1c * sw + (o - s * sw)];
       }
     }
     if (jb + 4 < nb) prefetch(jb + 4);
@@ -852,22 +840,13 @@ __global__ __launch_bounds__(512, 4) void k_rad_rr(RrArgs a) {
 #pragma unroll
     for (int e = 0; e < 4; e++)
 #pragma unroll
-      for (int t = 0; t < NP; t++) acc[t] = Mma<T>::mma(at[t][e], u[e], acc[t]);
+      for (int t = 0; t < NP; t++) acc[t] = M::mma(at[t][e], u[e], acc[t]);
   }
-  T ae[NP][4], ao[NP][4];
-  auto btab = [&](int rt) {
-#pragma unroll
-    for (int t = 0; t < NP; t++) {
-      ldv4(tb + (int64_t)(rt * 2 * NP + t) * 256 + 4 * lane, ae[t]);
-      ldv4(tb + (int64_t)(rt * 2 * NP + NP + t) * 256 + 4 * lane, ao[t]);
-    }
-  };
 #pragma unroll
   for (int t = 0; t < NP; t++) red[jw][par][t][lane] = acc[t];
-  if (PF && wave < nb) btab(wave);
   T wt[2][NP][4];
   {
-    const T* w = (const T*)a.wt + (int64_t)(ia * a.nk1 + mt) * (2 * NP * 256) + 4 * lane;
+    const T* w = a.wt + (int64_t)(ia * a.nk1 + mt) * (2 * NP * 256) + 4 * lane;
 #pragma unroll
     for (int p = 0; p < 2; p++)
 #pragma unroll
@@ -884,20 +863,24 @@ __global__ __launch_bounds__(512, 4) void k_rad_rr(RrArgs a) {
 #pragma unroll
       for (int r = 0; r < 4; r++) hw[p][t][r] = s[r] * wt[p][t][r];
     }
-  T* out = (T*)a.g2 + (int64_t)cia * a.ns * segw + k1 * sw;
+  T* out = a.g2 + (int64_t)cia * a.ns * segw + k1 * sw;
   auto at2 = [&](int R) { return out + (R >> swl) * segw + (R & (sw - 1)); };  // column R of row k1
 #pragma unroll 1
   for (int rt = wave; rt < nb; rt += 8) {
     V e = {0, 0, 0, 0}, o = {0, 0, 0, 0};
-    if constexpr (!PF) btab(rt);
+    T ae[NP][4], ao[NP][4];
+#pragma unroll
+    for (int t = 0; t < NP; t++) {
+      ldv4(tb + (int64_t)(rt * 2 * NP + t) * 256 + 4 * lane, ae[t]);
+      ldv4(tb + (int64_t)(rt * 2 * NP + NP + t) * 256 + 4 * lane, ao[t]);
+    }
 #pragma unroll
     for (int t = 0; t < NP; t++)
 #pragma unroll
       for (int r = 0; r < 4; r++) {
-        e = Mma<T>::mma(ae[t][r], hw[0][t][r], e);
-        o = Mma<T>::mma(ao[t][r], hw[1][t][r], o);
+        e = M::mma(ae[t][r], hw[0][t][r], e);
+        o = M::mma(ao[t][r], hw[1][t][r], o);
       }
-    if (PF && rt + 8 < nb) btab(rt + 8);
     const int R = 16 * rt + 4 * g;  // registers r: R + r
     if (k1 >= kst) continue;
     if constexpr (VEC) {
@@ -962,7 +945,62 @@ static hipError_t resident(const Ctx* c, int* blocks) {
   }
 }
 
-// strips, tiles and (where the low modes fit the kernels) tables of the step
+// FP64: the tables of k_rad_rr (S(R, k2) by parity for the R products, and the
+// weights), G and G2
+static hipError_t build_rr(Ctx* c, int k1max, int k2max) {
+  typedef Mma<double> M;
+  const HostTables& t = c->t;
+  const int n1 = t.n1, n2 = t.n2, na = t.na;
+  const int h = n2 / 2, ke = n2 - h, nb = (ke + 15) / 16, NP = c->rr_np;
+  c->up_kst = k1max;
+  c->rr_nb = nb;
+  int q2 = 0;
+  while (t.dst_sizes[q2] != n2) q2++;
+  auto S = [&](int j, int k) {
+    return j < ke && k < k2max ? t.dst_tables[(size_t)t.low_off[q2] + (size_t)k * t.low_ld[q2] + j]
+                               : 0.0;
+  };
+  std::vector<double> tf((size_t)nb * 2 * NP * 256), tb(tf.size());
+  size_t o = 0;
+  // back: row i of a table tile gives D's row i, which is to be R offset
+  // 4 g + r where i = row(g, r); its columns are the modes that result
+  // register r of lane group g holds
+  int inv[16];
+  for (int g = 0; g < 4; g++)
+    for (int r = 0; r < 4; r++) inv[M::row(g, r)] = 4 * g + r;
+  for (int b = 0; b < nb; b++)
+    for (int p = 0; p < 2; p++)
+      for (int u = 0; u < NP; u++)
+        for (int l = 0; l < 256; l++, o++) {
+          const int lg = l >> 6, li = (l >> 2) % 16, x = l % 4;
+          tf[o] = S(16 * b + 4 * lg + x, 2 * (16 * u + li) + p);
+          tb[o] = S(16 * b + inv[li], 2 * (16 * u + M::row(lg, x)) + p);
+        }
+  std::vector<double> wt((size_t)na * c->up_nk1 * 2 * NP * 256);
+  o = 0;
+  for (int ia = 0; ia < na; ia++)
+    for (int mt = 0; mt < c->up_nk1; mt++)
+      for (int p = 0; p < 2; p++)
+        for (int u = 0; u < NP; u++)
+          for (int l = 0; l < 256; l++, o++) {
+            const int k1 = 16 * mt + (l >> 2) % 16;
+            const int k2 = 2 * (16 * u + M::row(l >> 6, l % 4)) + p;
+            double w = 0.0;
+            if (k1 < t.k1lo[ia] && k2 < t.k2lo[ia])
+              w = t.radcut - (t.p2r1[(size_t)ia * n1 + k1] + t.p2r2[k2]);
+            wt[o] = w > 0.0 ? w * t.divi[ia] : 0.0;
+          }
+  hipError_t e;
+  const size_t row = sizeof(double) * (size_t)k1max * 16;
+  if ((e = upload_v(&c->d_rr_w, wt)) != hipSuccess) return e;
+  if ((e = upload_v(&c->d_rr_f, tf)) != hipSuccess) return e;
+  if ((e = upload_v(&c->d_rr_b, tb)) != hipSuccess) return e;
+  if ((e = zalloc((void**)&c->d_g1, row * (size_t)c->up_nseg)) != hipSuccess) return e;
+  return zalloc((void**)&c->d_g2, row * (size_t)t.nc * na * c->up_ns);
+}
+
+// strips and tiles of the update, and in FP64, where the low modes fit the
+// kernels, tables of the radial products
 template <typename T>
 static hipError_t build(Ctx* c) {
   const HostTables& t = c->t;
@@ -1025,7 +1063,7 @@ static hipError_t build(Ctx* c) {
     }
   // S(r, k1) per r size, zero at r >= nn1 and past the size's low modes
   const int kp = 16 * c->up_nk1;
-  std::vector<T> tab;
+  std::vector<double> tab;
   std::vector<int> off((size_t)na, 0), qoff(t.dst_sizes.size(), -1);
   for (int ia = 0; ia < na && kp; ia++) {
     int q = 0;
@@ -1040,13 +1078,13 @@ static hipError_t build(Ctx* c) {
           for (int l = 0; l < 256; l++) {
             const int r = 16 * rt + (l >> 2) % 16, k = 16 * j + 4 * (l >> 6) + l % 4;
             tab.push_back(r < t.nn1[ia] && k < kcap
-                              ? (T)t.dst_tables[(size_t)t.low_off[q] + (size_t)k * t.low_ld[q] + r]
-                              : (T)0);
+                              ? t.dst_tables[(size_t)t.low_off[q] + (size_t)k * t.low_ld[q] + r]
+                              : 0.0);
           }
     }
     off[ia] = qoff[q];
   }
-  if ((e = upload_v((T**)&c->d_up_tab, tab)) != hipSuccess) return e;
+  if (kp && (e = upload_v(&c->d_up_tab, tab)) != hipSuccess) return e;
   // Waves.  Few strips (every strip's block resident at once): a block per
   // strip, its waves an equal part each, so that a strip is one segment.  Else
   // runs of equal length over all channels' tiles, for as many waves as are
@@ -1129,52 +1167,7 @@ static hipError_t build(Ctx* c) {
   if ((e = upload_v((UpSeg**)&c->d_up_seg, segs)) != hipSuccess) return e;
   if ((e = upload_v(&c->d_up_tile, lists)) != hipSuccess) return e;
   if ((e = upload_v(&c->d_up_sfirst, sfirst)) != hipSuccess) return e;
-  if (!c->up_nk1) return hipSuccess;
-  c->up_kst = k1max;
-  // S(R, k2) by parity for the R products
-  const int h = n2 / 2, ke = n2 - h, nb = (ke + 15) / 16, NP = c->rr_np;
-  c->rr_nb = nb;
-  int q2 = 0;
-  while (t.dst_sizes[q2] != n2) q2++;
-  auto S = [&](int j, int k) {
-    return j < ke && k < k2max ? (T)t.dst_tables[(size_t)t.low_off[q2] + (size_t)k * t.low_ld[q2] + j]
-                               : (T)0;
-  };
-  std::vector<T> tf((size_t)nb * 2 * NP * 256), tb(tf.size());
-  size_t o = 0;
-  // back: row i of a table tile gives D's row i, which is to be R offset
-  // 4 g + r where i = row(g, r); its columns are the modes that result
-  // register r of lane group g holds
-  int inv[16];
-  for (int g = 0; g < 4; g++)
-    for (int r = 0; r < 4; r++) inv[Mma<T>::row(g, r)] = 4 * g + r;
-  for (int b = 0; b < nb; b++)
-    for (int p = 0; p < 2; p++)
-      for (int u = 0; u < NP; u++)
-        for (int l = 0; l < 256; l++, o++) {
-          const int lg = l >> 6, li = (l >> 2) % 16, x = l % 4;
-          tf[o] = S(16 * b + 4 * lg + x, 2 * (16 * u + li) + p);
-          tb[o] = S(16 * b + inv[li], 2 * (16 * u + Mma<T>::row(lg, x)) + p);
-        }
-  std::vector<T> wt((size_t)na * c->up_nk1 * 2 * NP * 256);
-  o = 0;
-  for (int ia = 0; ia < na; ia++)
-    for (int mt = 0; mt < c->up_nk1; mt++)
-      for (int p = 0; p < 2; p++)
-        for (int u = 0; u < NP; u++)
-          for (int l = 0; l < 256; l++, o++) {
-            const int k1 = 16 * mt + (l >> 2) % 16;
-            const int k2 = 2 * (16 * u + Mma<T>::row(l >> 6, l % 4)) + p;
-            double w = 0.0;
-            if (k1 < t.k1lo[ia] && k2 < t.k2lo[ia])
-              w = t.radcut - (t.p2r1[(size_t)ia * n1 + k1] + t.p2r2[k2]);
-            wt[o] = (T)(w > 0.0 ? w * t.divi[ia] : 0.0);
-          }
-  if ((e = upload_v((T**)&c->d_rr_w, wt)) != hipSuccess) return e;
-  if ((e = upload_v((T**)&c->d_rr_f, tf)) != hipSuccess) return e;
-  if ((e = upload_v((T**)&c->d_rr_b, tb)) != hipSuccess) return e;
-  if ((e = zalloc(&c->d_g1, sizeof(T) * (size_t)segs.size() * k1max * SW)) != hipSuccess) return e;
-  return zalloc(&c->d_g2, sizeof(T) * (size_t)t.nc * na * k1max * ns * SW);
+  return c->up_nk1 ? build_rr(c, k1max, k2max) : hipSuccess;
 }
 
 template <typename T, int NK1, int NT, int CPL, int AUX, int MODE>
@@ -1225,25 +1218,13 @@ static hipError_t update(Ctx* c, const UpArgs& a, int nk1, int cpl, int aux, int
   return hipGetLastError();
 }
 
-template <typename T, int NP>
+template <int NP>
 static void launch_rr(Ctx* c, const RrArgs& a) {
   const unsigned nb = (unsigned)(c->t.nc * c->t.na * c->up_nk1);
   if (c->t.n2 % 16 == 0)
-    hipLaunchKernelGGL((k_rad_rr<T, NP, true>), dim3(nb), dim3(512), 0, c->stream, a);
+    hipLaunchKernelGGL((k_rad_rr<NP, true>), dim3(nb), dim3(512), 0, c->stream, a);
   else
-    hipLaunchKernelGGL((k_rad_rr<T, NP, false>), dim3(nb), dim3(512), 0, c->stream, a);
-}
-
-template <typename T>
-static hipError_t rad_rr(Ctx* c, const RrArgs& a) {
-  switch (c->rr_np) {
-    case 1: launch_rr<T, 1>(c, a); break;
-    case 2: launch_rr<T, 2>(c, a); break;
-    case 3: launch_rr<T, 3>(c, a); break;
-    case 4: launch_rr<T, 4>(c, a); break;
-    default: return hipErrorInvalidValue;
-  }
-  return hipGetLastError();
+    hipLaunchKernelGGL((k_rad_rr<NP, false>), dim3(nb), dim3(512), 0, c->stream, a);
 }
 
 }  // namespace step
