@@ -180,34 +180,24 @@ const char* mw3_kernel_name(int32_t id) {
   return names[id];
 }
 
-// The buffers for what the updates leave per step (norms, slices, segment sums:
-// of the flux line's three rows, and a fourth with product weights), in place of
-// those there; nothing changes on failure.
-static hipError_t alloc_ring(Ctx* c, bool prod) {
-  const HostTables& t = c->t;
-  const size_t nw = 2 * (size_t)std::max(1, c->up_nwaves);
-  const size_t ns = t.ncvj > 0 ? (size_t)t.nc * t.n1 * t.na : 0;
-  const size_t np = t.nflux > 0 || prod
-                        ? (size_t)std::max(1, c->up_nseg) * (prod ? 4 : 3) * 16 * c->up_nt
-                        : 0;
-  const int d = ring_depth(sizeof(double) * (nw + ns + np));
-  double* p[3] = {nullptr, nullptr, nullptr};
-  const size_t n[3] = {nw, ns, np};
-  hipError_t e = hipSuccess;
-  for (int i = 0; i < 3 && e == hipSuccess; i++) {
-    if (!n[i]) continue;
-    // (rows of a slice without kept points stay zero; a step writes all of the others)
-    e = i == 1 ? alloc_zero((void**)&p[i], sizeof(double) * d * n[i])
-               : hipMalloc((void**)&p[i], sizeof(double) * d * n[i]);
-  }
-  double** const old[3] = {&c->d_norm_part, &c->d_ring_slice, &c->d_up_part};
-  if (e == hipSuccess)
-    for (int i = 0; i < 3; i++) std::swap(p[i], *old[i]);
-  for (double* q : p)
-    if (q) (void)hipFree(q);
-  if (e == hipSuccess) c->up_ring = d;
-  return e;
+// The buffer for the segment sums the updates leave (the flux line's three rows,
+// and a fourth with product weights), in place of the one there; nothing changes
+// on failure.
+static hipError_t alloc_segments(Ctx* c, bool prod) {
+  if (!prod && c->t.nflux == 0) return hipSuccess;
+  const size_t n = (size_t)std::max(1, c->up_nseg) * (prod ? 4 : 3) * 16 * c->up_nt;
+  const int d = ring_depth(sizeof(double) * n);
+  double* p = nullptr;  // (a step writes all of its place)
+  const hipError_t e = hipMalloc((void**)&p, sizeof(double) * d * n);
+  if (e != hipSuccess) return e;
+  if (c->d_up_part) (void)hipFree(c->d_up_part);
+  c->d_up_part = p;
+  c->seg_ring = d;
+  return hipSuccess;
 }
+
+// the ring starts anew: nothing of it is left to sum
+static void ring_reset(Ctx* c) { c->ring_fill = c->seg_from = c->slice_from = 0; }
 
 int32_t mw3_create(const mw3_setup* setup, int32_t precision, mw3_ctx** out) {
   if (!out) return seterr(nullptr, MW3_EINVAL, "mw3_create: out is NULL");
@@ -386,7 +376,16 @@ int32_t mw3_create(const mw3_setup* setup, int32_t precision, mw3_ctx** out) {
     CK(alloc_zero((void**)&c->d_zfe, sizeof(double) * 2 * setup->nofe * nd), "mw3_create: zfe");
   }
   CK(build_plans(c), "mw3_create: plans");
-  CK(alloc_ring(c, false), "mw3_create: sums of the steps");
+  CK(hipMalloc((void**)&c->d_norm_part,
+               sizeof(double) * 2 * kRing * (size_t)std::max(1, c->up_nwaves)),
+     "mw3_create: norms");
+  CK(alloc_segments(c, false), "mw3_create: segment sums");
+  if (t.ncvj > 0) {  // (rows without kept points stay zero)
+    const size_t n = (size_t)t.nc * t.n1 * t.na;
+    c->slice_ring = ring_depth(sizeof(double) * n);
+    CK(alloc_zero((void**)&c->d_ring_slice, sizeof(double) * c->slice_ring * n),
+       "mw3_create: slices");
+  }
   CK(hipStreamSynchronize(c->stream), "mw3_create: sync");
 #undef CK
   *out = reinterpret_cast<mw3_ctx*>(c);
@@ -439,7 +438,7 @@ static int clear_accumulators(Ctx* c) {
     HIPCHK(c, launch_zero(c, c->d_zs2prod, sizeof(double) * 2 * nx * netot), "clear");
     HIPCHK(c, launch_zero(c, c->d_cvjp_last, sizeof(double) * nx), "clear");
   }
-  c->ring_fill = c->sum_from = 0;
+  ring_reset(c);
   return MW3_OK;
 }
 
@@ -465,7 +464,7 @@ int32_t mw3_cheby_begin(mw3_ctx* ctx, const double* psi0, double* stats3) {
                              hipMemcpyDeviceToHost, c->stream),
            "mw3_cheby_begin: sums");
   }
-  c->ring_fill = c->sum_from = 0;
+  ring_reset(c);
   c->rec_it.clear();
   c->rec_cvj.clear();
   c->rec_cvjp.clear();
@@ -488,7 +487,7 @@ static size_t rec_nprod(const Ctx* c) {
 
 static int flush_ring(Ctx* c, double* norms_dst, double* auto_dst) {
   if (c->ring_fill == 0) return MW3_OK;
-  HIPCHK(c, launch_ring_sums(c), "ring sums");
+  HIPCHK(c, launch_ring_sums(c, S_ALL), "ring sums");
   HIPCHK(c, launch_energy_accum(c), "energy accumulation");
   std::vector<double> nb(2 * (size_t)c->ring_fill);
   HIPCHK(c, hipMemcpyAsync(nb.data(), c->d_ring_norm, nb.size() * sizeof(double),
@@ -516,7 +515,7 @@ static int flush_ring(Ctx* c, double* norms_dst, double* auto_dst) {
     if (auto_dst) auto_dst[i] = nb[2 * i + 1];
   }
   c->ring_k0 += c->ring_fill;
-  c->ring_fill = c->sum_from = 0;
+  ring_reset(c);
   if (c->timing) timer_collect(c);
   return MW3_OK;
 }
@@ -587,10 +586,13 @@ static bool step_pre(Ctx* c) {
 // The sums of the ring's steps so far, where the next `run` steps would take the
 // place of what they are formed from (none in a trial, whose ring is not read).
 static int ring_room(Ctx* c, int run) {
-  if (c->trial || c->ring_fill - c->sum_from + run <= c->up_ring) return MW3_OK;
+  const int end = c->ring_fill + run;
+  const int which = (end - c->seg_from > c->seg_ring ? S_SEG : 0) |
+                    (end - c->slice_from > c->slice_ring ? S_SLICE : 0);
+  if (c->trial || !which) return MW3_OK;
   const bool timed = c->timing_step;
   c->timing_step = true;  // like the energy sums: every ring's are timed
-  const hipError_t e = launch_ring_sums(c);
+  const hipError_t e = launch_ring_sums(c, which);
   c->timing_step = timed;
   HIPCHK(c, e, "mw3_cheby_steps: ring sums");
   return MW3_OK;
@@ -638,7 +640,7 @@ static int step_post(Ctx* c, int32_t* done, int32_t nsteps, double* norms,
   *done += 1;
   if (c->trial && (c->ring_fill == kRing || *done == nsteps)) {
     // autotuner trial: the ring is discarded unread
-    c->ring_fill = c->sum_from = 0;
+    ring_reset(c);
     return MW3_OK;
   }
   if (c->ring_fill == kRing || *done == nsteps) {
@@ -980,7 +982,7 @@ int32_t mw3_prod_attach(mw3_ctx* ctx, const mw3_prod_setup* ps) {
   if (e == hipSuccess) e = alloc_zero((void**)&c->d_cvjp_last, sizeof(double) * nx);
   if (e == hipSuccess) e = alloc_zero((void**)&c->d_zs2prod, sizeof(double) * 2 * nx * netot);
   if (e == hipSuccess) e = build_prod_plan(c);
-  if (e == hipSuccess) e = alloc_ring(c, true);
+  if (e == hipSuccess) e = alloc_segments(c, true);
   if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
   if (e != hipSuccess) {
     free_prod(c);
@@ -1267,7 +1269,7 @@ int32_t mw3_autotune(mw3_ctx* ctx, int32_t trial_steps, int32_t* chosen, double*
   c->d_psim132 = qm0;
   c->k = k0;
   c->ring_k0 = rk0;
-  c->ring_fill = c->sum_from = 0;
+  ring_reset(c);
   c->g_fresh = false;
   HIPCHK(c, hipMemcpyAsync(c->d_psi, c->d_hout, bytes, hipMemcpyDeviceToDevice, c->stream),
          "mw3_autotune: restore");

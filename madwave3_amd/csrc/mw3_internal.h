@@ -143,14 +143,15 @@ struct Ctx {
   void* d_up_seg = nullptr;         // [up_nseg] step::UpSeg
   uint32_t* d_up_tile = nullptr;    // [up_nwaves][up_tmax][64]
   int32_t* d_up_sfirst = nullptr;   // [nc na up_ns + 1] first segment of each strip
-  // What the updates leave for the sums of the ring (norms, flux columns,
-  // product weights, slices), for the last up_ring steps: the sums of steps
-  // sum_from .. ring_fill - 1 of the ring are formed before a step takes the
-  // place of one of them.  4 / n1 of a psi slab per step, so as many steps as
-  // fit 64 MB, from one graph launch to a whole ring (ring_depth).
-  double* d_up_part = nullptr;      // [up_ring][up_nseg][3, 4 with products][16 up_nt] sums over r
-  int up_ring = kRun;
-  int sum_from = 0;
+  // What the updates leave for the sums of a ring of steps: per wave (norms, for
+  // the whole ring) and, for the last seg_ring and slice_ring steps, per segment
+  // (flux columns, product weights) and per reactant slice.  The sums of steps
+  // seg_from and slice_from .. ring_fill - 1 of the ring are formed before a step
+  // takes the place of one of them.  A step's segments take about 4 / n1 of a psi
+  // slab, its slices 1 / n2 (ring_depth).
+  double* d_up_part = nullptr;      // [seg_ring][up_nseg][3, 4 with products][16 up_nt] sums over r
+  int seg_ring = kRun, slice_ring = kRun;
+  int seg_from = 0, slice_from = 0;
   int up_nwaves = 0, up_nseg = 0, up_tmax = 0, up_nt = 1, up_ns = 0, up_segmax = 0;
   int up_nk1 = 0;                 // 16-mode tiles of the low r modes (0: no r products here)
   int up_kst = 0;                 // low r modes kept of G, G2
@@ -208,7 +209,7 @@ struct Ctx {
   double* d_fdv = nullptr;
   double* d_dcvj = nullptr;
   uint8_t* d_cvj_skip = nullptr; // [ncvj] 1 if the reference state (kminelastic)
-  double* d_norm_part = nullptr; // update wave sums [up_ring][up_nwaves][2]
+  double* d_norm_part = nullptr; // update wave sums [kRing][up_nwaves][2]
   double* d_stats = nullptr;     // sums of mw3_cheby_begin (launch_stats)
   double* d_ring_norm = nullptr; // [kRing][2] (norm, autocorrelation)
   double* d_efe = nullptr;
@@ -271,7 +272,7 @@ struct Ctx {
 
   int32_t* d_fmap = nullptr;     // [nc][na][n2] flux point index or -1
   int32_t* d_ir1flux = nullptr;  // [na]
-  double* d_ring_slice = nullptr; // [up_ring][nc][na][n1] psi at R = ir2abs / sqrt(ah2)
+  double* d_ring_slice = nullptr; // [slice_ring][nc][na][n1] psi at R = ir2abs / sqrt(ah2)
 
   // product-state projection (iprod = 2, mw3_prod_attach).  Per step, the
   // update leaves funprod(c, l) = sum_r T psi_new (T = transRgjac on the dense
@@ -349,7 +350,8 @@ hipError_t launch_spectrum(hipStream_t s, const double* d_auto, double* d_a, int
 // 0: H psi into d_hout, 1: first step, 2: damped step (psi_new into d_psim1)
 hipError_t launch_update(Ctx* c, int mode, const double* psi, bool proj = false);
 int ring_depth(size_t bytes);
-hipError_t launch_ring_sums(Ctx* c);
+enum { S_NORM = 1, S_SEG = 2, S_SLICE = 4, S_ALL = 7 };
+hipError_t launch_ring_sums(Ctx* c, int which);
 hipError_t launch_energy_accum(Ctx* c);
 hipError_t launch_psie(Ctx* c, int k);
 hipError_t launch_zero(Ctx* c, void* p, size_t bytes);

@@ -629,19 +629,17 @@ hipError_t launch_slot_set(Ctx* c, int q, int v) {
 
 // ---------------------------------------------------------------------------
 // sums over a run of the ring's steps that the update leaves per block, per
-// reactant slice and per channel.  They run once per up_ring steps, one block
+// reactant slice and per channel.  They run for many steps at once, one block
 // (or grid row) per step, instead of as small kernels after every update: step
-// from + blockIdx.x (y) of the ring, at its place modulo up_ring in what the
+// from + blockIdx.y of the ring, at its place modulo the depth of what the
 // updates left.
 // ---------------------------------------------------------------------------
-// (norm, autocorrelation) of a step from the update's block sums
+// (norm, autocorrelation) of step blockIdx.x from the update's block sums
 __global__ __launch_bounds__(256) void k_norm_ring(const double* __restrict__ part_ring, int nb,
-                                                   double* __restrict__ out_ring, int from,
-                                                   int ring) {
+                                                   double* __restrict__ out_ring) {
   typedef double d2 __attribute__((ext_vector_type(2)));
-  const int slot = from + blockIdx.x;
-  const d2* p2 = (const d2*)part_ring + (int64_t)(slot & (ring - 1)) * nb;
-  double* __restrict__ out = out_ring + 2 * (int64_t)slot;
+  const d2* p2 = (const d2*)part_ring + (int64_t)blockIdx.x * nb;
+  double* __restrict__ out = out_ring + 2 * (int64_t)blockIdx.x;
   __shared__ double sh[2][256];
   d2 s0 = {0, 0}, s1 = {0, 0};
   int i = threadIdx.x;
@@ -3937,7 +3935,8 @@ static step::UpArgs update_args(Ctx* c, int mode, const double* psi, bool proj) 
     a.dslot_next = c->d_slot + (1 - q);
   }
   a.slot = c->ring_fill;
-  a.ring = c->up_ring;
+  a.seg_ring = c->seg_ring;
+  a.slice_ring = c->slice_ring;
   a.part = mode == 1 || mode == 2 ? c->d_norm_part : nullptr;
   if (proj && mode == 2) {
     a.slice = t.ncvj > 0 ? c->d_ring_slice : nullptr;
@@ -4170,49 +4169,57 @@ hipError_t launch_update(Ctx* c, int mode, const double* psi, bool proj) {
   return hipSuccess;
 }
 
-// Steps kept for the ring's sums, at `bytes` per step: as many as fit 64 MB,
-// from kRun to kRing.  A whole ring would take 2.4 GB at seven blocks of 192 x
-// 384 x 96 (psi slab 0.4 GB), 16 steps take 0.13.  The sums' three launches per
-// 16 steps are under a hundredth of the step there; grids whose steps are short
-// keep the whole ring.
+// Steps kept of what the updates leave for the ring's sums, at `bytes` per step:
+// as many as fit 128 MB, from kRun to kRing.  Segments of a whole ring would take
+// 2.4 GB at seven blocks of 192 x 384 x 96 (psi slab 0.4 GB), 16 steps 0.10 GB.  The
+// sums of a few steps are launches and latency: at 256 x 512 x 120 9 us for the
+// products, 6 for the flux line and 35 for the reactant states, so that summing
+// all of them every 16 steps made the FP64 step 2% longer; the slices, an eighth
+// of the segments there, keep a depth of their own.
 int ring_depth(size_t bytes) {
   int d = kRing;
-  while (d > kRun && d * bytes > ((size_t)64 << 20)) d /= 2;
+  while (d > kRun && d * bytes > ((size_t)128 << 20)) d /= 2;
   return d;
 }
 
-// per-step sums of the ring's steps from what the updates left, as far as they
-// are not formed yet
-hipError_t launch_ring_sums(Ctx* c) {
+// per-step sums of the ring's steps (S_NORM, S_SEG, S_SLICE) from what the updates
+// left, as far as they are not formed yet
+hipError_t launch_ring_sums(Ctx* c, int which) {
   const HostTables& t = c->t;
-  const int from = c->sum_from, ns = c->ring_fill - from, ring = c->up_ring;
+  const int end = c->ring_fill;
   hipError_t e;
-  if (ns <= 0) return hipSuccess;
   timer_begin(c, K_UPDATE_TAIL);
-  hipLaunchKernelGGL(k_norm_ring, dim3(ns), dim3(256), 0, c->stream, c->d_norm_part,
-                     c->up_nwaves, c->d_ring_norm, from, ring);
+  if ((which & S_NORM) && end > 0)
+    hipLaunchKernelGGL(k_norm_ring, dim3(end), dim3(256), 0, c->stream, c->d_norm_part,
+                       c->up_nwaves, c->d_ring_norm);
   if ((e = hipGetLastError()) != hipSuccess) return e;
-  if (t.nflux > 0) {
-    hipLaunchKernelGGL(k_flux_ring, dim3(nblk(t.nflux, 256), ns), dim3(256), 0, c->stream,
+  const int seg0 = c->seg_from, slice0 = c->slice_from;
+  if ((which & S_SEG) && end > seg0 && t.nflux > 0) {
+    hipLaunchKernelGGL(k_flux_ring, dim3(nblk(t.nflux, 256), end - seg0), dim3(256), 0, c->stream,
                        c->d_up_part, c->d_up_sfirst, c->d_flux_col, c->d_ring_zr, c->d_ring_zdr,
                        t.nflux, c->up_nseg, t.n2, t.nplane, c->up_ns, 16 * c->up_nt,
-                       c->prod_on ? 4 : 3, from, ring);
+                       c->prod_on ? 4 : 3, seg0, c->seg_ring);
     if ((e = hipGetLastError()) != hipSuccess) return e;
   }
   timer_end(c, K_UPDATE_TAIL);
-  if (t.ncvj > 0) {
-    timer_begin(c, K_PROJ);
-    const int nj = c->s.jmax - c->s.jini + 1, nv = c->s.nvmax - c->s.nvini + 1;
-    const int jb = std::max(1, std::min(CVJ_J, 8192 / t.n1));  // within 64 KB of LDS
-    hipLaunchKernelGGL(k_cvj_ring, dim3(t.nc * ((nj + jb - 1) / jb), ns), dim3(256),
-                       sizeof(double) * jb * t.n1, c->stream, c->d_ring_slice, c->d_dcvj,
-                       c->d_fdv, c->d_ring_cvj, t.nc, nj, nv, t.na, t.n1, jb, (int64_t)t.ncvj,
-                       from, ring);
-    if ((e = hipGetLastError()) != hipSuccess) return e;
-    timer_end(c, K_PROJ);
+  if ((which & S_SEG) && end > seg0) {
+    if (c->prod_on && (e = launch_prod_sums(c)) != hipSuccess) return e;
+    c->seg_from = end;
   }
-  if (c->prod_on && (e = launch_prod_sums(c)) != hipSuccess) return e;
-  c->sum_from = c->ring_fill;
+  if ((which & S_SLICE) && end > slice0) {
+    if (t.ncvj > 0) {
+      timer_begin(c, K_PROJ);
+      const int nj = c->s.jmax - c->s.jini + 1, nv = c->s.nvmax - c->s.nvini + 1;
+      const int jb = std::max(1, std::min(CVJ_J, 8192 / t.n1));  // within 64 KB of LDS
+      hipLaunchKernelGGL(k_cvj_ring, dim3(t.nc * ((nj + jb - 1) / jb), end - slice0), dim3(256),
+                         sizeof(double) * jb * t.n1, c->stream, c->d_ring_slice, c->d_dcvj,
+                         c->d_fdv, c->d_ring_cvj, t.nc, nj, nv, t.na, t.n1, jb, (int64_t)t.ncvj,
+                         slice0, c->slice_ring);
+      if ((e = hipGetLastError()) != hipSuccess) return e;
+      timer_end(c, K_PROJ);
+    }
+    c->slice_from = end;
+  }
   return hipSuccess;
 }
 
@@ -4313,11 +4320,11 @@ __global__ void k_prod_sum(const double* __restrict__ part, double* __restrict__
 
 hipError_t launch_prod_sums(Ctx* c) {
   timer_begin(c, K_PROD);
-  hipLaunchKernelGGL(k_prod_fun, dim3(nblk(c->pr_L, 256), c->ring_fill - c->sum_from), dim3(256),
+  hipLaunchKernelGGL(k_prod_fun, dim3(nblk(c->pr_L, 256), c->ring_fill - c->seg_from), dim3(256),
                      0, c->stream,
                      c->d_up_part, c->d_up_sfirst, c->d_dtrans, c->d_ch_elec, c->d_ring_prod,
                      c->t.nc, c->t.ne, c->pr_nomb, c->pr_L, c->t.na, c->pr_nap0, c->pr_n2p0,
-                     c->pr_n2p, c->up_nseg, c->up_ns, 16 * c->up_nt, c->sum_from, c->up_ring);
+                     c->pr_n2p, c->up_nseg, c->up_ns, 16 * c->up_nt, c->seg_from, c->seg_ring);
   const hipError_t e = hipGetLastError();
   timer_end(c, K_PROD);
   return e;

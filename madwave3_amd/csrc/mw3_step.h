@@ -229,14 +229,14 @@ struct UpArgs {
   const int32_t* dslot;
   int32_t* dslot_next;
   int slot;
-  // what the step leaves for the ring's sums, at place slot mod ring (a power
+  // what the step leaves for the ring's sums, at place slot mod its depth (a power
   // of two)
-  int ring;
-  double* part;          // [ring][nwaves][2] (norm, autocorrelation)
-  double* upart;         // [ring][nseg][3 or 4][16 NT]: sum_r of Re and Im zAR1flux
+  double* part;          // [kRing][nwaves][2] (norm, autocorrelation)
+  double* upart;         // [seg_ring][nseg][3 or 4][16 NT]: sum_r of Re and Im zAR1flux
                          // psi, psi at the flux row, with product weights those
                          // times psi; or null
-  double* slice;         // [ring][nc na][n1] or null
+  double* slice;         // [slice_ring][nc na][n1] or null
+  int seg_ring, slice_ring;
   int ir2abs;
 };
 
@@ -282,9 +282,8 @@ __global__ __launch_bounds__(64 * kUpWaves, 2) void k_update(UpArgs a) {
   const uint32_t rb = (uint32_t)n2 * 16u;  // values of a row tile
   T* const gl = lds + wave * (NG + NSTG);
   T* const stg = gl + NG;
-  const int islot = a.dslot ? *a.dslot : a.slot;
-  if (a.dslot_next && blockIdx.x == 0 && threadIdx.x == 0) *a.dslot_next = islot + 1;
-  const int64_t slot = islot & (a.ring - 1);
+  const int slot = a.dslot ? *a.dslot : a.slot;
+  if (a.dslot_next && blockIdx.x == 0 && threadIdx.x == 0) *a.dslot_next = slot + 1;
   if constexpr (MODE != 3)
     for (int k = threadIdx.x; k < 3 * n1; k += 64 * kUpWaves) {
       const int r = k / 3;
@@ -478,7 +477,8 @@ __global__ __launch_bounds__(64 * kUpWaves, 2) void k_update(UpArgs a) {
     }
     if constexpr (MODE == 2) {
       if (a.upart) {
-        double* up = a.upart + (slot * a.nseg + s.seg) * ((PRODP ? 4 : 3) * SW) + NT * i;
+        const int64_t at = (int64_t)(slot & (a.seg_ring - 1)) * a.nseg + s.seg;
+        double* up = a.upart + at * ((PRODP ? 4 : 3) * SW) + NT * i;
 #pragma unroll
         for (int k = 0; k < (PRODP ? 4 : 3); k++) {
           double x[NT];
@@ -664,7 +664,8 @@ __global__ __launch_bounds__(64 * kUpWaves, 2) void k_update(UpArgs a) {
           bst<float, NT>(ro4, so4[q], o32);
         }
         if (MODE == 2 && a.slice && (a.ir2abs - 1) / SW == sg.strip) {
-          double* sl = a.slice + (slot * a.nc * a.na + sg.cia) * (int64_t)n1;
+          double* sl =
+              a.slice + ((int64_t)(slot & (a.slice_ring - 1)) * a.nc * a.na + sg.cia) * n1;
 #pragma unroll
           for (int t = 0; t < NT; t++)
             if (sg.strip * SW + NT * i + t == a.ir2abs - 1 && ((keep >> (q * NT + t)) & 1u))
@@ -707,7 +708,7 @@ __global__ __launch_bounds__(64 * kUpWaves, 2) void k_update(UpArgs a) {
       if constexpr (AUTO) s_auto += __shfl_xor(s_auto, of);
     }
     if (lane0 == 0 && a.part && w < a.nwaves) {
-      double* p = a.part + 2 * (slot * a.nwaves + w);
+      double* p = a.part + 2 * ((int64_t)slot * a.nwaves + w);
       p[0] = s_norm;
       p[1] = s_auto;
     }

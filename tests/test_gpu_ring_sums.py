@@ -1,5 +1,6 @@
 """The sums of a ring of steps where what the updates leave is kept for fewer steps
-than a ring (64 MB: 16 steps at seven blocks of 64 x 256 x 64, 64 at 24 x 512 x 64):
+than a ring (128 MB: 16 steps at seven blocks of 48 x 512 x 64, 32 at 64 x 256 x 64,
+64 or 128 at 24 x 512 x 64, and other depths for segments and slices):
 one long call against many short ones, whose steps are summed as they come, by
 graphs and kernel by kernel.  Norms and per-step records are bitwise the same; the
 energy sums, added up in other groups, to the rounding of 300 terms."""
@@ -29,7 +30,7 @@ def run(c, prec, calls, graphs):
 
 
 @pytest.mark.parametrize("n1,n2,na,J,prec,prod", [(64, 256, 64, 12, MW3_FP64, False),
-                                                  (64, 256, 64, 12, MW3_MIXED, False),
+                                                  (48, 512, 64, 12, MW3_MIXED, False),
                                                   (24, 512, 64, 0, MW3_FP64, True),
                                                   (24, 512, 64, 0, MW3_MIXED, True)])
 def test_ring_places(n1, n2, na, J, prec, prod):

@@ -69,7 +69,8 @@ out["left"] = fake.fake_bytes()
 
 def test_device_memory_of_a_context(fake):
     """Within the slabs, accumulators and tables a propagation needs; what the
-    updates leave for the ring's sums takes at most 64 MB, or 16 steps'."""
+    updates leave for the ring's sums (segments, slices) takes at most 128 MB each, or
+    16 steps'."""
     out = fake(MEMORY)
     assert out.pop("left") == 0
     for r in out.values():
@@ -79,8 +80,9 @@ def test_device_memory_of_a_context(fake):
         state = 5 * 8 * grid + (3 * 4 * grid if r["prec"] else 0)  # psi, psi_{k-1}, psi0, H psi, input
         work = 5 * s * grid + s * grid / r["nc"] + 2 * 8 * r["ntot"]
         accum = r["nflux"] * (32 * r["netot"] + 24 * 256) + r["ncvj"] * (16 * r["netot"] + 8 * 256)
-        step = cols * 4 * 8 * 1.25 + 8 * r["nc"] * r["na"] * r["n1"]  # (strips cut in segments: 1.25)
-        rings = max(64 << 20, 16 * step)
+        seg = cols * 4 * 8 * 1.25  # (strips cut in segments: 1.25)
+        slices = 8 * r["nc"] * r["na"] * r["n1"]
+        rings = sum(min(256 * x, max(128 << 20, 16 * x)) for x in (seg, slices))
         low = 0 if r["prec"] else 2.5 * 8 * 48 * cols  # G, G2
         tables = 0.5 * 8 * grid + (4 << 20)
         limit = state + work + accum + rings + low + tables + r.get("prod", 0) + (
