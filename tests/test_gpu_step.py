@@ -99,3 +99,43 @@ def test_begin_sums(n1, n2, na):
     size = np.array([np.abs(psi * h).sum(), (psi * psi).sum(), (h * h).sum()])
     want = np.array([(psi * h).sum(), (psi * psi).sum(), (h * h).sum()])
     assert np.all(np.abs(g.begin(psi) - want) <= 2.0 * c.ntot * 2.0**-53 * size)
+
+
+# npun1, npun2, nangu, box r, box R (bohr), radial kernels (else GEMMs)
+BEYOND = [
+    (120, 256, 4, 20.0, 15.0, 1),   # more low r modes than the update takes: FP64 R passes in LDS
+    (128, 256, 4, 20.0, 10.0, 1),
+    (112, 320, 4, 20.0, 22.0, 1),
+    (96, 384, 5, 18.0, 6.0, 1),
+    (100, 512, 4, 18.0, 15.0, 1),
+    (2064, 256, 2, 8.0, 15.0, 1),   # more r rows than the update's products take
+    (128, 128, 4, 20.0, 15.0, 0),   # neither update nor R passes: GEMMs
+    (90, 100, 5, 20.0, 15.0, 0),
+    (700, 64, 6, 8.0, 15.0, 1),     # strips cut into many segments, vectorised and not
+    (705, 50, 6, 8.0, 15.0, 1),
+]
+
+
+@pytest.mark.parametrize("n1,n2,na,b1,b2,radial", BEYOND)
+def test_grids_beyond_the_update(n1, n2, na, b1, b2, radial):
+    p = leps.config(1)
+    p.update(npun1=n1, npun2=n2, nangu=na, npun1min=8, jmax=1, nvmax=1, netot=30, iprod=0,
+             kminelastic=4, width_bohr=0.6, absorb_bohr=4.5, rfin1_bohr=b1, rfin2_bohr=b2)
+    c = leps.build(p)
+    print("case", (n1, n2, na, b1, b2), c, flush=True)
+    o = Oracle(c)
+    psi = np.random.default_rng(n1 * 1000 + n2).standard_normal(c.ntot)
+    h = o.hphi(psi)
+    o.begin(c.rpaq0)
+    n_o = o.steps(20)[0]
+    for prec, bar in ((MW3_FP64, 1e-11), (MW3_MIXED, 2e-5)):
+        g = Propagator(c, prec)
+        if prec == MW3_FP64:
+            assert g.get_option(MW3_OPT_RADIAL) == radial
+        assert rel(g.hphi(psi), h) < bar
+        g.begin(c.rpaq0)
+        assert rel(g.steps(20)[0], n_o) < 10 * bar
+        # (of the packet's size at the start: some boxes have absorbed most of it by now)
+        d = np.max(np.abs(g.state()[1] - o.state()[1]))
+        assert d < 10 * bar * np.max(np.abs(c.rpaq0))
+        g.close()
