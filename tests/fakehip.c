@@ -2,6 +2,7 @@
  * counted and never touched, kernels and copies do nothing, captures give empty
  * graphs.  What the library does is logged, one letter per call:
  *   K kernel launch (k while capturing)   C begin of a capture   I instantiation
+ *   w wait of one stream for another while capturing
  *   G graph launch                        T record of a timing event
  * Loaded with global symbols before the library, its functions take the place of
  * the runtime's. */
@@ -69,7 +70,10 @@ err_t hipFuncGetAttributes(void *a, const void *f) { memset(a, 0, 56); return 0;
 err_t hipStreamCreateWithFlags(void **s, unsigned f) { *s = malloc(1); return 0; }
 err_t hipStreamDestroy(void *s) { free(s); return 0; }
 err_t hipStreamSynchronize(void *s) { return 0; }
-err_t hipStreamWaitEvent(void *s, void *e, unsigned f) { return 0; }
+err_t hipStreamWaitEvent(void *s, void *e, unsigned f) {
+  if (capturing) put('w');
+  return 0;
+}
 err_t hipStreamBeginCapture(void *s, int m) { capturing = 1; put('C'); return 0; }
 err_t hipStreamEndCapture(void *s, void **g) { capturing = 0; *g = malloc(1); return 0; }
 err_t hipGraphInstantiate(void **x, void *g, void *n, char *b, size_t l) {

@@ -169,3 +169,29 @@ def test_option_without_effect_keeps_graphs(fake):
     for prec in "01":
         assert "C" not in out[prec] and "I" not in out[prec] and "G" in out[prec], out[prec]
         assert out[prec + " bad"] == 1
+
+
+FORK = """
+for name, (n1, n2, na, J, kw) in dict(one_pass=(24, 48, 12, 0, {}), parts=(24, 48, 12, 2, {}),
+                                      gemms=(24, 48, 13, 2, {}), low=(24, 256, 13, 2, {}),
+                                      parts_large=(90, 300, 48, 12, {})).items():
+    c = case(n1, n2, na, J, **kw)
+    for prec in (0, 1):
+        g = L.Propagator(c, prec)
+        g.begin(c.rpaq0)
+        log()
+        g.steps(40)
+        out["%s %d" % (name, prec)] = [c.ntot, log().count("w")]
+        g.close()
+"""
+
+
+def test_captured_steps_fork_only_where_it_pays(fake):
+    """One stream in FP64, with the low-mode R passes, an angular term of one launch,
+    and the folded Coriolis parts below 1.5 M points; a fork and a join (two waits)
+    in each captured step otherwise."""
+    out = fake(FORK)
+    assert out["parts_large 1"][0] >= 1500000 > out["parts 1"][0]
+    for k, (_, waits) in out.items():
+        assert (waits > 0) == (k in ("gemms 1", "parts_large 1")), out
+        assert waits % 2 == 0
