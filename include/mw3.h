@@ -317,8 +317,8 @@ MW3_API int32_t mw3_cheby_spectrum(const double *autoc, int32_t kmax, double emi
    MW3_OPT_SIDE_STREAM  1: the angular term on its own stream beside the
                    radial passes (default in MW3_MIXED, where captured steps
                    do so only beside radial GEMMs and with an angular term of
-                   several launches, the folded Coriolis parts from 1500000
-                   points on); 0: one stream
+                   several launches: GEMMs from 500000 points on, the folded
+                   Coriolis parts from 1500000); 0: one stream
                    (default in MW3_FP64).
    MW3_OPT_ANGULAR_GRID 1 (default) or 2: the folded angular kernel runs
                    its blocks per channel divided by this value.

@@ -4071,18 +4071,20 @@ static hipError_t hpsi_impl(Ctx* c, const double* psi64) {
   // x 60: 44 us a step against 50; 256 x 512 x 120: 125 against 128; three states
   // 171 x 256 x 64: 92 against 97) and with an angular term of one launch (32 x 64 x
   // 16: 24 against 36; 256 x 480 x 120: 141 against 155).  Beside radial GEMMs they
-  // fork for an angular term of GEMMs, from the smallest grids on (forked against
-  // one stream: 64 x 100 x 140 with 65 000 points 50 against 60, J = 1 48 x 96 x 25
-  // with 79 000 38 against 41, 256 x 250 x 140 with 697 000 158 against 171), and
-  // for the two folded parts around the Coriolis coefficients from 1.5 M points
-  // (J = 1 80 x 160 x 40 with 358 000 51 against 47, 128 x 200 x 60 with 1.08 M 66
-  // against 62, 140 x 280 x 70 with 1.94 M 82 against 86, J = 2 160 x 300 x 80 with
-  // 4.1 M 152 against 163).
+  // fork for the two folded parts around the Coriolis coefficients from 1.5 M points
+  // (forked against one stream: J = 1 80 x 160 x 40 with 358 000 51 against 47, 128
+  // x 200 x 60 with 1.08 M 66 against 62, 140 x 280 x 70 with 1.94 M 82 against 86,
+  // J = 2 160 x 300 x 80 with 4.1 M 152 against 163), and for an angular term of
+  // GEMMs from 500 000.  A context alone gains there at any size (J = 1 48 x 96 x 25
+  // with 79 000 38 against 41, 80 x 160 x 41 with 366 000 49 against 58, 256 x 250 x
+  // 140 with 697 000 158 against 171), but two stepped as a batch share the hardware
+  // queues and lose (79 against 50, 101 against 69, 315 against 237; 1% at 4.4 M):
+  // the line keeps the smaller grids, which come in batches, on one stream.
   const bool low = c->opt_radial && c->rad_nitems;
   const bool one_pass = (c->ang_fold && c->opt_angular == 0) || (c->ang_nt && c->opt_angular <= 1);
   const bool parts = c->ang_fold_cor && c->opt_angular == 0 && c->opt_fp16;
   const bool one = c->graph_slot_dev && sizeof(T) == 4 &&
-                   (low || one_pass || (parts && t.ntot < 1500000));
+                   (low || one_pass || t.ntot < (parts ? 1500000 : 500000));
   hipStream_t sa = c->opt_side && !one ? c->side : s;
   if (sa != s) {
     if ((e = hipEventRecord(c->ev_psi, s)) != hipSuccess) return e;

@@ -172,10 +172,10 @@ def test_option_without_effect_keeps_graphs(fake):
 
 
 FORK = """
-for name, (n1, n2, na, J, kw) in dict(one_pass=(24, 48, 12, 0, {}), parts=(24, 48, 12, 2, {}),
-                                      gemms=(24, 48, 13, 2, {}), low=(24, 256, 13, 2, {}),
-                                      parts_large=(90, 300, 48, 12, {})).items():
-    c = case(n1, n2, na, J, **kw)
+for name, size in dict(one_pass=(24, 48, 12, 0), parts=(100, 225, 46, 1), gemms=(105, 225, 45, 1),
+                       gemms_small=(80, 160, 41, 1), low=(100, 256, 41, 1),
+                       parts_large=(90, 300, 48, 12)).items():
+    c = case(*size, **(dict(iparity=-1) if size[3] == 1 else {}))
     for prec in (0, 1):
         g = L.Propagator(c, prec)
         g.begin(c.rpaq0)
@@ -188,10 +188,11 @@ for name, (n1, n2, na, J, kw) in dict(one_pass=(24, 48, 12, 0, {}), parts=(24, 4
 
 def test_captured_steps_fork_only_where_it_pays(fake):
     """One stream in FP64, with the low-mode R passes, an angular term of one launch,
-    and the folded Coriolis parts below 1.5 M points; a fork and a join (two waits)
-    in each captured step otherwise."""
+    as GEMMs below 500 000 points and as folded Coriolis parts below 1.5 M; a fork and
+    a join (two waits) in each captured step otherwise."""
     out = fake(FORK)
-    assert out["parts_large 1"][0] >= 1500000 > out["parts 1"][0]
+    assert out["parts_large 1"][0] >= 1500000 > out["parts 1"][0] > 500000
+    assert out["gemms 1"][0] >= 500000 > out["gemms_small 1"][0]
     for k, (_, waits) in out.items():
         assert (waits > 0) == (k in ("gemms 1", "parts_large 1")), out
         assert waits % 2 == 0
