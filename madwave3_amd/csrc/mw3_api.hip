@@ -119,15 +119,15 @@ static hipError_t alloc_zero(void** p, size_t bytes) {
 }
 
 static void free_all(Ctx* c) {
-  void* ptrs[] = {c->d_pt_dense, c->d_mask, c->d_v, c->d_absfr1, c->d_absfr2, c->d_psi,
+  void* ptrs[] = {c->d_pt_dense, c->d_v, c->d_absfr2, c->d_psi,
                   c->d_psim1, c->d_psi0, c->d_a0, c->d_a0b, c->d_t1, c->d_t2, c->d_fbr,
                   c->d_ang, c->d_hout, c->d_nn1, c->d_p2r1, c->d_p2r2, c->d_divi,
                   c->d_dst_tables, c->d_Dmat, c->d_acoef, c->d_bcoef, c->d_nbr,
-                  c->d_flux_dense, c->d_flux_col, c->d_zar1flux, c->d_ring_zr, c->d_ring_zdr,
+                  c->d_flux_col, c->d_ring_zr, c->d_ring_zdr,
                   c->d_ring_cvj, c->d_zcr, c->d_zcdr, c->d_zs2, c->d_etot, c->d_fdv, c->d_dcvj,
                   c->d_cvj_skip, c->d_norm_part, c->d_ring_norm, c->d_stats, c->d_fbr_rng, c->d_efe, c->d_zfe, c->d_phi,
                   c->d_wmat, c->d_zero_skip, c->d_ch_elec, c->d_ch_omega, c->d_ch_cpl, c->d_potiflux,
-                  c->d_flux_elec, c->d_scratch, c->d_fmap, c->d_ir1flux, c->d_ring_slice,
+                  c->d_flux_elec, c->d_scratch, c->d_ring_slice,
                   c->d_psi32, c->d_psim132, c->d_scr32, c->d_up_wave, c->d_up_seg,
                   c->d_up_tile, c->d_up_sfirst, c->d_up_part,
                   c->d_up_row, c->d_up_tab, c->d_rr_f, c->d_rr_b, c->d_rr_w, c->d_g1,
@@ -247,13 +247,11 @@ int32_t mw3_create(const mw3_setup* setup, int32_t precision, mw3_ctx** out) {
   CK(hipEventCreateWithFlags(&c->ev_ang, evf), "mw3_create: event");
   CK(alloc_zero((void**)&c->d_slot, 2 * sizeof(int32_t)), "mw3_create: ring slot");
   CK(upload_raw(&c->d_pt_dense, t.pt_dense.data(), t.pt_dense.size()), "mw3_create: index map");
-  CK(upload_raw(&c->d_mask, t.mask.data(), t.mask.size()), "mw3_create: mask");
 
   if (precision == MW3_MIXED)
     CK(upload<float>(&c->d_v, t.vdense), "mw3_create: V");
   else
     CK(upload<double>(&c->d_v, t.vdense), "mw3_create: V");
-  CK(upload_raw(&c->d_absfr1, setup->absfr1, (size_t)t.n1), "mw3_create: absfr1");
   CK(upload_raw(&c->d_absfr2, setup->absfr2, (size_t)t.n2), "mw3_create: absfr2");
   CK(alloc_zero((void**)&c->d_psi, nd * sizeof(double)), "mw3_create: psi");
   c->graph_psi0 = c->d_psi;
@@ -311,15 +309,7 @@ int32_t mw3_create(const mw3_setup* setup, int32_t precision, mw3_ctx** out) {
   }
   // projections
   int netot = std::max(setup->netot, 0);
-  CK(upload_raw(&c->d_flux_dense, t.flux_dense.data(), t.flux_dense.size()), "mw3_create: flux");
   CK(upload_raw(&c->d_flux_col, t.flux_col.data(), t.flux_col.size()), "mw3_create: flux");
-  {
-    // zAR1flux is read by the update whenever projections run (zeros if the
-    // flux line has no point)
-    std::vector<double> zar(t.zar1flux.begin(), t.zar1flux.end());
-    if (zar.size() < 2 * (size_t)t.n1) zar.resize(2 * (size_t)t.n1, 0.0);
-    CK(upload_raw(&c->d_zar1flux, zar.data(), zar.size()), "mw3_create: flux");
-  }
   CK(upload_raw(&c->d_potiflux, t.potiflux.data(), t.potiflux.size()), "mw3_create: flux");
   CK(upload_raw(&c->d_flux_elec, t.flux_elec.data(), t.flux_elec.size()), "mw3_create: flux");
   {
@@ -349,20 +339,6 @@ int32_t mw3_create(const mw3_setup* setup, int32_t precision, mw3_ctx** out) {
       }
     }
     CK(upload_raw(&c->d_up_row, row.data(), row.size()), "mw3_create: update rows");
-  }
-  {
-    std::vector<int32_t> fmap((size_t)t.nc * t.na * t.n2, -1);
-    for (int64_t f = 0; f < t.nflux; f++) {
-      // flux_col is the dense index of (c, ia, 0, R): c*slab + ia*plane + R
-      uint32_t col = t.flux_col[f];
-      int64_t cia = col / t.nplane;
-      int64_t R = col % t.n2;
-      fmap[(size_t)cia * t.n2 + R] = (int32_t)f;
-    }
-    CK(upload_raw(&c->d_fmap, fmap.data(), fmap.size()), "mw3_create: flux map");
-    std::vector<int32_t> i1f(t.ir1flux.begin(), t.ir1flux.end());
-    if (i1f.empty()) i1f.assign(t.na, 1);
-    CK(upload_raw(&c->d_ir1flux, i1f.data(), i1f.size()), "mw3_create: flux map");
   }
   CK(alloc_zero((void**)&c->d_ring_norm, sizeof(double) * 2 * kRing), "mw3_create: norms");
   CK(alloc_zero((void**)&c->d_stats, sizeof(double) * stats_doubles()), "mw3_create: sums");

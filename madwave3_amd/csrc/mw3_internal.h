@@ -2,7 +2,8 @@
 //
 // Device data model (one context = one propagation on one GPU):
 //   dense slabs  X[ch][iang][ir1][ir2]   ir2 (R) fastest, iang = global angle-1
-//   mask         uint8 [iang][ir1][ir2]  1 on the kept (compressed) points
+//   mask         uint8 [iang][ir1][ir2]  1 on the kept (compressed) points (host;
+//                the device has lists made from it)
 //   V            [et][es][iang][ir1][ir2] (0 off the mask)
 //   FBR          Xt[ch][jj][ir1][ir2]    angular functions index jj
 // The compressed A0 vector of the ABI maps to the slabs through pt_dense.
@@ -135,7 +136,6 @@ struct Ctx {
 
   // device buffers
   uint32_t* d_pt_dense = nullptr;
-  uint8_t* d_mask = nullptr;
   // update: strips of 16 up_nt consecutive R of one (channel, angle), their
   // 16-row tiles with a kept point in runs of up_tmax per wave, and the radial
   // tables (mw3_step.h)
@@ -165,7 +165,6 @@ struct Ctx {
   double* d_g2 = nullptr;         // [nc na][up_ns][up_kst][16]
   bool g_fresh = false;           // d_g1 is G of d_psi
   void* d_v = nullptr;  // double or float dense V
-  double* d_absfr1 = nullptr;
   double* d_absfr2 = nullptr;
   double* d_psi = nullptr;    // psi_k dense
   double* d_psim1 = nullptr;  // psi_{k-1} dense
@@ -196,9 +195,7 @@ struct Ctx {
   void* d_bcoef = nullptr;
   int32_t* d_nbr = nullptr;
   // projections
-  uint32_t* d_flux_dense = nullptr;
   uint32_t* d_flux_col = nullptr; // [nflux] dense index of (c, ia, 0, ir2)
-  double* d_zar1flux = nullptr;
   double* d_ring_zr = nullptr;   // [kRing][nflux]
   double* d_ring_zdr = nullptr;  // [kRing][nflux][2]
   double* d_ring_cvj = nullptr;  // [kRing][ncvj]
@@ -270,8 +267,6 @@ struct Ctx {
   double* d_potiflux = nullptr;
   int32_t* d_flux_elec = nullptr;
 
-  int32_t* d_fmap = nullptr;     // [nc][na][n2] flux point index or -1
-  int32_t* d_ir1flux = nullptr;  // [na]
   double* d_ring_slice = nullptr; // [slice_ring][nc][na][n1] psi at R = ir2abs / sqrt(ah2)
 
   // product-state projection (iprod = 2, mw3_prod_attach).  Per step, the
