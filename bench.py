@@ -39,7 +39,7 @@ def build_case(cfg):
 
 
 # kernel launches per step in each group (mixed; in FP64 radial_dst is one), per
-# ring of steps for the last four
+# many steps at once for the last four
 GROUP_LAUNCHES = {"radial_dst": 3, "angular": 1, "update_fused": 1, "coriolis": 1,
                   "update_tail": 2, "projections": 1, "energy_sums": 2, "products": 1}
 RING_GROUPS = ("update_tail", "projections", "energy_sums", "products")
@@ -53,11 +53,11 @@ def kernel_groups(times, steps):
     a stream of its own beside the radial passes), update_fused (the update
     kernel), coriolis (the FBR coefficient pass with the Omega +- 1 stencil, run
     instead of the fused forward epilogue when channels are Coriolis-coupled)
-    and, once per ring of steps, update_tail (norms and flux columns),
+    and, for many steps at once, update_tail (norms and flux columns),
     projections (reactant-state sums), products (the product-state reduction)
-    and energy_sums (with the product-state GEMM of the ring): the total time
-    over the timed region divided by the `steps` timed steps, since every flush
-    is timed."""
+    and energy_sums (with the product-state GEMM, once per ring of steps): the
+    total time over the timed region divided by the `steps` timed steps, since
+    every one of these sums is timed."""
     acc = {}
     for name, (ms, cnt) in times.items():
         if name.startswith("dst"):
@@ -454,12 +454,12 @@ def main():
             # (e) energy projection: 8 netot n_flux flops per step (time only)
             "energy_sums": ("hbm", 16.0 * nflux, "GB/s"),
             "projections": ("hbm", 8.0 * case.nangu * case.npun1, "GB/s"),
-            # flux columns and norm of the step (second stream): the flux
-            # line values written to the ring (time only, like energy_sums)
+            # flux columns and norms: the flux line values written to the ring
+            # (time only, like energy_sums)
             "update_tail": ("hbm", 16.0 * nflux, "GB/s"),
             # (d) Coriolis stencil in the FBR: 2 s N bytes over the Omega-coupled blocks
             "coriolis": ("hbm", 2.0 * s_op * N, "GB/s"),
-            # product reduction: 64 partials per update item, dtrans, ring row
+            # product reduction: segment sums, dtrans, ring row
             "products": ("hbm", 8.0 * 3 * max(nprod_l, 1), "GB/s"),
         }
         for k, ms in per.items():

@@ -19,9 +19,10 @@
 
 namespace mw3 {
 
-// Chebyshev steps buffered between energy sums: the FP64 accumulators (about
-// 1 GB at 500 energies and 61,440 flux points) are read and written once per
-// ring, so a longer ring moves fewer accumulator bytes per step
+// Chebyshev steps buffered between energy sums: the FP64 accumulators (0.2 GB at
+// 500 energies and 12 868 flux points, 0.9 GB with seven helicity blocks) are read
+// and written once per ring, so a longer ring moves fewer accumulator bytes per
+// step
 constexpr int kRing = 256;
 
 // Steps of one graph launch where that many are to come.  Between two graphs
@@ -306,7 +307,7 @@ struct Ctx {
   // persistent low-mode kernels (1) or as GEMMs (0); angular term by the
   // parity-folded one-pass kernel (0), the unfolded one-pass kernel (1) or
   // GEMMs (2), each falling back to the next where not built; the angular
-  // term on the third stream (1) or the main one (0)
+  // term on the second stream (1; captured steps where it pays) or the main one (0)
   int opt_radial = 1, opt_angular = 0, opt_side = 0;
   int opt_ang_grid = 1;           // folded angular kernel: blocks per channel / this
   int flux_etest = 1;             // E > V(flux point) test when the flux sums are read
@@ -359,8 +360,8 @@ hipError_t build_prod_plan(Ctx* c);
 hipError_t launch_prod_sums(Ctx* c);
 hipError_t launch_prod_flush(Ctx* c);
 
-// most channels of one product-state context (LDS of the per-step product
-// reduction: 64 doubles per channel)
+// most channels of one product-state context: the documented limit of
+// mw3_prod_attach (no kernel depends on it)
 constexpr int kProdMaxCh = 64;
 
 // GEMM passes of the step (template tag: one kernel symbol per pass)

@@ -11,10 +11,11 @@
 //                   projection, damped three-term update
 //                   (SRC/main_madwave3.f:332-339), the sums over r of the
 //                   per-step projections (mw3_step.h);
-//   once per ring of kRing steps: norms, flux-line samples
-//                   (SRC/mod_flux_01y2.f:598-628), reactant- and product-state
-//                   amplitudes (SRC/mod_flux_01y2.f:672-702), and the energy
-//                   sums sum_k C_k(E) x_k (CoefEcheby,
+//   once per many steps: flux-line samples (SRC/mod_flux_01y2.f:598-628) and
+//                   reactant- and product-state amplitudes
+//                   (SRC/mod_flux_01y2.f:672-702);
+//   once per ring of kRing steps: norms, and the energy sums
+//                   sum_k C_k(E) x_k (CoefEcheby,
 //                   SRC/main_madwave3.f:462-490) as complex products.
 #include <hip/hip_runtime.h>
 
@@ -746,7 +747,6 @@ __global__ __launch_bounds__(256) void k_cvj_ring(const double* __restrict__ sli
   }
 }
 
-// ---------------------------------------------------------------------------
 // ---------------------------------------------------------------------------
 // energy accumulation over a ring of steps k0 .. k0+ns-1
 //   acc[x][E] += sum_s C_{k0+s}(E) z[s][x],  C_k(E) = 2 hbr/delta e^{-i k acos Es}/sqrt(1-Es^2)
@@ -3877,7 +3877,6 @@ void free_plans(Ctx* c) {
   for (auto* p : ps) free_plan(p);
 }
 
-// H psi terms into work slabs: d_t2 = T psi (rows r < nn1), d_ang = angular
 // psi in the operator precision T: the FP32 copy in mixed mode
 template <typename T>
 static const T* op_psi(Ctx* c, const double* psi);
@@ -4053,6 +4052,8 @@ static hipError_t angular_impl(Ctx* c, const T* psi, hipStream_t s) {
   return hipSuccess;
 }
 
+// H psi terms for the update: d_ang = the angular term; the radial correction as
+// G2 (FP64 with the r products in the update) or as rows r < nn1 of d_t2
 template <typename T>
 static hipError_t hpsi_impl(Ctx* c, const double* psi64) {
   const T* psi = op_psi<T>(c, psi64);
@@ -4139,6 +4140,7 @@ static hipError_t hpsi_impl(Ctx* c, const double* psi64) {
   }
   return hipSuccess;
 }
+
 __global__ void k_to_f32(const double* __restrict__ src, float* __restrict__ dst, int64_t n) {
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
        i += (int64_t)gridDim.x * blockDim.x)

@@ -741,8 +741,8 @@ struct RrArgs {
                      // the first product's results
   int na, n1, n2, nk1, kst, nb;
   const int32_t* sfirst;  // [nc na ns + 1] first segment of each strip
-  // strips per row, log2 of their width (4; as a constant the addresses built on it
-  // are all formed ahead, which spills: 28.9 us against 28.6), most segments of one
+  // strips per row, log2 of their width (4; with a constant the compiler forms more
+  // addresses ahead and spills at NP = 3), most segments of one
   int ns, swl, segmax;
 };
 
